@@ -8,26 +8,20 @@
 
 namespace abkv {
 
-constexpr int kBM = 64;                  // query rows per workgroup
-constexpr int kBN = 64;                  // keys per tile
 constexpr int kTileElems = kBN * kHeadDim;
 
-// Per-element visibility for layouts whose tiles cannot be classified (unaligned masked prefill); other kernels never
-// call it (their tiles are always aligned: kAligned = true). quota[u]: code slots visible to this wave's head u;
-// tail: the retained tail T under ``policy`` (a block's codes never see its own last T content rows).
-struct MaskGeom {
-  int qrow, S0, C, per, plen;
-  int quota[2];
-  int tail;
-  int policy;
-  int xattn;      // code rows' attention to their own pass's code rows (kXattn*)
-  int K, L;       // code rows per pause pass, passes per block
-  int copy;       // copy-region rows at the end of the S0 rows
-  int R;          // replay rows per block
-  bool rx;        // the codes do not see the block's last R content rows
-  __device__ __forceinline__ bool visible(int kv, int u) const {
-    return compress_visible(qrow, kv, S0, copy, C, K, L, per, plen, quota[u], tail, policy, xattn, R, rx);
-  }
+// What a wave's lanes need to mask a tile: the first key its query row does not see causally (mode 1) and, for walks
+// that yield span tiles (mode 3), the row's facts and its heads' code quotas.
+struct CausalLane {
+  int limit;
+};
+template <int H>
+struct SpanLane {
+  int limit;
+  MaskShape g;
+  RowFacts row;
+  int plen;
+  int quota[H];
 };
 
 __device__ __forceinline__ u32x4 ld16g(const __bf16* p) { return *reinterpret_cast<const u32x4*>(p); }
@@ -129,13 +123,6 @@ __device__ __forceinline__ void store_bf16x8(__bf16* dst, const floatx4& lo, con
   *reinterpret_cast<u32x4*>(dst) = wv;
 }
 
-struct TileMask {
-  int mode;        // 0 none, 1 key < this lane's limit, 2 key < limit[u] (this wave's head u), 3 per-element mask,
-                   // 4 key < this lane's limit and outside the excluded range [limit[0], limit[1]),
-                   // 5 key < limit[0] or key >= this lane's limit + limit[1] (a band that moves with the query row)
-  int limit[2];
-};
-
 // V^T operand of one PV MFMA from the swizzled V tile with two ds_read_b64_tr_b16 (LDS transpose reads). Within a
 // 16-lane group, lane i of a transpose read receives element i % 4 of the 8-byte chunk addressed by lane
 // 4e + i / 4, for e = 0..3. The operand row m of dim slab t is dim 32 * (m / 4) + 4t + m % 4 and its k-index
@@ -196,17 +183,16 @@ __device__ __forceinline__ void tile_scores(const __bf16* Kbuf, const bf16x8 (&q
       }
 }
 
-// Hidden keys of a partial tile get score -inf (tm.mode 0: nothing hidden). kElem: an aligned walk that may yield
-// per-element tiles (mode 3, the full predicate MaskGeom::visible) beside the limit modes. kBand: a walk that may
-// yield band tiles (mode 5, the rolling retained tail).
-template <int H, bool kAligned, bool kHole = false, bool kElem = false, bool kBand = false>
-__device__ __forceinline__ void tile_mask(floatx4 (&s)[2][2][H], int k0, const TileMask& tm, int lane_limit,
-                                          const MaskGeom& geo, int j) {
+// Hidden keys of a partial tile get score -inf (tm.mode 0: nothing hidden). The walk says which modes occur beyond the
+// limits: kHole an excluded key range (mode 4), kBand a band that moves with the row (mode 5), kSpan the row's span of
+// a segment (mode 3).
+template <int H, class Walk, class Lane>
+__device__ __forceinline__ void tile_mask(floatx4 (&s)[2][2][H], int k0, const TileMask& tm, const Lane& lane, int j) {
   static_assert(H <= 2, "TileMask holds two per-head limits");
   if (tm.mode == 0) return;
-  if constexpr (kHole) {
-    if (tm.mode == 4 || (kBand && tm.mode == 5)) {       // an excluded key range (code step, retained tail) or a band
-      const bool band = kBand && tm.mode == 5;
+  if constexpr (Walk::kHole) {
+    if (tm.mode == 4 || (Walk::kBand && tm.mode == 5)) { // an excluded key range (code step, retained tail) or a band
+      const bool band = Walk::kBand && tm.mode == 5;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -214,18 +200,39 @@ __device__ __forceinline__ void tile_mask(floatx4 (&s)[2][2][H], int k0, const T
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int kv = k0 + 32 * kk + 16 * t + 4 * j + r;
-            const bool ok = band ? (kv < tm.limit[0] || kv >= lane_limit + tm.limit[1])
-                                 : kv < lane_limit && (kv < tm.limit[0] || kv >= tm.limit[1]);
+            const bool ok = band ? (kv < tm.limit[0] || kv >= lane.limit + tm.limit[1])
+                                 : kv < lane.limit && (kv < tm.limit[0] || kv >= tm.limit[1]);
 #pragma unroll
             for (int u = 0; u < H; ++u) s[kk][t][u][r] = ok ? s[kk][t][u][r] : -INFINITY;
           }
       return;
     }
   }
-  // every partial tile of an aligned layout is "key < lim[u]" with a per-column limit (per head or per lane)
+  // "key < lim[u]" with a per-column limit (per head or per lane); a span adds the keys from lo[u] on, `len` of them
   int lim[H];
 #pragma unroll
-  for (int u = 0; u < H; ++u) lim[u] = tm.mode == 1 ? lane_limit : tm.limit[u];
+  for (int u = 0; u < H; ++u) lim[u] = tm.mode == 1 ? lane.limit : tm.limit[u];
+  if constexpr (Walk::kSpan) {
+    if (tm.mode == 3) {
+      int lo = kNoKey;
+#pragma unroll
+      for (int u = 0; u < H; ++u)
+        lane_span(lane.g, lane.row, tm.seg, tm.kb, tm.limit[0], tm.limit[1], lane.plen, lane.quota[u], lim[u], lo);
+      const unsigned len = imax(tm.limit[1] - lo, 0);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kv = k0 + 32 * kk + 16 * t + 4 * j + r;
+            const bool suffix = (unsigned)(kv - lo) < len;
+#pragma unroll
+            for (int u = 0; u < H; ++u) s[kk][t][u][r] = kv < lim[u] || suffix ? s[kk][t][u][r] : -INFINITY;
+          }
+      return;
+    }
+  }
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -235,15 +242,7 @@ __device__ __forceinline__ void tile_mask(floatx4 (&s)[2][2][H], int k0, const T
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int kv = k0 + 32 * kk + 16 * t + 4 * j + r;
-          bool ok;
-          if constexpr (kAligned && kElem) {
-            ok = tm.mode == 3 ? geo.visible(kv, u) : kv < lim[u];
-          } else if constexpr (kAligned) {
-            ok = kv < lim[u];
-          } else {
-            ok = geo.visible(kv, u);
-          }
-          s[kk][t][u][r] = ok ? s[kk][t][u][r] : -INFINITY;
+          s[kk][t][u][r] = kv < lim[u] ? s[kk][t][u][r] : -INFINITY;
         }
 }
 
@@ -355,16 +354,16 @@ struct Slot {
 //   iteration (past the last tile they re-load tile n into slots nobody reads again) so that each iteration has the
 //   same count of loads in flight: the waits below and the compiler's own then stay exact.
 //   mask + rescale of tile n; scores of tile n+1 (MFMA) with the probabilities of tile n (VALU); O += V(n) . P(n)
-// Walk::next(kt, tm, first) yields the tiles in order. Rows addresses key rows; keys >= n_keys are never read.
+// Walk::next(k0, tm, first) yields the tiles in order (k0: the first key). Rows addresses key rows; keys >= n_keys are never read.
 // On return l_run[u] is the full weight sum of column (u, m16) in every lane of the column (o and m_run as above).
-template <int H, bool kAligned, int kWaves, class Rows, class Walk>
+template <int H, int kWaves, class Rows, class Walk, class Lane>
 __device__ __forceinline__ void attend_tiles(const Rows& rows, Walk& walk, int n_keys, __bf16* const (&K)[kStages],
                                              __bf16* const (&V)[kStages], const bf16x8 (&qop)[H][4],
                                              floatx4 (&o)[8][H], float (&m_run)[H], float (&l_run)[H],
-                                             int lane_limit, float scale_log2, const MaskGeom& geo, int w, int lane) {
+                                             const Lane& lane_mask, float scale_log2, int w, int lane) {
   constexpr int kPerWave = 16 / kWaves;
   const int m16 = lane & 15, j = lane >> 4;
-  int t0 = 0, t1 = 0, t2 = 0;                      // tiles n, n+1, n+2
+  int t0 = 0, t1 = 0, t2 = 0;                      // first keys of tiles n, n+1, n+2
   TileMask m0, m1, m2;
   if (!walk.next(t0, m0, true)) return;
   t1 = t0;
@@ -372,15 +371,15 @@ __device__ __forceinline__ void attend_tiles(const Rows& rows, Walk& walk, int n
   t2 = t1;
   bool h2 = h1 && walk.next(t2, m2, false);
   {
-    const auto s0 = rows.template src<kPerWave>(t0 * kBN, w, n_keys);
+    const auto s0 = rows.template src<kPerWave>(t0, w, n_keys);
     issue_half<kWaves, false>(rows, s0, n_keys, K[0], w, lane);
     issue_half<kWaves, true>(rows, s0, n_keys, V[0], w, lane);
     if (h1) {
-      const auto s1 = rows.template src<kPerWave>(t1 * kBN, w, n_keys);
+      const auto s1 = rows.template src<kPerWave>(t1, w, n_keys);
       issue_half<kWaves, false>(rows, s1, n_keys, K[1], w, lane);
       issue_half<kWaves, true>(rows, s1, n_keys, V[1], w, lane);
     }
-    if (h2) issue_half<kWaves, false>(rows, rows.template src<kPerWave>(t2 * kBN, w, n_keys), n_keys, K[2], w, lane);
+    if (h2) issue_half<kWaves, false>(rows, rows.template src<kPerWave>(t2, w, n_keys), n_keys, K[2], w, lane);
   }
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
@@ -396,8 +395,8 @@ __device__ __forceinline__ void attend_tiles(const Rows& rows, Walk& walk, int n
     int t3 = t2;
     TileMask m3;
     const bool h3 = h2 && walk.next(t3, m3, false);
-    const auto src_k = rows.template src<kPerWave>((h3 ? t3 : t0) * kBN, w, n_keys);
-    const auto src_v = rows.template src<kPerWave>((h2 ? t2 : t0) * kBN, w, n_keys);
+    const auto src_k = rows.template src<kPerWave>(h3 ? t3 : t0, w, n_keys);
+    const auto src_v = rows.template src<kPerWave>(h2 ? t2 : t0, w, n_keys);
     // Plain s_barrier: each wave first waits for its own DMAs of two iterations back (vmcnt: the last iteration's
     // 2 x 16 / kWaves stay in flight) and its LDS and scalar reads (lgkmcnt).
     if constexpr (kWaves == 8) __asm__ volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
@@ -405,7 +404,7 @@ __device__ __forceinline__ void attend_tiles(const Rows& rows, Walk& walk, int n
     __builtin_amdgcn_s_barrier();
     issue_half<kWaves, false>(rows, src_k, n_keys, K[slot], w, lane);
     issue_half<kWaves, true>(rows, src_v, n_keys, V[slot2], w, lane);
-    tile_mask<H, kAligned, Walk::kHole, Walk::kElem, Walk::kBand>(s_cur, t0 * kBN, m0, lane_limit, geo, j);
+    tile_mask<H, Walk>(s_cur, t0, m0, lane_mask, j);
     bf16x8 pop[2][H];
     tile_softmax<H>(s_cur, o, m_run, lsum, scale_log2, pop);
     // Unconditional so that the MFMAs can overlap the softmax work: after the last tile the scores are computed from

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "mask_walk.h"
+
 namespace abkv {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -20,18 +22,6 @@ constexpr int kHeadsQ = kHeadsKV * kGroup;
 constexpr int kSlotElems = kHeadsKV * kHeadDim;            // 1024 elements = 2 KiB per slot per K or V
 constexpr int kHalfElems = kPage * kSlotElems;             // 16384 elements = 32 KiB (K half of a page)
 constexpr int kPageElems = 2 * kHalfElems;                 // 32768 elements = 64 KiB
-
-// Retained-tail policies (retain_tail_policy): which later rows see an earlier block's last T content rows.
-constexpr int kTailStatic = 0;   // every later row
-constexpr int kTailRolling = 1;  // the next block's i-th content row sees the tail's rows i .. T-1
-constexpr int kTailSticky = 2;   // every content row of the next block
-constexpr int kTailRaw = 3;      // the rolling window of raw_tail (compress_forward.py:89-96): the codes see the whole
-                                 // block, their own tail included (code_excluded_tail = 0, :309-311)
-
-// pause_xattn: which code rows of its own pass and block a code row sees (compress_forward.py:313-314, 622-625).
-constexpr int kXattnFull = 0;     // all of them (bidirectional)
-constexpr int kXattnCausal = 1;   // those at or before its own position
-constexpr int kXattnNone = 2;     // none, itself included
 
 // Whether content row kw (in-block offset) of block kb is a retained-tail row visible to row qw of block qb under the
 // policy (abridgekv/compress_forward.py:99-124; the caller adds causality, the raw prompt and the codes' exclusion of

@@ -84,18 +84,18 @@ struct PackedRows {
 // that meet the excluded key range [ex_lo, ex_hi) (empty when ex_lo >= ex_hi) mask it as well.
 struct RangeWalk {
   static constexpr bool kHole = true;
-  static constexpr bool kElem = false;
   static constexpr bool kBand = false;
+  static constexpr bool kSpan = false;
   int kt_begin, kt_end, k_full, ex_lo, ex_hi;
-  __device__ __forceinline__ bool next(int& kt, TileMask& tm, bool first) {
-    kt = first ? kt_begin : kt + 1;
-    tm.mode = (kt + 1) * kBN <= k_full ? 0 : 1;
-    if (kt * kBN < ex_hi && (kt + 1) * kBN > ex_lo) {
+  __device__ __forceinline__ bool next(int& k0, TileMask& tm, bool first) {
+    k0 = first ? kt_begin * kBN : k0 + kBN;
+    tm.mode = k0 + kBN <= k_full ? 0 : 1;
+    if (k0 < ex_hi && k0 + kBN > ex_lo) {
       tm.mode = 4;
       tm.limit[0] = ex_lo;
       tm.limit[1] = ex_hi;
     }
-    return kt < kt_end;
+    return k0 < kt_end * kBN;
   }
 };
 
@@ -168,7 +168,6 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
   const int k_end = causal ? min(limit, kv0 + q_hi + 1) : limit;
   const int k_full = causal ? min(limit, kv0 + q0 + 1) : limit;
   const int n_k_tiles = (k_end + kBN - 1) / kBN;
-  const MaskGeom geo{};
   // key tiles of this block: all of them, or split z's share when the launch is split along the keys
   RangeWalk walk;
   walk.kt_begin = a.split_tiles > 0 ? split * a.split_tiles : 0;
@@ -186,12 +185,12 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
     __syncthreads();
     const PackedRows rows{a.side_kv + (long)a.side_o[kvh] * kHeadDim, side_table, side_q, 1.f / (float)side_q,
                           2L * a.side_rows * kHeadDim, (long)a.side_rows * kHeadDim};
-    attend_tiles<H, true, kWaves>(rows, walk, k_end, Kbuf, Vbuf, qop, o, m_run, l_run, lane_limit, a.scale_log2, geo,
-                                  w, lane);
+    attend_tiles<H, kWaves>(rows, walk, k_end, Kbuf, Vbuf, qop, o, m_run, l_run, CausalLane{lane_limit}, a.scale_log2,
+                            w, lane);
   } else {
     const PagedRows rows{a.kv + kvh * kHeadDim, a.block_table + (long)r * a.bt_stride, a.bt_width, a.num_pages};
-    attend_tiles<H, true, kWaves>(rows, walk, k_end, Kbuf, Vbuf, qop, o, m_run, l_run, lane_limit, a.scale_log2, geo,
-                                  w, lane);
+    attend_tiles<H, kWaves>(rows, walk, k_end, Kbuf, Vbuf, qop, o, m_run, l_run, CausalLane{lane_limit}, a.scale_log2,
+                            w, lane);
   }
 
   // Split partials: the split's output normalised by its weight sum l, in fp16 (half the bytes the epilogue writes

@@ -104,7 +104,6 @@ __global__ __launch_bounds__(512, 1) void prefill_bwd_dq_kernel(PrefillBwdArgs a
   const int lane = threadIdx.x & 63;
   const int m16 = lane & 15, j = lane >> 4;
   const int rg = w / 2, hbase = H * (w % 2);
-  const int per = kAligned ? f.C + f.K : f.C + f.L * f.K + f.R;
   const int q0 = qt * kBM;
   const int qrow = q0 + 16 * rg + m16;
   const int plen = f.prompt_len ? f.prompt_len[b] : 0;
@@ -147,16 +146,16 @@ __global__ __launch_bounds__(512, 1) void prefill_bwd_dq_kernel(PrefillBwdArgs a
   const DenseRows<kAligned> rows{f.k + (long)b * f.k_sb + (long)kvh * f.k_sh, f.v + (long)b * f.v_sb + (long)kvh * f.v_sh,
                                  f.k_ss, f.v_ss};
   const int wq0 = hbase ? quota_all[2] : quota_all[0], wq1 = hbase ? quota_all[3] : quota_all[1];
-  const MaskGeom geo{qrow, f.S0, f.C, per, plen, {wq0, wq1}, f.tail, f.policy, f.xattn, f.K, kAligned ? 1 : f.L,
-                     kAligned ? 0 : f.copy, kAligned ? 0 : f.R, !kAligned && f.rx};
   const int q_last = min(q0 + kBM, f.S0) - 1;
-  TileWalk<kAligned, kTail, kWindow> walk(q0, q_last, f.C, per, f.S0, plen, qmin, qmax, wq0, wq1, f.tail, f.policy);
+  typedef MaskWalk<kAligned, kTail, kWindow> MW;
+  MW mw(f, q0, q_last, qrow, plen, qmin, qmax, wq0, wq1);
+  auto& walk = mw.walk;
 
   int tc = 0;
   TileMask mc;
   if (walk.next(tc, mc, true)) {
     {
-      const auto s0 = rows.template src<2>(tc * kBN, w, f.S0);
+      const auto s0 = rows.template src<2>(tc, w, f.S0);
       issue_half<kWaves, false>(rows, s0, f.S0, Kb[0], w, lane);
       issue_half<kWaves, true>(rows, s0, f.S0, Vb[0], w, lane);
     }
@@ -167,7 +166,7 @@ __global__ __launch_bounds__(512, 1) void prefill_bwd_dq_kernel(PrefillBwdArgs a
       int tn = tc;
       TileMask mn;
       const bool hn = walk.next(tn, mn, false);
-      const auto src = rows.template src<2>((hn ? tn : tc) * kBN, w, f.S0);
+      const auto src = rows.template src<2>(hn ? tn : tc, w, f.S0);
       __asm__ volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       issue_half<kWaves, false>(rows, src, f.S0, Kb[1 - sl], w, lane);
@@ -175,7 +174,7 @@ __global__ __launch_bounds__(512, 1) void prefill_bwd_dq_kernel(PrefillBwdArgs a
       floatx4 s[2][2][H], dp[2][2][H];
       tile_scores<H>(Kb[sl], qop, s, m16, j);
       tile_scores<H>(Vb[sl], gop, dp, m16, j);
-      tile_mask<H, kAligned, kTail, false, kWindow>(s, tc * kBN, mc, qrow + 1, geo, j);
+      tile_mask<H, typename MW::Walk>(s, tc, mc, mw.lane, j);
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll

@@ -16,13 +16,12 @@ struct PrefillArgs {
   float scale_log2;
   __bf16* out;      long o_sb, o_ss, o_sh;   // [B, S0, 32, 128]
   float* lse;                                // [B, 32, S0] natural log, or nullptr
-  int aligned;                               // C % 64 == 0 && K % 64 == 0 (the walk over visible tiles)
+  int aligned;                               // C % 64 == 0 && K % 64 == 0 and only content and codes (TileWalk)
   int num_q_tiles;
   int tail;                                  // retained tail T (0: none)
   int policy;                                // its policy: kTailStatic, kTailRolling, kTailSticky, kTailRaw
-  int xattn;                                 // code <-> code attention in a block (kXattn*; the aligned walks
-                                             // serve kXattnFull, the others take the per-element walk)
-  int L;                                     // pause passes of K code rows per block (the aligned walks serve 1)
+  int xattn;                                 // code <-> code attention in a block (kXattn*; aligned: kXattnFull)
+  int L;                                     // pause passes of K code rows per block (aligned: 1)
   int copy;                                  // copy-region rows after the N blocks (S0 counts them; aligned: 0)
   int R;                                     // replay rows after each block's codes (aligned: 0)
   int rx;                                    // code_exclude_replay_tail: the codes do not see the last R content rows
@@ -40,8 +39,8 @@ __device__ __forceinline__ GridPos grid_pos(int batch) {
   return {l / (kHeadsKV * batch), l % kHeadsKV, (l / kHeadsKV) % batch};
 }
 
-// Walk over the key tiles one query tile attends to, with the mask mode of each.
-// Aligned layouts (C and K multiples of 64): a key tile is named by (block kb, tile tw of the block's C + K rows).
+// Walk over the key tiles one query tile attends to, with the mask mode of each, in aligned layouts (C and K multiples
+// of 64; SegWalk in mask_walk.h takes the others). A key tile is named by (block kb, tile tw of the block's C + K rows).
 // Within a segment (one block's content, one block's codes) visibility is monotone in tw, so the first invisible tile
 // ends the segment and the walk jumps to the next one: no per-tile test of skipped tiles and no integer division.
 // kTail (aligned layouts with a retained tail of T rows): an earlier block's content is visible where it is raw
@@ -51,14 +50,13 @@ __device__ __forceinline__ GridPos grid_pos(int batch) {
 // end and the tail (mode 4). kWindow (the rolling and sticky policies): only content query tiles of the next block see
 // a block's tail; under "rolling" query row i of the block sees tail rows i.. (content rows >= C - T + i), so the tile
 // where the band starts, and those it crosses, take the band mask (mode 5).
-// Unaligned layouts: every tile up to the last visible block, mask evaluated per element (mode 3).
-template <bool kAligned, bool kTail = false, bool kWindow = false>
+template <bool kTail, bool kWindow>
 struct TileWalk {
   static_assert(kTail || !kWindow, "a window tail is a retained tail");
   static constexpr bool kHole = kTail;                      // yields excluded key ranges (mode 4) with a tail
-  static constexpr bool kElem = false;                      // aligned walks never yield per-element tiles
+  static constexpr bool kSpan = false;
   static constexpr bool kBand = kWindow;                    // yields band tiles (mode 5) under the rolling policy
-  int q0, q_last, qb, C, per, tpb, ct, plen, qmin, qmax, n_tiles, tail;
+  int q0, q_last, qb, C, per, tpb, ct, plen, qmin, qmax, tail;
   bool q_code;
   int kb, tw;
   int wq0, wq1;                                             // code quotas of this wave's two heads
@@ -66,7 +64,7 @@ struct TileWalk {
                                                             // this query tile sees (kWindow)
   bool rolling;
 
-  __device__ __forceinline__ TileWalk(int q0_, int q_last_, int C_, int per_, int S0, int plen_, int qmin_, int qmax_,
+  __device__ __forceinline__ TileWalk(int q0_, int q_last_, int C_, int per_, int plen_, int qmin_, int qmax_,
                                       int wq0_, int wq1_, int tail_ = 0, int policy_ = kTailStatic)
       : q0(q0_), q_last(q_last_), C(C_), per(per_), plen(plen_), qmin(qmin_), qmax(qmax_), tail(kTail ? tail_ : 0),
         kb(0), tw(0), wq0(wq0_), wq1(wq1_) {
@@ -74,7 +72,6 @@ struct TileWalk {
     q_code = q0 - qb * per >= C;
     tpb = per / kBN;
     ct = C / kBN;
-    n_tiles = (S0 + kBN - 1) / kBN;
     rolling = kWindow && policy_ == kTailRolling;
     first_tail = C - tail + (rolling ? q0 - qb * per : 0);
   }
@@ -157,20 +154,41 @@ struct TileWalk {
   }
 
   // next tile to attend (the first call gives the first); false when the walk is done
-  __device__ __forceinline__ bool next(int& kt, TileMask& tm, bool first) {
-    if constexpr (kAligned) {
-      if (!first) ++tw;
-      if (!seek()) return false;
-      kt = kb * tpb + tw;
-      mask(tm);
-      return true;
-    } else {
-      kt = first ? 0 : kt + 1;
-      tm.mode = 3;
-      // keys up to the query tile's last row, or in a block up to its own (codes of the own block): a prefix
-      return kt < n_tiles && (kt * kBN <= q_last || (kt * kBN) / per <= q_last / per);
-    }
+  __device__ __forceinline__ bool next(int& k0, TileMask& tm, bool first) {
+    if (!first) ++tw;
+    if (!seek()) return false;
+    k0 = kb * per + kBN * tw;
+    mask(tm);
+    return true;
   }
+};
+
+// The mask's geometry from the kernel arguments.
+__device__ __forceinline__ MaskShape mask_shape(const PrefillArgs& a) {
+  return MaskShape{a.S0, a.C, a.K, a.L, a.R, a.copy, a.C + a.L * a.K + a.R, a.N, a.tail, a.policy, a.xattn, a.rx != 0};
+}
+
+// Key walk and per-lane mask facts of a wave (query tile q0 .. q_last, lane row qrow, heads with code quotas wq0, wq1).
+template <bool kAligned, bool kTail, bool kWindow>
+struct MaskWalk;
+template <bool kTail, bool kWindow>
+struct MaskWalk<true, kTail, kWindow> {
+  typedef TileWalk<kTail, kWindow> Walk;
+  Walk walk;
+  CausalLane lane;
+  __device__ __forceinline__ MaskWalk(const PrefillArgs& a, int q0, int q_last, int qrow, int plen, int qmin, int qmax,
+                                      int wq0, int wq1)
+      : walk(q0, q_last, a.C, a.C + a.K, plen, qmin, qmax, wq0, wq1, a.tail, a.policy), lane{qrow + 1} {}
+};
+template <>
+struct MaskWalk<false, false, false> {
+  typedef SegWalk Walk;
+  Walk walk;
+  SpanLane<2> lane;
+  __device__ __forceinline__ MaskWalk(const PrefillArgs& a, int q0, int q_last, int qrow, int plen, int qmin, int qmax,
+                                      int wq0, int wq1)
+      : walk(mask_shape(a), q0, q_last, plen, qmin, qmax, wq0, wq1),
+        lane{qrow + 1, mask_shape(a), row_facts(mask_shape(a), qrow), plen, {wq0, wq1}} {}
 };
 
 // Linear grid of the prefill kernels (grid_pos): num_q_tiles x 8 x batch workgroups; 0 when the launch's work-item
