@@ -18,7 +18,7 @@ every decoder layer runs ``abkv_prefill_masked_attn`` through a HuggingFace atte
 ``"abridgekv_hip"`` in place of FlexAttention with a BlockMask (``_arith_mask_mod`` / ``_mask_mod`` /
 ``_mask_rawprompt_mod`` / ``_quota_key_allowed``, compress_forward.py:230-236, 566-649, 695-727, 815-894). The mask
 is never materialised: the kernel evaluates it from (C, K, L, R, N, prompt_len, head quota, tail, xattn); layouts off
-the 64-row tile grid, L > 1, replay rows, the raw tail and non-full xattn take its per-element walk.
+the 64-row tile grid, L > 1, replay rows, the raw tail and non-full xattn take its walk over segments.
 
 The raw tail (``raw_tail`` = W, a training ablation the reference's serving refuses, compress_forward.py:89-96):
 content row i of the next block sees the block's last W - i content rows (the rolling window of a retained tail),

@@ -278,4 +278,52 @@ struct SegWalk {
   }
 };
 
+// The query rows that see one key: [a1, e1) and [a2, e2) (empty ranges are [0, 0)); a code key only for heads whose
+// quota exceeds its slot.
+struct KeySpan {
+  int a1, e1, a2, e2;
+  int slot;          // index within its pass, -1 for a key that is no code
+};
+ABKV_HD KeySpan key_span(const MaskShape& g, int key, int plen) {
+  KeySpan s{0, 0, 0, 0, -1};
+  if (key >= g.S0) return s;
+  const int rows = g.block_rows();
+  if (key >= rows) {                                          // copy rows: themselves, causally
+    s.a1 = key;
+    s.e1 = g.S0;
+    return s;
+  }
+  const int kb = key / g.per, kw = key - kb * g.per;
+  const int b0 = kb * g.per, b1 = b0 + g.per, ce = b0 + g.code_end();
+  if (kw < g.C) {
+    const bool hidden = kw >= g.C - g.hidden();               // from its own block's codes
+    s.a1 = key;
+    s.e1 = hidden ? b0 + g.C : b1;
+    s.a2 = hidden ? ce : b1;
+    s.e2 = b1;                                                // then the own block's replay rows
+    const int t = kw - (g.C - g.tail);                        // index in the retained tail
+    if (kb * g.C + kw < plen) s.e2 = rows;
+    else if (g.tail > 0 && t >= 0)
+      s.e2 = imin(rows, g.policy == kTailStatic ? rows : b1 + (g.policy == kTailSticky ? g.C : t + 1));
+  } else if (b0 + kw < ce) {
+    const int p = (kw - g.C) / g.K, p0 = b0 + g.C + p * g.K, p1 = p0 + g.K;
+    s.slot = kw - g.C - p * g.K;
+    s.a1 = g.xattn == kXattnFull ? p0 : g.xattn == kXattnCausal ? key : p1;
+    s.e1 = p1;
+    s.a2 = p1;
+    s.e2 = p + 1 < g.L ? p1 + g.K : kb == g.N - 1 ? g.S0 : rows;
+  } else {                                                    // replay row r: its block's later ones, and content rows
+    s.a1 = key;                                               // 0 .. r of the next block
+    s.e1 = imin(rows, b1 + (b0 + kw - ce) + 1);
+    if (kb == g.N - 1) s.e1 = b1;
+  }
+  if (s.e1 >= s.a2 && s.a2 < s.e2) {                          // adjoining ranges: one
+    s.e1 = imax(s.e1, s.e2);
+    s.a2 = s.e2 = 0;
+  }
+  if (s.a1 >= s.e1) s.a1 = s.e1 = 0;
+  if (s.a2 >= s.e2) s.a2 = s.e2 = 0;
+  return s;
+}
+
 }  // namespace abkv

@@ -28,8 +28,7 @@
 // code attention) walk key tiles that start at each visible segment (SegWalk, mask_walk.h): bounded by tile count like
 // the aligned walk, at most one ragged tile a segment; only tiles whose rows lie in several segments, or that meet a
 // window tail or replay rows, evaluate a span per row. Before, they walked every tile up to the query's block with the
-// mask's predicate per element. Forward and dQ of B=1, 8 x (512 + 128 codes + 16 replay rows), one kernel each:
-// 2936 + 2760 us before, about 165 us each now.
+// mask's predicate per element. B=1, 8 x (512 + 128 codes + 16 replay rows): forward 2936 -> 147 us, dQ 2760 -> 208 us.
 #include "prefill_common.h"
 
 namespace abkv {

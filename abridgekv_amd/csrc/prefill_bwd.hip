@@ -8,7 +8,11 @@
 //                            2 heads); per key tile S^T = K Q^T and dP^T = V dO^T, dQ^T += K^T dS^T
 //   prefill_bwd_dkv_kernel   roles swapped: workgroup = 64 keys of a KV head, wave = 16 keys; the (query tile, head)
 //                            pairs that see the key tile are staged in LDS (Q, dO, lse2, D); S = Q K^T and
-//                            dP = dO V^T as the forward's score tiles, dV^T += dO^T P and dK^T += Q^T dS as its PV step
+//                            dP = dO V^T as the forward's score tiles, dV^T += dO^T P and dK^T += Q^T dS as its PV step.
+//                            A key is seen by at most two ranges of query rows in every layout (key_span), so one
+//                            instance serves all of them and a mask test is two range tests per element: 3220 -> 583 us
+//                            (layouts off the 64-row grid, B=1, 8 x (512 + 128 + 16 rows)); on the grid, where it
+//                            replaced a classification per tile pair, 988 -> 965 us (B=2, 12 x (512 + 128 rows))
 #include "prefill_common.h"
 
 namespace abkv {
@@ -209,79 +213,46 @@ __global__ __launch_bounds__(512, 1) void prefill_bwd_dq_kernel(PrefillBwdArgs a
   }
 }
 
-// Visibility of the 64-key tile kt to the 64-row query tile qt for a head of code quota qh, aligned layouts (C, K
-// multiples of 64; the classification of the forward's TileWalk::seek / mask for one key tile): -1 hidden, 0 every
-// pair visible, 1 key <= query, 2 key < lim0 (without a tail the per-element predicate decides these tiles),
-// kTail: 4 key outside [lim0, lim1) (the tile of an earlier block where hidden rows give way to its retained tail).
-// kWindow (rolling / sticky tails: only the next block's content tiles see a block's tail): rolling, 5 key < lim0 or
-// key - query >= lim1 (query row i of the block sees tail rows i..).
-template <bool kTail, bool kWindow>
-__device__ __forceinline__ int pair_mode(int qt, int kt, int qh, int S0, int C, int per, int plen, int tail,
-                                         bool rolling, int& lim0, int& lim1) {
-  const int q0 = qt * kBN, k0 = kt * kBN;
-  const int qb = q0 / per, kb = k0 / per;
-  if (kb > qb) return -1;
-  const bool q_code = q0 - qb * per >= C;
-  const int tw = (k0 - kb * per) / kBN, ct = C / kBN;
-  if (tw < ct) {
-    if (kb == qb) {
-      if (kTail && q_code) {                                // codes see their block's content below C - T
-        const int lo = kBN * tw;
-        if (lo >= C - tail) return -1;
-        if (lo + kBN > C - tail) {
-          lim0 = kb * per + C - tail;
-          return 2;
-        }
-        return 0;
-      }
-      const int q_last = min(q0 + kBN, S0) - 1;
-      if (!(q_code || k0 <= q_last)) return -1;
-      return (!q_code && k0 + kBN - 1 > q0) ? 1 : 0;
-    }
-    if constexpr (kTail) {
-      const int pl = min(max(plen - kb * C, 0), C);         // raw-prompt rows of this block's content
-      const int lo = kBN * tw, hi = lo + kBN;
-      if constexpr (kWindow) {
-        if (hi <= pl) return 0;                             // all prompt
-        const int first = C - tail + (rolling ? q0 - qb * per : 0);   // first tail row the query tile sees
-        if (q_code || kb + 1 != qb || first >= C || hi <= C - tail) {  // no tail rows seen: a prompt prefix or nothing
-          if (lo >= pl) return -1;
-          lim0 = kb * per + pl;
-          return 2;
-        }
-        if (rolling) {
-          if (lo >= pl && hi <= first) return -1;           // no prompt row, no row of any query row's band
-          if (lo >= first + kBN - 1) return 0;              // past every query row's band start
-          lim0 = kb * per + pl;
-          lim1 = C - tail - per;
-          return 5;
-        }
-      }
-      if (hi <= pl || lo >= C - tail) return 0;             // all prompt, or all tail
-      if (hi <= C - tail) {                                 // no tail rows: a prompt prefix or nothing
-        if (lo >= pl) return -1;
-        lim0 = kb * per + pl;
-        return 2;
-      }
-      if (pl >= C - tail) return 0;                         // prompt rows up to the tail
-      lim0 = kb * per + pl;                                 // [prompt rows,] hidden rows, tail rows
-      lim1 = kb * per + C - tail;
-      return 4;
-    }
-    if (kb * C + kBN * tw >= plen) return -1;
-    if (kb * C + kBN * tw + kBN > plen) {
-      lim0 = kb * per + (plen - kb * C);
-      return 2;
-    }
-    return 0;
-  }
-  if (!(kb < qb || q_code) || kBN * (tw - ct) >= qh) return -1;
-  if (kBN * (tw - ct) + kBN > qh) {
-    lim0 = kb * per + C + qh;
-    return 2;
-  }
-  return 0;
+// Smallest v over the wave's lanes.
+__device__ __forceinline__ int wave_min(int v) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v = min(v, __shfl_xor(v, m, 64));
+  return __builtin_amdgcn_readfirstlane(v);
 }
+
+// Which query tiles a 64-key tile is seen by, from the query ranges of its keys (lane l: key k0 + l; wave-uniform and
+// the same in every wave): a query tile outside the hulls of the ranges is hidden, one inside the common part of the
+// first (or of the second) ranges of all 64 keys is visible throughout, the others take the ranges per key.
+struct TileSpan {
+  int a1, e1, a2, e2;        // hulls over the keys that are no codes
+  int ca, ce;                // hull over the codes
+  int f1, g1, f2, g2;        // [f1, g1) and [f2, g2): rows that see every key (given the quota)
+  int slot_min, slot_max;    // of the codes
+  __device__ __forceinline__ explicit TileSpan(const KeySpan& s) {
+    const bool code = s.slot >= 0;
+    const bool r1 = s.a1 < s.e1, r2 = s.a2 < s.e2;
+    a1 = wave_min(!code && r1 ? s.a1 : kNoKey);
+    e1 = -wave_min(!code && r1 ? -s.e1 : 0);
+    a2 = wave_min(!code && r2 ? s.a2 : kNoKey);
+    e2 = -wave_min(!code && r2 ? -s.e2 : 0);
+    ca = wave_min(code && r1 ? s.a1 : code && r2 ? s.a2 : kNoKey);
+    ce = -wave_min(code ? -max(s.e1, s.e2) : 0);
+    f1 = -wave_min(-s.a1);
+    g1 = wave_min(s.e1);
+    f2 = -wave_min(-s.a2);
+    g2 = wave_min(s.e2);
+    slot_min = wave_min(code ? s.slot : kNoKey);
+    slot_max = -wave_min(-s.slot);
+  }
+  __device__ __forceinline__ int first_row() const { return min(min(a1, a2), ca); }
+  __device__ __forceinline__ int last_row() const { return max(max(e1, e2), ce); }
+  // -1 hidden, 0 every pair visible, 1 per key
+  __device__ __forceinline__ int mode(int q0, int q1, int quota) const {
+    const bool seen = (q0 < e1 && q1 > a1) || (q0 < e2 && q1 > a2) || (slot_min < quota && q0 < ce && q1 > ca);
+    if (!seen) return -1;
+    return ((q0 >= f1 && q1 <= g1) || (q0 >= f2 && q1 <= g2)) && slot_max < quota ? 0 : 1;
+  }
+};
 
 // S = Q K^T and dP = dO V^T of a wave's 16 keys over one staged tile (32 ds_read_b128, 32 MFMAs). The two products
 // are interleaved and the reads run eight ahead of the MFMAs: at 2 waves per SIMD the other wave alone cannot cover
@@ -337,11 +308,11 @@ __device__ __forceinline__ void dkv_acc(const __bf16* Qbuf, const __bf16* Gbuf, 
   __builtin_amdgcn_sched_group_barrier(0x008, 4, 1);
 }
 
-template <bool kAligned, bool kTail, bool kWindow>
 __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs a) {
   constexpr int kWaves = 4;
   __shared__ __attribute__((aligned(16))) __bf16 Q0[kTileElems], Q1[kTileElems], G0[kTileElems], G1[kTileElems];
   __shared__ __attribute__((aligned(16))) float L0[kBN], L1[kBN], E0[kBN], E1[kBN];
+  __shared__ KeySpan key_spans[kBN];
   __bf16* const Qb[2] = {Q0, Q1};
   __bf16* const Gb[2] = {G0, G1};
   float* const Lb[2] = {L0, L1};
@@ -354,13 +325,14 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int m16 = lane & 15, j = lane >> 4;
-  const int per = kAligned ? f.C + f.K : f.C + f.L * f.K + f.R;
   const int k0 = kt * kBN;
   const int key = k0 + 16 * w + m16;                        // this lane's column
   const int plen = f.prompt_len ? f.prompt_len[b] : 0;
-  int quota_all[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) quota_all[u] = f.head_quota ? f.head_quota[kvh * kGroup + u] : f.K;
+  // the four heads' code quotas, two to a register pair (an indexed array would live in scratch memory)
+  auto quota_of = [&](int u) { return f.head_quota ? f.head_quota[kvh * kGroup + u] : f.K; };
+  auto pair_of = [&](int u) { return (uint64_t)(uint32_t)quota_of(u) | (uint64_t)(uint32_t)quota_of(u + 1) << 32; };
+  const uint64_t quota01 = pair_of(0), quota23 = pair_of(2);
+  auto head_quota = [&](int u) { return (int)(uint32_t)((u & 2 ? quota23 : quota01) >> (32 * (u & 1))); };
 
   bf16x8 kop[4], vop[4];
   {
@@ -380,28 +352,14 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
 #pragma unroll
   for (int i = 0; i < 8; ++i) dk[i][0] = dv[i][0] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // (query tile, head) pairs that can see this key tile, head fastest; queries start at the key's block
-  const int qt_lo = (k0 / per) * per / kBN;
-  // aligned: a content tile outside the raw prompt and the retained tail is seen by its own block's rows only, so
-  // the walk ends there
-  const int tail = kTail ? f.tail : 0;
-  int qt_end = f.num_q_tiles;
-  if (kAligned && k0 - (k0 / per) * per + kBN <= f.C - tail && (k0 / per) * f.C + (k0 - (k0 / per) * per) >= plen)
-    qt_end = min(qt_end, (k0 / per + 1) * per / kBN);
-  if constexpr (kWindow) {                                  // a window tail: the next block's rows at most
-    if (k0 - (k0 / per) * per < f.C && (k0 / per) * f.C + (k0 - (k0 / per) * per) >= plen)
-      qt_end = min(qt_end, (k0 / per + 2) * per / kBN);
-  }
-  const bool rolling = kWindow && f.policy == kTailRolling;
-  // the per-element predicate's tail: none in the aligned no-tail instance, static in the aligned static one
-  const int etail = kAligned && !kTail ? 0 : f.tail;
-  const int epolicy = kAligned && !kWindow ? kTailStatic : f.policy;
-  const int exattn = kAligned ? kXattnFull : f.xattn;
-  const int epasses = kAligned ? 1 : f.L;
-  const int ecopy = kAligned ? 0 : f.copy;
-  const int erep = kAligned ? 0 : f.R;
-  const bool erx = !kAligned && f.rx;
-  int qt = qt_lo, h = -1, mode = 0, lim0 = 0, lim1 = 0;
+  // (query tile, head) pairs that can see this key tile, head fastest
+  const MaskShape shape = mask_shape(f);
+  const KeySpan lane_key = key_span(shape, k0 + lane, plen);
+  if (w == 0) key_spans[lane] = lane_key;                   // read by masked tiles (held in registers it spills);
+                                                            // published by the first step's barrier
+  const TileSpan span(lane_key);
+  const int qt_end = (span.last_row() + kBN - 1) / kBN;
+  int qt = span.first_row() / kBN, h = -1, mode = 0;
   auto next_pair = [&]() -> bool {
     for (;;) {
       if (++h == kGroup) {
@@ -409,14 +367,8 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
         ++qt;
       }
       if (qt >= qt_end) return false;
-      if constexpr (kAligned) {
-        const int qh = h == 0 ? quota_all[0] : h == 1 ? quota_all[1] : h == 2 ? quota_all[2] : quota_all[3];
-        mode = pair_mode<kTail, kWindow>(qt, kt, qh, f.S0, f.C, per, plen, tail, rolling, lim0, lim1);
-        if (mode >= 0) return true;
-      } else {
-        mode = 3;
-        return true;
-      }
+      mode = span.mode(qt * kBN, min(qt * kBN + kBN, f.S0), head_quota(h));
+      if (mode >= 0) return true;
     }
   };
   // Q / dO rows of (qt, head) as the tile rows, lse2 / D rows beside them (waves 0 and 1, 4 bytes per lane)
@@ -436,14 +388,12 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
     auto step = [&](auto buf_c) -> bool {
       constexpr int sl = decltype(buf_c)::value;
       const int cq = qt, ch = h, cmode = mode;
-      const int clim0 = kTail ? lim0 : 0, clim1 = kTail ? lim1 : 0;
       const bool hn = next_pair();
       __asm__ volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       if (hn) issue(qt, h, 1 - sl);
       floatx4 s[2][2][1], dp[2][2][1];
       dkv_scores(Qb[sl], Gb[sl], kop, vop, s, dp, m16, j);
-      const int qh = ch == 0 ? quota_all[0] : ch == 1 ? quota_all[1] : ch == 2 ? quota_all[2] : quota_all[3];
       if (cmode == 0) {                                     // wave-uniform: every pair of the tile visible
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
@@ -459,24 +409,10 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
               dp[kk][t][0][r] = pr * (dp[kk][t][0][r] - e4[r]);
             }
           }
-      } else if (kTail && (cmode == 2 || cmode == 4)) {     // visibility independent of the query row
-        // mode 2 key < lim0; mode 4 key outside [lim0, lim1): one flag for this lane's key column
-        const bool vis = cmode == 2 ? key < clim0 : (key < clim0 || key >= clim1);
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            const int r0 = 32 * kk + 16 * t + 4 * j;
-            const floatx4 l4 = *reinterpret_cast<const floatx4*>(Lb[sl] + r0);
-            const floatx4 e4 = *reinterpret_cast<const floatx4*>(Eb[sl] + r0);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float pr = vis ? fast_exp2(fmaf(s[kk][t][0][r], f.scale_log2, -l4[r])) : 0.f;
-              s[kk][t][0][r] = pr;
-              dp[kk][t][0][r] = pr * (dp[kk][t][0][r] - e4[r]);
-            }
-          }
-      } else {
+      } else {                                              // the rows that see this lane's key
+        const KeySpan ks = key_spans[16 * w + m16];
+        const bool slot_ok = ks.slot < head_quota(ch);
+        const unsigned m1 = slot_ok ? ks.e1 - ks.a1 : 0, m2 = slot_ok ? ks.e2 - ks.a2 : 0;
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -487,13 +423,7 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int qrow = cq * kBN + r0 + r;
-              // diagonal tiles: key <= row; a rolling tail's band (mode 5); bounded (mode 2, no tail) and unaligned
-              // tiles: the per-element predicate
-              const bool vis = cmode == 1                   ? key <= qrow
-                               : (kWindow && cmode == 5) ? (key < clim0 || key - qrow >= clim1)
-                                                         : compress_visible(qrow, key, f.S0, ecopy, f.C, f.K,
-                                                                            epasses, per, plen, qh, etail, epolicy,
-                                                                            exattn, erep, erx);
+              const bool vis = (unsigned)(qrow - ks.a1) < m1 || (unsigned)(qrow - ks.a2) < m2;
               const float pr = vis ? fast_exp2(fmaf(s[kk][t][0][r], f.scale_log2, -l4[r])) : 0.f;
               s[kk][t][0][r] = pr;
               dp[kk][t][0][r] = pr * (dp[kk][t][0][r] - e4[r]);
@@ -615,12 +545,7 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
   err = hipGetLastError();
   if (err != hipSuccess) return (int)err;
   const unsigned gk = prefill_grid(f.num_q_tiles, batch, 256);
-  if (f.aligned && retain_tail == 0)
-    hipLaunchKernelGGL((prefill_bwd_dkv_kernel<true, false, false>), gk, dim3(256), 0, stream, a);
-  else if (f.aligned && !window)
-    hipLaunchKernelGGL((prefill_bwd_dkv_kernel<true, true, false>), gk, dim3(256), 0, stream, a);
-  else if (f.aligned) hipLaunchKernelGGL((prefill_bwd_dkv_kernel<true, true, true>), gk, dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL((prefill_bwd_dkv_kernel<false, false, false>), gk, dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(prefill_bwd_dkv_kernel, gk, dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 

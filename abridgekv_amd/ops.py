@@ -399,7 +399,7 @@ def prefill_masked_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
                              copy_rows: int = 0, replay_rows: int = 0, replay_exclude: bool = False):
     """Teacher-forced attention under the compression mask (N blocks of [C content | L passes of K codes],
     L = ``pause_passes``: pass l reads its block's content, its pass l - 1 and its own pass by ``pause_xattn``; later
-    blocks read the final pass only; L > 1 evaluates the mask per element), ``replay_rows`` = R replay rows after each
+    blocks read the final pass only), ``replay_rows`` = R replay rows after each
     block's codes (a block's last R content tokens again: they see their block and its final pass; content row i of
     the next block sees them from row i on; ``replay_exclude`` hides the last R content rows from the codes), then
     ``copy_rows`` rows of a copy region that see the last block's final pass and themselves causally. ``codes_k`` = 0:
@@ -411,8 +411,7 @@ def prefill_masked_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     content rows, hidden from its own codes) and ``tail_policy`` the later rows that see it: "static" every later row,
     "sticky" the next block's content rows, "rolling" the next block's i-th content row from tail row i on, "raw"
     (CompressLM's raw_tail, T <= C) as rolling but not hidden from the codes;
-    ``pause_xattn`` a code row's attention to its block's code rows ("full", "causal", "none"; the non-full ones
-    evaluate the mask per element). Returns
+    ``pause_xattn`` a code row's attention to its block's code rows ("full", "causal", "none"). Returns
     (out [B, S0, 32, 128] bf16, lse [B, 32, S0] fp32 natural log or None). fp32 q/k/v select the fp32 mode (out fp32).
     """
     B, S0 = q.shape[0], q.shape[1]

@@ -131,7 +131,7 @@ int abkv_slot_mapping(const int32_t* req_idx, const int64_t* positions, int num_
  * layout N blocks of [block_c content | pause_passes passes of codes_k codes], seq_len = N * (block_c + pause_passes
  * * codes_k) (L = pause_passes, compress_forward.py:20-31, 566-649: pass l of a block reads its block's content, its
  * pass l - 1 and its own pass (by pause_xattn); later blocks read only the final pass; the quota counts a code row's
- * slot within its pass; L > 1 runs the per-element mask).
+ * slot within its pass).
  * q [batch, seq_len, 32, 128], k/v [batch, seq_len, 8, 128], out [batch, seq_len, 32, 128] bf16 with element strides
  * (dims contiguous); prompt_len [batch] int32 raw-prompt content tokens (NULL: none); head_quota [32] int32 code slots
  * visible per query head (NULL: all); retain_tail = T of a retained tail (retain_tail_kv; 0: none; 0 <= T <
@@ -140,7 +140,7 @@ int abkv_slot_mapping(const int32_t* req_idx, const int64_t* positions, int num_
  * later row, ABKV_TAIL_STICKY every content row of the next block, ABKV_TAIL_ROLLING content row i of the next block
  * from tail row i on (key in-block offset >= block_c - T + i); ABKV_TAIL_RAW is CompressLM's raw_tail = T
  * (_raw_tail_visible, compress_forward.py:89-96; 0 <= T <= block_c): the rolling window, with the codes seeing their
- * whole block (code_excluded_tail = 0, :309-311), on the per-element mask; lse [batch, 32, seq_len] fp32 natural log
+ * whole block (code_excluded_tail = 0, :309-311); lse [batch, 32, seq_len] fp32 natural log
  * (NULL: not written).
  * ------------------------------------------------------------------------------------------------------------- */
 #define ABKV_TAIL_STATIC 0
@@ -149,7 +149,7 @@ int abkv_slot_mapping(const int32_t* req_idx, const int64_t* positions, int num_
 #define ABKV_TAIL_RAW 3
 /* pause_xattn: a code row's attention to its own block's code rows (compress_forward.py:313-314, 622-625): all of
  * them (ABKV_XATTN_FULL, the served setting), those at or before its own row (ABKV_XATTN_CAUSAL), none
- * (ABKV_XATTN_NONE). The non-full settings run the per-element mask on every tile up to the query's block. */
+ * (ABKV_XATTN_NONE). */
 #define ABKV_XATTN_FULL 0
 #define ABKV_XATTN_CAUSAL 1
 #define ABKV_XATTN_NONE 2

@@ -62,4 +62,18 @@ long walk_counts(const int32_t* params, int plen, const int32_t* quota, uint8_t*
   return tiles;
 }
 
+// counts [4][S0][S0] from the query ranges of every key.
+void key_counts(const int32_t* params, int plen, const int32_t* quota, uint8_t* counts) {
+  const MaskShape g = shape(params);
+  const long S = g.S0;
+  for (int key = 0; key < g.S0; ++key) {
+    const KeySpan k = key_span(g, key, plen);
+    for (int u = 0; u < 4; ++u) {
+      if (k.slot >= quota[u]) continue;
+      for (int q = k.a1; q < k.e1; ++q) ++counts[(u * S + q) * S + key];
+      for (int q = k.a2; q < k.e2; ++q) ++counts[(u * S + q) * S + key];
+    }
+  }
+}
+
 }

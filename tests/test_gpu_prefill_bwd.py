@@ -126,6 +126,14 @@ def test_replay_rows(exclude):
     _check(C=128, K=64, N=3, B=2, prompt_len=[100, 0], head_quota=quota, seed=40, replay=16, replay_exclude=exclude)
 
 
+@pytest.mark.parametrize("C,K,R,passes,copy", [(63, 65, 0, 1, 0), (65, 1, 0, 1, 0), (192, 64, 16, 1, 0),
+                                               (130, 63, 5, 2, 0), (64, 64, 1, 1, 129), (200, 40, 64, 1, 0)])
+def test_segments_around_the_tile_size(C, K, R, passes, copy):
+    """Content, code, replay and copy segments one row short of, at and past the 64-row tiles (test tolerance)."""
+    _check(C=C, K=K, N=3, B=2, prompt_len=[C + 7, 0], seed=47, replay=R, passes=passes, copy_rows=copy,
+           head_quota=np.repeat([K, 1, (K + 1) // 2, K, K, 1, K, K], 4).tolist())
+
+
 @pytest.mark.parametrize("W", [20, 128])
 def test_raw_tail(W):
     """The raw tail (the rolling window that the codes also see), up to the whole block."""

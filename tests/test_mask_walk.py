@@ -1,4 +1,4 @@
-"""The key-tile walk and the per-row key ranges of the masked kernels (csrc/mask_walk.h, built for the host) against the
+"""The key-tile walk, the per-row key ranges and the per-key query ranges of the masked kernels (csrc/mask_walk.h, built for the host) against the
 compression mask: every visible (query, key) pair is covered exactly once, no hidden one ever, over the block layouts,
 tails, replay rows, passes, copy rows, prompts and quotas that the kernels take."""
 import ctypes as C
@@ -83,5 +83,11 @@ def test_walk_covers_the_mask_once(harness, case):
     n = harness.walk_counts(_params(case), case["plen"], (C.c_int32 * 4)(*quota),
                             counts.ctypes.data_as(C.POINTER(C.c_uint8)))
     assert n >= 0
-    bad = np.argwhere(counts != _mask(case, quota))
+    mask = _mask(case, quota)
+    bad = np.argwhere(counts != mask)
+    assert bad.size == 0, (bad[:5].tolist(), len(bad))
+    counts[:] = 0
+    harness.key_counts(_params(case), case["plen"], (C.c_int32 * 4)(*quota),
+                       counts.ctypes.data_as(C.POINTER(C.c_uint8)))
+    bad = np.argwhere(counts != mask)
     assert bad.size == 0, (bad[:5].tolist(), len(bad))
