@@ -3,9 +3,9 @@
 // Same semantics as the bf16 kernels (decode_attn.hip, paged_prefill.hip, prefill_attn.hip), with fp32 queries,
 // keys, values and outputs, fp32 accumulation in a fixed order and accurate expf/logf: the mode the reference's
 // PyTorch paths run in fp32 (abridgekv/gen_compress.py:359-360, 555; compresslm_packed_kv.py:608-613;
-// compress_forward.py:695-727 under FlexAttention) for tight parity checks. It is a correctness mode: plain VALU
-// arithmetic, one wave per (query token, KV head), keys in tiles of 64 (lane = key for QK^T, lane = 2 output dims for
-// PV with the tile's probabilities broadcast from LDS).
+// compress_forward.py:695-727 under FlexAttention) for tight parity checks. Every product is a fp32 matrix instruction
+// (v_mfma_f32_16x16x4_f32: fp32 inputs, fp32 sums). Masked B=1, 3 x (512 + 128) rows, 200 raw prompt rows: 1546 -> 228 us
+// a call against one wave per (token, KV head) of VALU dot products with the mask's predicate per key.
 #include <cstring>
 
 #include "common.h"
@@ -13,20 +13,19 @@
 namespace abkv {
 
 struct F32Args {
-  int mode;                    // 0: paged, per-request key limits; 1: dense, compression mask; 2: paged decode
   const float* q;
-  long q_sb, q_st, q_sh;       // mode 1: [B, S, 32, 128]; modes 0/2: [T, 32, 128] (q_sb unused)
-  // paged keys (modes 0 and 2): [num_pages, 2, 16, 8, 128]
+  long q_sb, q_st, q_sh;       // masked: [B, S, 32, 128]; paged and decode: [T, 32, 128] (q_sb unused)
+  // paged keys (paged and decode): [num_pages, 2, 16, 8, 128]
   const float* kv;
   int num_pages;
   const int32_t* block_table;
   long bt_stride;
   int bt_width;
-  // dense keys (mode 1): [B, S, 8, 128]
+  // dense keys (masked): [B, S, 8, 128]
   const float* k;
   const float* v;
   long k_sb, k_ss, k_sh, v_sb, v_ss, v_sh;
-  // mode 0
+  // paged: per-request key limits
   const int32_t* tok_req;      // [T] request of every query token
   const int32_t* q_start;      // [B + 1]
   const int32_t* kv_start;     // [B]
@@ -34,11 +33,11 @@ struct F32Args {
   const int32_t* kv_excluded;  // [B][2] physical [start, end) hidden from the request, or nullptr
   const int32_t* causal;       // [B] or nullptr (causal_default)
   int causal_default;
-  // mode 2
+  // decode
   const int32_t* seq_lens;     // [B]
   int max_pages;
-  // mode 1
-  int block_c, codes_k, seq_len;
+  // masked
+  int batch, num_blocks, block_c, codes_k, seq_len;
   const int32_t* prompt_len;   // [B] or nullptr
   const int32_t* head_quota;   // [32] or nullptr
   int retain_tail;             // retained tail T (0: none)
@@ -52,178 +51,414 @@ struct F32Args {
   float scale;
   float* out;
   long o_sb, o_st, o_sh;
-  float* lse;                  // modes 0/2: [T, 32]; mode 1: [B, 32, S]; or nullptr
+  float* lse;                  // paged and decode: [T, 32]; masked: [B, 32, S]; or nullptr
 };
 
-constexpr int kF32Waves = 4;
-
-// LDS written by some lanes of a wave and read by others: order the accesses within the wave.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// Unaligned-safe vector access (rows are 4-byte aligned at least).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ floatx4 ldf4(const float* p) { return *reinterpret_cast<const f32x4u*>(p); }
+__device__ __forceinline__ void stf4(float* p, const floatx4& x) { *reinterpret_cast<f32x4u*>(p) = x; }
+__device__ __forceinline__ floatx4 mfma16x16x4(float a, float b, const floatx4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Compression-mask visibility of key row kr for query row qr (L = 1; _arith_mask_mod, abridgekv/compress_forward.py:
-// 695-727, with the retained-tail term of _retained_tail_visible :99-124):
-//   (k <= q) & (own-block content | earlier blocks' codes | raw-prompt content | earlier blocks' tail rows the policy
-//   shows this row) | (code q & code k & same block), a code query never sees its own block's last T content rows,
-//   and a code key of slot s is visible to a head only if s < quota.
-__device__ __forceinline__ bool f32_visible(const F32Args& a, int qr, int kr, int plen, int quota) {
-  return compress_visible(qr, kr, a.seq_len, a.copy_rows, a.block_c, a.codes_k, a.pause_passes,
-                          a.block_c + a.pause_passes * a.codes_k + a.replay_rows, plen, quota, a.retain_tail,
-                          a.tail_policy, a.pause_xattn, a.replay_rows, a.replay_exclude != 0);
-}
+constexpr int kF32Rows = 16;             // query rows of a workgroup (MFMA columns of each of its waves)
+constexpr int kF32Keys = 32;             // keys per LDS stage
+constexpr int kF32StageElems = kF32Keys * kHeadDim;
+constexpr float kF32Headroom = 8.f;      // the running max moves only when a score exceeds it by more (p <= e^8)
 
-__global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(F32Args a) {
-  __shared__ float q_lds[kF32Waves][kGroup][kHeadDim];
-  __shared__ float p_lds[kF32Waves][kGroup][64];
-  const int w = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * kF32Waves + w;          // query token (mode 1: b * seq_len + row)
-  const int kvh = blockIdx.y;
-  if (t >= a.num_tokens) return;                      // whole wave exits together; no block barrier below
-
-  // Which keys, and how a key row is addressed.
-  int b = 0, qrow = 0, n_keys = 0, lim_lane = 0, plen = 0, ex_lo = 0, ex_hi = 0;
-  const int32_t* table = nullptr;
-  int quota[kGroup] = {1 << 30, 1 << 30, 1 << 30, 1 << 30};
-  if (a.mode == 1) {
-    b = t / a.seq_len;
-    qrow = t - b * a.seq_len;
-    const int per = a.block_c + a.pause_passes * a.codes_k + a.replay_rows;
-    const int s0 = a.seq_len - a.copy_rows;
-    // nothing after the query's own block is visible; a copy row sees up to itself
-    n_keys = qrow >= s0 ? qrow + 1 : min(s0, (qrow / per + 1) * per);
-    plen = a.prompt_len ? a.prompt_len[b] : 0;
-    if (a.head_quota)
+// Scores of 16 keys x 16 columns: s[r] = q(column m16) . k(key 4g + r). The operands' contraction order is dim
+// 16c + 4g + e at step (c, e), so a lane's K and Q are 16-byte pieces; two accumulators halve the length of the sums.
+__device__ __forceinline__ floatx4 f32_scores(const floatx4 (&kx)[8], const floatx4 (&q)[8]) {
+  floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u) quota[u] = a.head_quota[kvh * kGroup + u];
-  } else if (a.mode == 0) {
-    b = a.tok_req[t];
-    const int i = t - a.q_start[b];
-    const int pos = a.kv_start[b] + i;
-    const int limit = a.kv_limit[b];
-    const bool causal = a.causal ? a.causal[b] != 0 : a.causal_default != 0;
-    n_keys = min(causal ? min(limit, pos + 1) : limit, a.bt_width * kPage);
-    table = a.block_table + (long)b * a.bt_stride;
-    if (a.kv_excluded != nullptr) {
-      ex_lo = a.kv_excluded[2 * b];
-      ex_hi = a.kv_excluded[2 * b + 1];
+  for (int c = 0; c < 8; c += 2)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s0 = mfma16x16x4(kx[c][e], q[c][e], s0);
+      s1 = mfma16x16x4(kx[c + 1][e], q[c + 1][e], s1);
     }
+  return s0 + s1;
+}
+
+// Online softmax of n 16-key score tiles of a wave's columns (hidden scores are -inf), in place: t becomes exp(t - m).
+template <int N>
+__device__ __forceinline__ void f32_softmax(floatx4 (&t)[N], float& m, float& l, floatx4 (&o)[8]) {
+  float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, t[i][r]);
+  if (__any(m == -INFINITY ? mx > -INFINITY : mx > m + kF32Headroom)) {
+    const float m_new = fmaxf(m, max_xor32(max_xor16(mx)));
+    const float alpha = m == -INFINITY ? 0.f : expf(m - m_new);
+    m = m_new;
+    l *= alpha;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] *= alpha;
+  }
+  float sum = 0.f;                                           // summed before it meets l: short chains round less
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[i][r] = t[i][r] == -INFINITY ? 0.f : expf(t[i][r] - m);
+    sum += (t[i][0] + t[i][1]) + (t[i][2] + t[i][3]);
+  }
+  l += sum;
+}
+
+// O^T += V^T . P^T over 16 keys: step r contracts the keys 4g + r, which is the order the scores lie in; o[t][r] is the
+// dim 64 * (t / 4) + 16g + 4r + t % 4 of column m16. va[r], vb[r]: V row 4g + r, dims 4 * m16 .. + 3 and 64 + those.
+__device__ __forceinline__ void f32_pv(const floatx4 (&va)[4], const floatx4 (&vb)[4], const floatx4& p,
+                                       floatx4 (&o)[8]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] = mfma16x16x4(va[r][e], p[r], o[e]);
+      o[4 + e] = mfma16x16x4(vb[r][e], p[r], o[4 + e]);
+    }
+}
+
+// Keys a lane's column sees in a stage: key < lim, or lo <= key < lo + len.
+struct F32Span {
+  int lim, lo;
+  unsigned len;
+};
+struct F32Stage {
+  int k0, end;             // keys [k0, min(k0 + 32, end)); rows at or past end are replaced by row end - 1 (weight 0)
+  F32Span span;
+};
+
+// Stages of the compression mask: SegWalk's 64-key tiles, each in up to two stages.
+struct MaskedStages {
+  const float* k;
+  const float* v;
+  long k_ss, v_ss;
+  SegWalk walk;
+  MaskShape g;
+  RowFacts row;
+  int plen, quota, u;      // u: which of the walk's two head limits is this wave's
+  int k0 = 0, left = 0;    // the tile's next stage, keys left in it
+  F32Span span;
+  __device__ __forceinline__ bool next(F32Stage& st) {
+    if (left <= 0) {
+      TileMask tm;
+      if (!walk.next(k0, tm, false)) return false;
+      left = min(kBN, walk.end - k0);
+      span = F32Span{tm.mode == 0 ? kNoKey : tm.mode == 1 ? row.q + 1 : u ? tm.limit[1] : tm.limit[0], 0, 0u};
+      if (tm.mode == 3) {
+        int lo = kNoKey;
+        lane_span(g, row, tm.seg, tm.kb, tm.limit[0], tm.limit[1], plen, quota, span.lim, lo);
+        span.lo = lo;
+        span.len = (unsigned)imax(tm.limit[1] - lo, 0);
+      }
+    }
+    st = F32Stage{k0, min(k0 + kF32Keys, k0 + left), span};
+    k0 += kF32Keys;
+    left -= kF32Keys;
+    return true;
+  }
+  // K and V rows of half h (rows 16h .. 16h + 15) of a stage
+  struct Half {
+    const float* k;
+    const float* v;
+    long k_ss, v_ss;
+  };
+  __device__ __forceinline__ Half half(const F32Stage& st, int) const {
+    return Half{k + (long)st.k0 * k_ss, v + (long)st.k0 * v_ss, k_ss, v_ss};
+  }
+  __device__ __forceinline__ static int row_of(const F32Stage& st, int row) { return min(row, st.end - 1 - st.k0); }
+};
+
+// Stages of one request's paged keys [0, n_keys) (the largest limit of the rows), with an excluded range.
+struct PagedStages {
+  const float* kv;         // cache base + head * 128
+  const int32_t* table;
+  int num_pages, n_keys, k0;
+  F32Span span;
+  __device__ __forceinline__ bool next(F32Stage& st) {
+    if (k0 >= n_keys) return false;
+    st = F32Stage{k0, min(k0 + kF32Keys, n_keys), span};
+    k0 += kF32Keys;
+    return true;
+  }
+  struct Half {
+    const float* k;
+    const float* v;
+    static constexpr long k_ss = kSlotElems, v_ss = kSlotElems;
+  };
+  __device__ __forceinline__ Half half(const F32Stage& st, int h) const {
+    const __attribute__((address_space(4))) int32_t* t = (const __attribute__((address_space(4))) int32_t*)table;
+    const int page = min(max(t[min(st.k0 / kPage + h, (st.end - 1) / kPage)], 0), num_pages - 1);
+    const float* p = kv + (long)page * kPageElems;
+    return Half{p, p + kHalfElems};
+  }
+  __device__ __forceinline__ static int row_of(const F32Stage& st, int row) {
+    return min(st.k0 + row, st.end - 1) & (kPage - 1);
+  }
+};
+
+// One wave's head over the stages: 16 query rows against K and V stages that the four waves of the workgroup load
+// together. The next stage's rows are on their way (in registers) while this one is multiplied. Row r's 16-byte chunk
+// c lies at chunk c ^ (r & 15), so both read patterns hit all banks.
+template <class Stages>
+__device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx4 (&q)[8], float scale, float& m,
+                                           float& l, floatx4 (&o)[8]) {
+  const int tid = threadIdx.x, lane = tid & 63, m16 = lane & 15, g = lane >> 4;
+  const int r0 = tid >> 5, chunk = tid & 31;
+  floatx4 kr[4], vr[4];
+  auto load = [&](const F32Stage& st) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const auto base = src.half(st, h);
+#pragma unroll
+      for (int i = 2 * h; i < 2 * h + 2; ++i) {
+        const int row = Stages::row_of(st, 8 * i + r0);
+        kr[i] = ldf4(base.k + row * base.k_ss + 4 * chunk);
+        vr[i] = ldf4(base.v + row * base.v_ss + 4 * chunk);
+      }
+    }
+  };
+  auto store = [&](int n) {                                  // buffer n: K rows, then V rows
+    float* kb = lds + 2 * n * kF32StageElems;
+    float* vb = kb + kF32StageElems;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 8 * i + r0, at = row * kHeadDim + 4 * (chunk ^ (row & 15));
+      *reinterpret_cast<floatx4*>(kb + at) = kr[i];
+      *reinterpret_cast<floatx4*>(vb + at) = vr[i];
+    }
+  };
+  F32Stage cur, nxt;
+  if (!src.next(cur)) return;
+  load(cur);
+  store(0);
+  __syncthreads();
+  for (int n = 0;; n ^= 1) {
+    const bool more = src.next(nxt);
+    if (more) load(nxt);
+    const float* kb = lds + 2 * n * kF32StageElems;
+    const float* vb = kb + kF32StageElems;
+    floatx4 t[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      floatx4 kx[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        kx[c] = *reinterpret_cast<const floatx4*>(kb + (16 * i + m16) * kHeadDim + 4 * ((4 * c + g) ^ m16));
+      t[i] = f32_scores(kx, q);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = cur.k0 + 16 * i + 4 * g + r;
+        const bool vis = key < cur.end && (key < cur.span.lim || (unsigned)(key - cur.span.lo) < cur.span.len);
+        t[i][r] = vis ? t[i][r] * scale : -INFINITY;
+      }
+    }
+    f32_softmax(t, m, l, o);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      floatx4 va[4], vb4[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * g + r;
+        const float* p = vb + (16 * i + row) * kHeadDim;
+        va[r] = *reinterpret_cast<const floatx4*>(p + 4 * (m16 ^ row));
+        vb4[r] = *reinterpret_cast<const floatx4*>(p + 4 * ((16 + m16) ^ row));
+      }
+      f32_pv(va, vb4, t[i], o);
+    }
+    if (!more) break;
+    store(n ^ 1);                            // read last before the barrier that closed the previous stage
+    __syncthreads();
+    cur = nxt;
+  }
+  l = sum_xor32(sum_xor16(l));
+}
+
+__device__ __forceinline__ void f32_load_q(const float* row, int g, bool ok, floatx4 (&q)[8]) {
+#pragma unroll
+  for (int c = 0; c < 8; ++c) q[c] = ok ? ldf4(row + 16 * c + 4 * g) : floatx4{0.f, 0.f, 0.f, 0.f};
+}
+
+__device__ __forceinline__ void f32_store(float* row, int g, float l, const floatx4 (&o)[8]) {
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      stf4(row + 64 * h + 16 * g + 4 * r, floatx4{o[4 * h][r], o[4 * h + 1][r], o[4 * h + 2][r], o[4 * h + 3][r]} * inv);
+}
+
+// The sum in 64 bits: m lies up to the headroom below the largest score, so log(l) alone would round more coarsely.
+__device__ __forceinline__ float f32_lse(float m, float l) {
+  return l > 0.f ? (float)((double)m + log((double)l)) : -INFINITY;
+}
+
+// Multi-query attention, masked (kMasked) or paged: a workgroup of 4 waves takes 16 query rows of one KV head, one query
+// head per wave. Bound by the fp32 matrix rate (16x16x4: 256 flop per clock and CU). Matrix instructions, LDS stages
+// shared by the four heads and the segment walk instead of VALU dot products per key with the mask's predicate per
+// element: masked, B=1, 3 x (512 + 128) rows 1546 -> 228 us; a code step of 256 rows over 4000 keys 2059 -> 455 us.
+template <bool kMasked>
+__global__ __launch_bounds__(256, 2) void attn_f32_rows_kernel(F32Args a) {
+  __shared__ __attribute__((aligned(16))) float lds[4 * kF32StageElems];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+  const int kvh = blockIdx.x % kHeadsKV;
+  const int head = kvh * kGroup + w;
+  floatx4 q[8], o[8];
+  float m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (kMasked) {
+    const int rank = blockIdx.x / kHeadsKV;                  // later (costlier) rows first, every sequence of a rank
+    const int b = rank % a.batch;
+    const int q0 = ((a.seq_len + kF32Rows - 1) / kF32Rows - 1 - rank / a.batch) * kF32Rows;
+    const int qrow = q0 + m16;
+    const int plen = a.prompt_len ? a.prompt_len[b] : 0;
+    int qmin = kNoKey, qmax = 0, quota = 0;
+#pragma unroll
+    for (int u = 0; u < kGroup; ++u) {
+      const int x = a.head_quota ? a.head_quota[kvh * kGroup + u] : a.codes_k;
+      qmin = min(qmin, x);
+      qmax = max(qmax, x);
+      if (u == w) quota = x;
+    }
+    const MaskShape g_ = {a.seq_len, a.block_c, a.codes_k, a.pause_passes, a.replay_rows, a.copy_rows,
+                          a.block_c + a.pause_passes * a.codes_k + a.replay_rows, a.num_blocks, a.retain_tail,
+                          a.tail_policy, a.pause_xattn, a.replay_exclude != 0};
+    f32_load_q(a.q + (long)b * a.q_sb + (long)min(qrow, a.seq_len - 1) * a.q_st + (long)head * a.q_sh, g,
+               qrow < a.seq_len, q);
+    MaskedStages src{a.k + (long)b * a.k_sb + (long)kvh * a.k_sh, a.v + (long)b * a.v_sb + (long)kvh * a.v_sh,
+                     a.k_ss, a.v_ss,
+                     SegWalk(g_, q0, min(q0 + kF32Rows, a.seq_len) - 1, plen, qmin, qmax, quota, quota), g_,
+                     row_facts(g_, qrow), plen, quota, 0};
+    f32_attend(src, lds, q, a.scale, m, l, o);
+    if (qrow >= a.seq_len) return;
+    f32_store(a.out + (long)b * a.o_sb + (long)qrow * a.o_st + (long)head * a.o_sh, g, l, o);
+    if (a.lse != nullptr && g == 0) a.lse[((long)b * kHeadsQ + head) * a.seq_len + qrow] = f32_lse(m, l);
   } else {
-    b = t;
-    n_keys = max(min(a.seq_lens[b], a.max_pages * kPage), 0);
-    table = a.block_table + (long)b * a.bt_stride;
-  }
-  lim_lane = n_keys;
-
-  // Query heads of this KV head into LDS.
-  const float* qbase = a.mode == 1 ? a.q + (long)b * a.q_sb + (long)qrow * a.q_st : a.q + (long)t * a.q_st;
-  for (int i = lane; i < kGroup * kHeadDim; i += 64)
-    q_lds[w][i / kHeadDim][i % kHeadDim] = qbase[(long)(kvh * kGroup + i / kHeadDim) * a.q_sh + (i % kHeadDim)];
-  wave_sync();
-
-  float m[kGroup], l[kGroup], o[kGroup][2];
-#pragma unroll
-  for (int u = 0; u < kGroup; ++u) {
-    m[u] = -INFINITY;
-    l[u] = 0.f;
-    o[u][0] = o[u][1] = 0.f;
-  }
-
-  for (int j0 = 0; j0 < n_keys; j0 += 64) {
-    const int j = j0 + lane;
-    float s[kGroup];
-    bool vis[kGroup];
-#pragma unroll
-    for (int u = 0; u < kGroup; ++u) {
-      vis[u] = j < lim_lane && (j < ex_lo || j >= ex_hi) && (a.mode != 1 || f32_visible(a, qrow, j, plen, quota[u]));
-      s[u] = -INFINITY;
-    }
-    if (vis[0] || vis[1] || vis[2] || vis[3]) {
-      const float* krow;
-      if (a.mode == 1) {
-        krow = a.k + (long)b * a.k_sb + (long)j * a.k_ss + (long)kvh * a.k_sh;
-      } else {
-        const int page = min(max(table[j / kPage], 0), a.num_pages - 1);
-        krow = a.kv + (long)page * kPageElems + (j % kPage) * kSlotElems + kvh * kHeadDim;
+    // the rows of 16 consecutive tokens, request by request (uniform over the workgroup)
+    const int t0 = blockIdx.x / kHeadsKV * kF32Rows, t_end = min(t0 + kF32Rows, a.num_tokens);
+    const int my_req = a.tok_req[min(t0 + m16, t_end - 1)];
+    for (int t = t0; t < t_end;) {
+      const int b = __builtin_amdgcn_readlane(my_req, t - t0);
+      // tokens of this request from t on (lanes 0 .. 15 hold the window's requests)
+      const unsigned differs = (unsigned)__ballot(my_req != b) & 0xffffu & (~0u << (t - t0));
+      const int t1 = min(differs ? t0 + __ffs(differs) - 1 : t_end, t_end);
+      const int n = t1 - t;
+      const int row = t + m16;                               // this lane's token (valid below t1)
+      const int pos = a.kv_start[b] + t - a.q_start[b];      // position of row t
+      const int limit = min(a.kv_limit[b], a.bt_width * kPage);
+      const bool causal = a.causal ? a.causal[b] != 0 : a.causal_default != 0;
+      const int lane_limit = row >= t1 ? 0 : causal ? min(limit, pos + m16 + 1) : limit;
+      F32Span span{lane_limit, 0, 0u};
+      if (a.kv_excluded != nullptr) {
+        const int lo = a.kv_excluded[2 * b], hi = a.kv_excluded[2 * b + 1];
+        if (lo < hi) span = F32Span{min(lane_limit, lo), hi, (unsigned)max(lane_limit - hi, 0)};
       }
-      float acc[kGroup] = {0.f, 0.f, 0.f, 0.f};
-      for (int d = 0; d < kHeadDim; d += 4) {
-        const floatx4 kx = *reinterpret_cast<const floatx4*>(krow + d);
-#pragma unroll
-        for (int u = 0; u < kGroup; ++u) {
-          acc[u] = fmaf(q_lds[w][u][d], kx[0], acc[u]);
-          acc[u] = fmaf(q_lds[w][u][d + 1], kx[1], acc[u]);
-          acc[u] = fmaf(q_lds[w][u][d + 2], kx[2], acc[u]);
-          acc[u] = fmaf(q_lds[w][u][d + 3], kx[3], acc[u]);
-        }
+      f32_load_q(a.q + (long)min(row, t1 - 1) * a.q_st + (long)head * a.q_sh, g, row < t1, q);
+      PagedStages src{a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages,
+                      causal ? min(limit, pos + n) : limit, 0, span};
+      f32_attend(src, lds, q, a.scale, m, l, o);
+      if (row < t1) {
+        f32_store(a.out + (long)row * a.o_st + (long)head * a.o_sh, g, l, o);
+        if (a.lse != nullptr && g == 0) a.lse[(long)row * kHeadsQ + head] = f32_lse(m, l);
       }
+      t = t1;
+      m = -INFINITY;
+      l = 0.f;
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u)
-        if (vis[u]) s[u] = acc[u] * a.scale;
-    }
-    // online softmax per head over the tile
-#pragma unroll
-    for (int u = 0; u < kGroup; ++u) {
-      float tmax = s[u];
-      for (int off = 32; off > 0; off >>= 1) tmax = fmaxf(tmax, __shfl_xor(tmax, off, 64));
-      const float m_new = fmaxf(m[u], tmax);
-      const float alpha = m[u] == -INFINITY ? 0.f : expf(m[u] - m_new);
-      const float p = vis[u] ? expf(s[u] - m_new) : 0.f;
-      float psum = p;
-      for (int off = 32; off > 0; off >>= 1) psum += __shfl_xor(psum, off, 64);
-      l[u] = l[u] * alpha + psum;
-      o[u][0] *= alpha;
-      o[u][1] *= alpha;
-      m[u] = m_new;
-      p_lds[w][u][lane] = p;
-    }
-    wave_sync();
-    const int n_tile = min(64, n_keys - j0);
-    for (int jj = 0; jj < n_tile; ++jj) {
-      const int jk = j0 + jj;
-      const float* vrow;
-      if (a.mode == 1) {
-        vrow = a.v + (long)b * a.v_sb + (long)jk * a.v_ss + (long)kvh * a.v_sh;
-      } else {
-        const int page = min(max(table[jk / kPage], 0), a.num_pages - 1);
-        vrow = a.kv + (long)page * kPageElems + kHalfElems + (jk % kPage) * kSlotElems + kvh * kHeadDim;
-      }
-      const float2 vx = *reinterpret_cast<const float2*>(vrow + 2 * lane);
-#pragma unroll
-      for (int u = 0; u < kGroup; ++u) {
-        const float p = p_lds[w][u][jj];
-        o[u][0] = fmaf(p, vx.x, o[u][0]);
-        o[u][1] = fmaf(p, vx.y, o[u][1]);
-      }
-    }
-    wave_sync();
-  }
-
-#pragma unroll
-  for (int u = 0; u < kGroup; ++u) {
-    const int head = kvh * kGroup + u;
-    const float inv = l[u] > 0.f ? 1.f / l[u] : 0.f;
-    float* orow = a.mode == 1 ? a.out + (long)b * a.o_sb + (long)qrow * a.o_st + (long)head * a.o_sh
-                              : a.out + (long)t * a.o_st + (long)head * a.o_sh;
-    *reinterpret_cast<float2*>(orow + 2 * lane) = make_float2(o[u][0] * inv, o[u][1] * inv);
-    if (a.lse != nullptr && lane == 0) {
-      const float v = l[u] > 0.f ? m[u] + logf(l[u]) : -INFINITY;
-      if (a.mode == 1)
-        a.lse[((long)b * kHeadsQ + head) * a.seq_len + qrow] = v;
-      else
-        a.lse[(long)t * kHeadsQ + head] = v;
+      for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      __syncthreads();                                       // the next request's first stage overwrites this one's
     }
   }
 }
 
-static int launch_f32(const F32Args& a, hipStream_t stream) {
-  if (a.num_tokens <= 0) return 0;
-  dim3 grid((a.num_tokens + kF32Waves - 1) / kF32Waves, kHeadsKV);
-  hipLaunchKernelGGL(attn_f32_kernel, grid, dim3(64 * kF32Waves), 0, stream, a);
-  return (int)hipGetLastError();
+// Decode: a workgroup of 8 waves per (sequence, KV head); wave w takes pages w, w + 8, ... straight into operand
+// registers (the next page's K loads while this page is multiplied) and the eight partial results meet in LDS. The four
+// heads fill the 16 columns four times over: the path is bound by memory, not by the matrix rate. 32 sequences of
+// 900 .. 9500 rows 7014 -> 286 us (4.8 TB/s), one of 5000 rows 2102 -> 108 us, against the VALU form of one wave each.
+constexpr int kDecWaves = 8;
+__global__ __launch_bounds__(64 * kDecWaves, 2) void decode_f32_kernel(F32Args a) {
+  __shared__ __attribute__((aligned(16))) float po[kDecWaves][kGroup][kHeadDim];
+  __shared__ float pm[kDecWaves][kGroup], pl[kDecWaves][kGroup];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+  const int kvh = blockIdx.x % kHeadsKV, b = blockIdx.x / kHeadsKV;
+  const int n_keys = max(min(a.seq_lens[b], a.max_pages * kPage), 0);
+  const int n_pages = (n_keys + kPage - 1) / kPage;
+  const __attribute__((address_space(4))) int32_t* table =
+      (const __attribute__((address_space(4))) int32_t*)(a.block_table + (long)b * a.bt_stride);
+  floatx4 q[8], o[8], kx[8];
+  f32_load_q(a.q + (long)b * a.q_st + (long)(kvh * kGroup + (m16 & 3)) * a.q_sh, g, true, q);
+  float m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto page_of = [&](int p) {
+    return a.kv + (long)min(max(table[p], 0), a.num_pages - 1) * kPageElems + kvh * kHeadDim;
+  };
+  auto load_k = [&](const float* page, int p) {              // rows past the end: the last row (weight 0)
+    const float* r = page + min(m16, n_keys - 1 - p * kPage) * kSlotElems + 4 * g;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) kx[c] = ldf4(r + 16 * c);
+  };
+  if (w < n_pages) {
+    const float* page = page_of(w);
+    load_k(page, w);
+    for (int p = w; p < n_pages; p += kDecWaves) {
+      floatx4 va[4], vb[4], t[1];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float* vr = page + kHalfElems + min(4 * g + r, n_keys - 1 - p * kPage) * kSlotElems + 4 * m16;
+        va[r] = ldf4(vr);
+        vb[r] = ldf4(vr + 64);
+      }
+      t[0] = f32_scores(kx, q);
+      if (p + kDecWaves < n_pages) {
+        page = page_of(p + kDecWaves);
+        load_k(page, p + kDecWaves);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t[0][r] = p * kPage + 4 * g + r < n_keys ? t[0][r] * a.scale : -INFINITY;
+      f32_softmax(t, m, l, o);
+      f32_pv(va, vb, t[0], o);
+    }
+  }
+  l = sum_xor32(sum_xor16(l));
+  if (m16 < kGroup) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<floatx4*>(&po[w][m16][64 * h + 16 * g + 4 * r]) =
+            floatx4{o[4 * h][r], o[4 * h + 1][r], o[4 * h + 2][r], o[4 * h + 3][r]};
+    if (g == 0) {
+      pm[w][m16] = m;
+      pl[w][m16] = l;
+    }
+  }
+  __syncthreads();
+  const int u = threadIdx.x / kHeadDim, d = threadIdx.x % kHeadDim;   // 512 threads: 4 heads x 128 dims
+  float M = -INFINITY, L = 0.f, acc = 0.f;
+#pragma unroll
+  for (int i = 0; i < kDecWaves; ++i) M = fmaxf(M, pm[i][u]);
+#pragma unroll
+  for (int i = 0; i < kDecWaves; ++i) {
+    if (pl[i][u] == 0.f && pm[i][u] == -INFINITY) continue;           // a wave that had no page
+    const float f = expf(pm[i][u] - M);
+    L += pl[i][u] * f;
+    acc += po[i][u][d] * f;
+  }
+  const int head = kvh * kGroup + u;
+  a.out[(long)b * a.o_st + (long)head * a.o_sh + d] = L > 0.f ? acc * (1.f / L) : 0.f;
+  if (a.lse != nullptr && d == 0) a.lse[(long)b * kHeadsQ + head] = f32_lse(M, L);
+}
+
+// Workgroups of the row kernels: 8 KV heads x (16-row tiles); 0 when the work items would not fit the grid.
+static unsigned f32_grid(long tiles) {
+  const long n = tiles * kHeadsKV;
+  return n <= 0 || n * 256 > 0xFFFFFFFFL ? 0u : (unsigned)n;
 }
 
 static F32Args f32_defaults() {
@@ -246,7 +481,6 @@ int abkv_decode_attn_f32(const float* q, long q_stride_seq, long q_stride_head, 
       num_pages <= 0 || max_pages_per_seq <= 0 || block_table_stride < max_pages_per_seq)
     return (int)hipErrorInvalidValue;
   F32Args a = f32_defaults();
-  a.mode = 2;
   a.q = q;
   a.q_st = q_stride_seq;
   a.q_sh = q_stride_head;
@@ -262,7 +496,9 @@ int abkv_decode_attn_f32(const float* q, long q_stride_seq, long q_stride_head, 
   a.o_st = out_stride_seq;
   a.o_sh = out_stride_head;
   a.lse = lse;
-  return launch_f32(a, stream);
+  if ((long)num_seqs * kHeadsKV * 64 * kDecWaves > 0xFFFFFFFFL) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(decode_f32_kernel, dim3((unsigned)num_seqs * kHeadsKV), dim3(64 * kDecWaves), 0, stream, a);
+  return (int)hipGetLastError();
 }
 
 int abkv_paged_prefill_attn_f32(const float* q, long q_stride_t, long q_stride_h, const float* kv_cache, int num_pages,
@@ -277,7 +513,6 @@ int abkv_paged_prefill_attn_f32(const float* q, long q_stride_t, long q_stride_h
       kv_limit == nullptr || tok_req == nullptr || out == nullptr || num_pages <= 0 || block_table_width <= 0)
     return (int)hipErrorInvalidValue;
   F32Args a = f32_defaults();
-  a.mode = 0;
   a.q = q;
   a.q_st = q_stride_t;
   a.q_sh = q_stride_h;
@@ -299,7 +534,10 @@ int abkv_paged_prefill_attn_f32(const float* q, long q_stride_t, long q_stride_h
   a.o_st = out_stride_t;
   a.o_sh = out_stride_h;
   a.lse = lse;
-  return launch_f32(a, stream);
+  const unsigned grid = f32_grid(((long)num_tokens + kF32Rows - 1) / kF32Rows);
+  if (grid == 0) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(attn_f32_rows_kernel<false>, dim3(grid), dim3(256), 0, stream, a);
+  return (int)hipGetLastError();
 }
 
 int abkv_prefill_masked_attn_f32(const float* q, long q_sb, long q_ss, long q_sh, const float* k, long k_sb,
@@ -322,7 +560,6 @@ int abkv_prefill_masked_attn_f32(const float* q, long q_sb, long q_ss, long q_sh
       pause_xattn > kXattnNone)
     return (int)hipErrorInvalidValue;
   F32Args a = f32_defaults();
-  a.mode = 1;
   a.q = q;
   a.q_sb = q_sb;
   a.q_st = q_ss;
@@ -347,14 +584,18 @@ int abkv_prefill_masked_attn_f32(const float* q, long q_sb, long q_ss, long q_sh
   a.copy_rows = copy_rows;
   a.replay_rows = replay_rows;
   a.replay_exclude = replay_exclude;
-  a.num_tokens = batch * seq_len;
+  a.batch = batch;
+  a.num_blocks = num_blocks;
   a.scale = scale;
   a.out = out;
   a.o_sb = o_sb;
   a.o_st = o_ss;
   a.o_sh = o_sh;
   a.lse = lse;
-  return launch_f32(a, stream);
+  const unsigned grid = f32_grid(((long)seq_len + kF32Rows - 1) / kF32Rows * batch);
+  if (grid == 0) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(attn_f32_rows_kernel<true>, dim3(grid), dim3(256), 0, stream, a);
+  return (int)hipGetLastError();
 }
 
 }  // extern "C"

@@ -122,3 +122,53 @@ def test_masked_prefill_f32_matches_fp64(prompt_len, quota, tail, policy):
         ro, rl = op.masked_attention_fp64(q[b].numpy(), k[b].numpy(), v[b].numpy(), mask, 128 ** -0.5)
         assert np.abs(got_o[b] - ro).max() <= TOL
         assert np.abs(got_l[b].T - rl).max() <= TOL
+
+
+def test_decode_f32_page_and_wave_edges():
+    """Row counts around one page, the eight pages that the workgroup's waves start with, and their second turn.
+    Tolerance: fp32 sums of 128 products and up to 300 weights, under 1e-5 with |out| <= 5."""
+    from abridgekv_amd import ops
+    lens = [1, 15, 16, 17, 127, 128, 129, 144, 256, 257, 300]
+    cache, tables = _paged(lens, 200, 20)
+    g = torch.Generator().manual_seed(21)
+    q = 2.5 * torch.randn((len(lens), 32, 128), generator=g, dtype=torch.float32)
+    dev = torch.device("cuda")
+    lse = torch.empty((len(lens), 32), dtype=torch.float32, device=dev)
+    out, _ = ops.decode_attention(q.to(dev), cache.to(dev), torch.from_numpy(tables).to(dev),
+                                  torch.tensor(lens, dtype=torch.int32, device=dev), 128 ** -0.5, lse=lse)
+    ref_o, ref_l = od.decode_paged_fp64(q.numpy(), cache.numpy(), tables, lens, 128 ** -0.5)
+    assert np.abs(out.cpu().numpy() - ref_o).max() <= TOL
+    assert np.abs(lse.cpu().numpy() - ref_l).max() <= TOL
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_paged_f32_tiles_with_rows_of_several_requests(causal):
+    """16-row tiles that hold rows of one to six requests, key ranges around the 32-key stages, a request without
+    keys. Tolerance as above."""
+    from abridgekv_amd import ops
+    qlen = [1, 5, 16, 3, 33, 1, 1, 2, 15]
+    past = [31, 27, 16, 0, 64, 32, 300, 30, 1]
+    sls = [a + b for a, b in zip(qlen, past)]
+    limits = [sl if causal else max(0, sl - 1) for sl in sls]
+    cache, tables = _paged(sls, 120, 22)
+    qsl = np.concatenate([[0], np.cumsum(qlen)])
+    if not causal:
+        limits[6] = 0
+    g = torch.Generator().manual_seed(23)
+    q = torch.randn((int(qsl[-1]), 32, 128), generator=g, dtype=torch.float32)
+    dev = torch.device("cuda")
+    lse = torch.empty((int(qsl[-1]), 32), dtype=torch.float32, device=dev)
+    out, _ = ops.paged_prefill_attention(q.to(dev), cache.to(dev), torch.from_numpy(tables).to(dev), qsl, past,
+                                         limits, causal, lse=lse)
+    got_o, got_l = out.cpu().numpy(), lse.cpu().numpy()
+    for r, sl in enumerate(sls):
+        a, z = qsl[r], qsl[r + 1]
+        if limits[r] == 0:
+            assert np.all(got_o[a:z] == 0) and np.all(np.isneginf(got_l[a:z]))
+            continue
+        k, v = od.paged_rows(cache.numpy(), tables[r], limits[r])
+        for i in range(qlen[r]):
+            n = min(limits[r], past[r] + i + 1) if causal else limits[r]
+            ro, rl = od.decode_fp64(q[a + i].numpy(), k[:n], v[:n], 128 ** -0.5)
+            assert np.abs(got_o[a + i] - ro).max() <= TOL, f"request {r} row {i}"
+            assert np.abs(got_l[a + i] - rl).max() <= TOL, f"request {r} row {i}"
