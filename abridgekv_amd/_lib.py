@@ -24,6 +24,7 @@ SIGNATURES = {
                                         _vp, _vp, C.c_int, _vp]),
     "abkv_kv_move_mixed": (C.c_int, [C.POINTER(_vp), C.c_int, C.c_int, C.c_int, C.c_long, C.c_long, C.c_int,
                                      _vp, _vp, C.c_int, _vp, C.c_int, _vp]),
+    "abkv_kv_move_groups": (C.c_int, [_vp, C.c_int, C.c_int, C.c_long, C.c_long, C.c_int, _vp]),
     "abkv_kv_stage_bytes": (C.c_size_t, [C.c_int, C.c_int, C.c_int]),
     "abkv_kv_copy_staged": (C.c_int, [C.POINTER(_vp), C.c_int, C.c_int, C.c_int, C.c_long, C.c_long, C.c_int, _vp,
                                       C.c_int, _vp, C.c_size_t, _vp]),

@@ -241,24 +241,46 @@ def kv_move_segments(layer_caches, ops: torch.Tensor, seg_offsets: torch.Tensor)
     check(rc, "abkv_kv_move_segments")
 
 
+class _MoveGroup(C.Structure):
+    """abkv_move_group."""
+    _fields_ = [("layer_caches", C.POINTER(C.c_void_p)), ("n_layers", C.c_int), ("num_pages", C.c_int),
+                ("ops", C.c_void_p), ("seg_offsets", C.c_void_p), ("n_segments", C.c_int), ("free_ops", C.c_void_p),
+                ("n_free", C.c_int)]
+
+
+def kv_move_groups(groups) -> None:
+    """abkv_kv_move_groups: the moves of several KV-cache groups in one launch (per 8 groups). ``groups``: a list of
+    (layer caches, ops, seg_offsets, free_ops) as :func:`kv_move_mixed` takes them. Groups that share layer caches must
+    not touch each other's slots (a planner step's groups own disjoint pages)."""
+    table = (_MoveGroup * len(groups))()
+    n, arrays = 0, []
+    for layer_caches, ops, seg_offsets, free_ops in groups:
+        for name, t in (("ops", ops), ("free_ops", free_ops)):
+            _require(t.is_cuda and t.dtype == torch.int32 and t.dim() == 2 and t.shape[1] == 4 and t.is_contiguous(),
+                     f"{name} must be contiguous cuda int32 [n, 4]")
+        _require(seg_offsets.is_cuda and seg_offsets.dtype == torch.int32 and seg_offsets.is_contiguous()
+                 and seg_offsets.numel() >= 1, "seg_offsets must be contiguous cuda int32 with at least one entry")
+        n_seg = seg_offsets.numel() - 1 if ops.shape[0] else 0
+        n_free = free_ops.shape[0]
+        if n_seg == 0 and n_free == 0:
+            continue
+        arr, num_pages = _layer_ptrs(layer_caches)
+        arrays.append(arr)
+        table[n] = _MoveGroup(arr, len(layer_caches), num_pages, ops.data_ptr() if n_seg else None,
+                              seg_offsets.data_ptr() if n_seg else None, n_seg,
+                              free_ops.data_ptr() if n_free else None, n_free)
+        n += 1
+    if n == 0:
+        return
+    rc = lib().abkv_kv_move_groups(C.byref(table), n, PAGE, PAGE_BYTES, HALF_BYTES, SLOT_BYTES, C.c_void_p(_stream()))
+    check(rc, "abkv_kv_move_groups")
+
+
 def kv_move_mixed(layer_caches, ops: torch.Tensor, seg_offsets: torch.Tensor, free_ops: torch.Tensor) -> None:
     """abkv_kv_move_mixed, one launch: the ordered segments of :func:`kv_move_segments` (``ops`` [n, 4] with
     ``seg_offsets`` [n_seg + 1]; n_seg may be 0) and the independent ops ``free_ops`` [m, 4] -- ops that read or write
     no slot another op of the call writes (:func:`abridgekv_amd.worker.pack_fused_moves` builds both)."""
-    for name, t in (("ops", ops), ("free_ops", free_ops)):
-        _require(t.is_cuda and t.dtype == torch.int32 and t.dim() == 2 and t.shape[1] == 4 and t.is_contiguous(),
-                 f"{name} must be contiguous cuda int32 [n, 4]")
-    _require(seg_offsets.is_cuda and seg_offsets.dtype == torch.int32 and seg_offsets.is_contiguous()
-             and seg_offsets.numel() >= 1, "seg_offsets must be contiguous cuda int32 with at least one entry")
-    n_seg = seg_offsets.numel() - 1 if ops.shape[0] else 0
-    n_free = free_ops.shape[0]
-    if n_seg == 0 and n_free == 0:
-        return
-    arr, num_pages = _layer_ptrs(layer_caches)
-    rc = lib().abkv_kv_move_mixed(arr, len(layer_caches), num_pages, PAGE, PAGE_BYTES, HALF_BYTES, SLOT_BYTES,
-                                  _ptr(ops) if n_seg else None, _ptr(seg_offsets) if n_seg else None, n_seg,
-                                  _ptr(free_ops) if n_free else None, n_free, C.c_void_p(_stream()))
-    check(rc, "abkv_kv_move_mixed")
+    kv_move_groups([(layer_caches, ops, seg_offsets, free_ops)])
 
 
 def kv_copy_staged(layer_caches, ops: torch.Tensor, stage: torch.Tensor | None = None) -> None:

@@ -201,23 +201,32 @@ def device_move_lists(dev_buf: torch.Tensor, parts):
 
 
 def launch_moves(prepared, layer_caches_by_group, events=None) -> None:
-    """Device side of :func:`execute_fused_moves`: one launch per group (and per 16 layer tensors). ``events``, if
-    given, is a list that receives (start, end) CUDA events recorded around every launch."""
-    for gid, ops_d, offs_d, free_d in prepared:
-        caches = layer_caches_by_group[gid]
-        for lo in range(0, len(caches), 16):
-            if events is not None:
-                s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                s.record()
-            ops.kv_move_mixed(caches[lo: lo + 16], ops_d, offs_d, free_d)
-            if events is not None:
-                e.record()
-                events.append((s, e))
+    """Device side of :func:`execute_fused_moves`: the step's groups in one launch (per 8 groups; a group of more than
+    16 layer tensors counts once per 16). No op of a step touches a slot of another group: a page of the pool belongs
+    to one request and group. ``events``, if given, is a list that receives the (start, end) CUDA events recorded
+    around the launch."""
+    start = 0
+    while start < len(prepared):
+        gids, groups = set(), []
+        for gid, ops_d, offs_d, free_d in prepared[start:]:
+            if gid in gids:                                    # a group's second list may build on its first
+                break
+            gids.add(gid)
+            caches = layer_caches_by_group[gid]
+            groups += [(caches[lo: lo + 16], ops_d, offs_d, free_d) for lo in range(0, len(caches), 16)]
+        start += len(gids)
+        if events is not None:
+            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            s.record()
+        ops.kv_move_groups(groups)
+        if events is not None:
+            e.record()
+            events.append((s, e))
 
 
 def execute_fused_moves(fused_moves: np.ndarray, layer_caches_by_group, check: bool = True) -> None:
-    """Apply a planner step's fused move rows (request, group, src_block, src_off, dst_block, dst_off): one launch
-    per group. Rows of one (request, group) are monotone (increasing source, dst < src): a run whose ops depend on
+    """Apply a planner step's fused move rows (request, group, src_block, src_off, dst_block, dst_off) in one
+    launch. Rows of one (request, group) are monotone (increasing source, dst < src): a run whose ops depend on
     each other's order is walked in order by the in-register chunked copy, every other op moves independently."""
     if fused_moves.size == 0:
         return

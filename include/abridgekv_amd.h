@@ -87,6 +87,22 @@ int abkv_kv_move_segments(void* const* layer_caches, int n_layers, int num_pages
 int abkv_kv_move_mixed(void* const* layer_caches, int n_layers, int num_pages, int block_size, long page_bytes,
                        long half_bytes, int slot_bytes, const int32_t* ops, const int32_t* seg_offsets, int n_segments,
                        const int32_t* free_ops, int n_free, abkv_stream_t stream);
+/* abkv_kv_move_groups: abkv_kv_move_mixed over several KV-cache groups in one launch (up to 8; more take more
+ * launches): group i's ops apply to its n_layers (<= 16) layer caches of num_pages pages. Groups may share layer
+ * caches when no op of one group reads or writes a slot that another group writes (a planner step's groups own
+ * disjoint pages). Groups without ops are skipped. */
+typedef struct abkv_move_group {
+  void* const* layer_caches;
+  int n_layers;
+  int num_pages;
+  const int32_t* ops;
+  const int32_t* seg_offsets;
+  int n_segments;
+  const int32_t* free_ops;
+  int n_free;
+} abkv_move_group;
+int abkv_kv_move_groups(const abkv_move_group* groups, int n_groups, int block_size, long page_bytes, long half_bytes,
+                        int slot_bytes, abkv_stream_t stream);
 size_t abkv_kv_stage_bytes(int n_layers, int n_ops, int slot_bytes);
 int abkv_kv_copy_staged(void* const* layer_caches, int n_layers, int num_pages, int block_size, long page_bytes,
                         long half_bytes, int slot_bytes, const int32_t* ops, int n_ops, void* stage, size_t stage_bytes, abkv_stream_t stream);

@@ -187,3 +187,37 @@ def _segments(fused):
     cut = np.flatnonzero(np.any(np.diff(fused[:, :2], axis=0) != 0, axis=1)) + 1
     for rows in np.split(fused, cut):
         yield (int(rows[0, 0]), int(rows[0, 1])), rows
+
+
+@pytest.mark.parametrize("n_groups", [1, 8, 9, 17])
+def test_move_groups_of_one_launch_and_of_several(n_groups):
+    """Groups over shared layer tensors, up to and past the eight groups of one launch: ordered segments (a shift by
+    three rows over several 64-row chunks), independent ops with a remainder of four, groups without one kind or
+    without any, 1 .. 3 layers. Whole rows, bit for bit."""
+    rng = np.random.default_rng(n_groups)
+    dev = torch.device("cuda")
+    pages = 24
+    P = pages * n_groups
+    caches = [torch.randint(-2 ** 15, 2 ** 15, ops.kv_cache_shape(P), dtype=torch.int16,
+                            generator=torch.Generator().manual_seed(10 * n_groups + i)) for i in range(3)]
+    want = [c.clone() for c in caches]
+    on_gpu = [c.view(torch.bfloat16).to(dev) for c in caches]
+    groups = []
+    for g in range(n_groups):
+        ids = rng.permutation(np.arange(g * pages, (g + 1) * pages))
+        slot = lambda i: (int(ids[i // 16]), i % 16)           # row i of the group
+        n_ord = [0, 1, 64, 65, 150][g % 5]
+        n_free = [0, 1, 4, 7, 90, 0][g % 6]
+        ordered = [(*slot(i + 3), *slot(i)) for i in range(n_ord)]
+        free = [(*slot(290 + i), *slot(180 + i)) for i in range(n_free)]
+        n_layers = 1 + g % 3
+        for w in want[:n_layers]:
+            src = [w[a, :, b].clone() for a, b, _, _ in ordered + free]
+            for row, (_, _, c, d) in zip(src, ordered + free):
+                w[c, :, d] = row
+        t = lambda x: torch.tensor(x, dtype=torch.int32).reshape(-1, 4).to(dev)
+        groups.append((on_gpu[:n_layers], t(ordered), torch.tensor([0, n_ord] if n_ord else [0],
+                                                                     dtype=torch.int32).to(dev), t(free)))
+    ops.kv_move_groups(groups)
+    for got, w in zip(on_gpu, want):
+        assert torch.equal(got.cpu().view(torch.int16), w)
