@@ -17,7 +17,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 DEVICE_SOURCES = ["decode_attn.hip", "kv_cache.hip", "prefill_attn.hip", "prefill_bwd.hip", "paged_prefill.hip",
                   "attn_f32.hip"]
-HOST_SOURCES = ["planner.cpp"]
+HOST_SOURCES = ["planner.cpp", "paged_plan.cpp"]
 PROBE_SOURCES = ["probes.hip"]
 
 # -packed-fp32-ops off: hipcc would otherwise emit v_pk_{add,mul,fma}_f32 from scalar float code.

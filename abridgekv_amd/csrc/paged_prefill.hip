@@ -8,7 +8,8 @@
 //   query row i of request r sits at physical position kv_start[r] + i and sees keys k < kv_limit[r]
 //   (and k <= its own position when request r is causal; a batch may mix causal chunks and code steps).
 // Prompt chunks are the causal case with kv_limit = seq_len. Same tile machinery as the masked-prefill kernel
-// (attn_tile.h): 8 waves x (16 rows x 2 heads), 64-key tiles DMA'd from the page table into double-buffered LDS.
+// (attn_tile.h): 8 waves x (16 rows x 2 heads), 64-key tiles DMA'd from the page table into double-buffered LDS. A mixed
+// batch runs the work items of a host plan (paged_plan.cpp), in which only long key ranges are split.
 #include "attn_tile.h"
 
 namespace abkv {
@@ -28,11 +29,14 @@ struct PagedPrefillArgs {
   float scale_log2;
   __bf16* out; long o_st, o_sh;                // [T, 32, 128]
   float* lse;                                  // [T, 32] natural log, or nullptr
-  int num_tiles;                               // query tiles; the grid is 8 x num_tiles x splits (linear_block)
-  int split_tiles;                             // > 0: key tiles per split, partials to part_*
+  const int32_t* items;                        // [n][5] work items (abkv_paged_plan), or nullptr: uniform splits
+  const int32_t* merges;                       // [m][4] query tiles whose items' partials are merged
+  int num_tiles;                               // uniform: query tiles; the grid is 8 x num_tiles x splits
+  int split_tiles;                             // uniform: > 0: key tiles per split, partials to part_*
   int num_tokens;
-  _Float16* part_o;                            // [splits, T, 32, 128] split output / (l * scale), fp16
-  float* part_ml;                              // [splits, T, 32, 4] (max in log2 units, weight sum l, scale, unused)
+  _Float16* part_o;                            // [rows, 32, 128] split output / (l * scale), fp16
+  float* part_ml;                              // [rows, 32, 4] (max in log2 units, weight sum l, scale, unused);
+                                               // uniform: rows = splits x T
   int split_base;                              // first partial slot of this launch's splits
   const int32_t* head_quota;                   // [8] or nullptr: a non-causal request sees keys < kv_start + q_h
   // side rows (per-head packed code pages, attended by every query of the request); see PackedRows
@@ -107,14 +111,30 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
   __shared__ __attribute__((aligned(16))) __bf16 V0[kTileElems], V1[kTileElems], V2[kTileElems];
   __bf16* const Kbuf[kStages] = {K0, K1, K2};
   __bf16* const Vbuf[kStages] = {V0, V1, V2};
-  // linear grid, KV head fastest, then query tile, then key split: workgroups go to the 8 XCDs round-robin by
-  // linear id, so the query tiles of one request that read the same K/V tiles (same head, same split) share an L2
+  // linear grid, KV head fastest, then the work item (uniform: query tile, then key split): workgroups go to the 8 XCDs
+  // round-robin by linear id, so the query tiles of one request that read the same K/V tiles (same head) share an L2
   const int l = blockIdx.x;
   const int kvh = l % kHeadsKV;
-  const int tile = (l / kHeadsKV) % a.num_tiles;
-  const int split = l / (kHeadsKV * a.num_tiles);
-  const int r = a.tile_req[tile];
-  const int q0 = a.tile_q0[tile];
+  int r, q0, kt_begin = 0, kt_end = kNoKey;
+  long part_row = -1;                                       // partial row of query row q0; < 0: final output
+  if (a.items != nullptr) {
+    const int32_t* it = a.items + 5 * (l / kHeadsKV);
+    r = it[0];
+    q0 = it[1];
+    kt_begin = it[2];
+    kt_end = it[3];
+    part_row = it[4];
+  } else {
+    const int tile = (l / kHeadsKV) % a.num_tiles;
+    const int split = l / (kHeadsKV * a.num_tiles);
+    r = a.tile_req[tile];
+    q0 = a.tile_q0[tile];
+    if (a.split_tiles > 0) {
+      kt_begin = split * a.split_tiles;
+      kt_end = kt_begin + a.split_tiles;
+      part_row = (long)(a.split_base + split) * a.num_tokens + a.q_start[r] + q0;
+    }
+  }
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index (uniform)
   const int lane = tid & 63;
@@ -168,10 +188,9 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
   const int k_end = causal ? min(limit, kv0 + q_hi + 1) : limit;
   const int k_full = causal ? min(limit, kv0 + q0 + 1) : limit;
   const int n_k_tiles = (k_end + kBN - 1) / kBN;
-  // key tiles of this block: all of them, or split z's share when the launch is split along the keys
-  RangeWalk walk;
-  walk.kt_begin = a.split_tiles > 0 ? split * a.split_tiles : 0;
-  walk.kt_end = a.split_tiles > 0 ? min(n_k_tiles, walk.kt_begin + a.split_tiles) : n_k_tiles;
+  RangeWalk walk;                                           // this workgroup's key tiles
+  walk.kt_begin = kt_begin;
+  walk.kt_end = min(n_k_tiles, kt_end);
   walk.k_full = k_full;
   walk.ex_lo = walk.ex_hi = 0;
   if (!kSide && a.kv_excluded != nullptr) {
@@ -198,7 +217,7 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
   // exceed that), and the record (m, l, scale). The scale needs the row's largest |o| over its 128 dims, which lie in
   // the row's four lane groups (lanes m16 + 16j): reduced before any lane leaves.
   float amax[H];
-  if (a.split_tiles > 0) {
+  if (part_row >= 0) {
 #pragma unroll
     for (int u = 0; u < H; ++u) {
       float x = 0.f;
@@ -210,7 +229,7 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
     }
   }
   if (!qvalid) return;
-  if (a.split_tiles > 0) {                                   // partials of this key split
+  if (part_row >= 0) {                                       // partials of this key split
 #pragma unroll
     for (int u = 0; u < H; ++u) {
       const float l = l_run[u];
@@ -218,7 +237,7 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
       const float an = amax[u] * inv;
       const float scale = an > 32768.f ? an * (1.f / 32768.f) : 1.f;
       const int head = kvh * kGroup + hbase + u;
-      const long row = ((long)(a.split_base + split) * a.num_tokens + (t0 + qi)) * kHeadsQ + head;
+      const long row = (part_row + (qi - q0)) * kHeadsQ + head;
       _Float16* po = a.part_o + row * kHeadDim + 32 * j;
 #pragma unroll
       for (int p = 0; p < 4; ++p) store_acc_f16x8(po + 8 * p, o[2 * p][u], o[2 * p + 1][u], j, inv / scale);
@@ -239,15 +258,25 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
   }
 }
 
-// Combine the key-split partials of every query token: workgroup (token, group of 8 heads); thread t handles head
-// 8 * blockIdx.y + t / 32 and dims 4 * (t % 32) .. +4.
+// Combine the key-split partials of a query token: workgroup (token, group of 8 heads); thread t handles head
+// 8 * blockIdx.y + t / 32 and dims 4 * (t % 32) .. +4. Uniform splits: blockIdx.x is the token; work items: row
+// blockIdx.x % 64 of merged tile blockIdx.x / 64, whose splits' partials lie 64 rows apart.
 __global__ __launch_bounds__(256) void paged_merge_kernel(PagedPrefillArgs a, int n_splits) {
   typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-  const long tok = blockIdx.x;
+  long tok = blockIdx.x, first = tok, step = a.num_tokens;   // partial rows of the token: first, first + step, ...
+  if (a.merges != nullptr) {
+    const int32_t* mt = a.merges + 4 * (blockIdx.x / kBM);
+    const int row = blockIdx.x % kBM;
+    if (row >= mt[1]) return;
+    tok = mt[0] + row;
+    first = (long)mt[2] + row;
+    step = kBM;
+    n_splits = mt[3];
+  }
   const int head = 8 * blockIdx.y + (threadIdx.x >> 5);
   const int d0 = (threadIdx.x & 31) * 4;
-  const long stride = (long)a.num_tokens * kHeadsQ;          // rows per split
-  const float* pml = a.part_ml + (tok * kHeadsQ + head) * 4;
+  const long stride = step * kHeadsQ;                        // partial rows x heads per split
+  const float* pml = a.part_ml + (first * kHeadsQ + head) * 4;
   float M = -INFINITY;
 #pragma unroll 8
   for (int s = 0; s < n_splits; ++s) M = fmaxf(M, pml[s * stride * 4]);
@@ -260,7 +289,7 @@ __global__ __launch_bounds__(256) void paged_merge_kernel(PagedPrefillArgs a, in
       const float w = fast_exp2(rec[0] - M) * rec[1];      // the split's weight (0 for a split that saw no key)
       const float ws = w * rec[2];
       L += w;
-      const f16x4 h = *reinterpret_cast<const f16x4*>(a.part_o + ((s * stride) + tok * kHeadsQ + head) * kHeadDim + d0);
+      const f16x4 h = *reinterpret_cast<const f16x4*>(a.part_o + ((s * stride) + first * kHeadsQ + head) * kHeadDim + d0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[r] += ws * (float)h[r];
     }
@@ -333,6 +362,7 @@ int abkv_paged_prefill_attn(const void* q, long q_stride_t, long q_stride_h, con
   a.lse = lse;
   a.num_tokens = num_tokens;
   a.split_tiles = 0;
+  a.items = a.merges = nullptr;
   a.part_o = nullptr;
   a.part_ml = nullptr;
   a.split_base = 0;
@@ -353,6 +383,61 @@ int abkv_paged_prefill_attn(const void* q, long q_stride_t, long q_stride_h, con
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || num_splits <= 1) return (int)err;
   hipLaunchKernelGGL(paged_merge_kernel, dim3(num_tokens, kHeadsQ / 8), dim3(256), 0, stream, a, num_splits);
+  return (int)hipGetLastError();
+}
+
+int abkv_paged_prefill_attn_items(const void* q, long q_stride_t, long q_stride_h, const void* kv_cache, int num_pages,
+                                  const int32_t* block_table, long block_table_stride, int block_table_width,
+                                  const int32_t* q_start, const int32_t* kv_start, const int32_t* kv_limit,
+                                  const int32_t* kv_excluded, const int32_t* causal, const int32_t* items, int n_items,
+                                  const int32_t* merges, int n_merges, int part_rows, float scale, void* out,
+                                  long out_stride_t, long out_stride_h, float* lse, void* workspace,
+                                  size_t workspace_bytes, hipStream_t stream) {
+  using namespace abkv;
+  if (n_items <= 0) return 0;
+  if (q == nullptr || kv_cache == nullptr || block_table == nullptr || q_start == nullptr || kv_start == nullptr ||
+      kv_limit == nullptr || causal == nullptr || items == nullptr || out == nullptr || num_pages <= 0 ||
+      block_table_width <= 0 || n_merges < 0 || part_rows < 0 || (n_merges > 0 && merges == nullptr) ||
+      (part_rows > 0 && (workspace == nullptr || workspace_bytes < abkv_paged_prefill_workspace_size(part_rows, 1))) ||
+      (long)n_merges * kBM * 256 > 0xFFFFFFFFL)
+    return (int)hipErrorInvalidValue;
+  PagedPrefillArgs a;
+  a.q = static_cast<const __bf16*>(q);
+  a.q_st = q_stride_t;
+  a.q_sh = q_stride_h;
+  a.kv = static_cast<const __bf16*>(kv_cache);
+  a.num_pages = num_pages;
+  a.block_table = block_table;
+  a.bt_stride = block_table_stride;
+  a.bt_width = block_table_width;
+  a.q_start = q_start;
+  a.kv_start = kv_start;
+  a.kv_limit = kv_limit;
+  a.kv_excluded = kv_excluded;
+  a.tile_req = a.tile_q0 = nullptr;
+  a.causal = causal;
+  a.causal_default = 1;
+  a.scale_log2 = scale * 1.4426950408889634f;
+  a.out = static_cast<__bf16*>(out);
+  a.o_st = out_stride_t;
+  a.o_sh = out_stride_h;
+  a.lse = lse;
+  a.items = items;
+  a.merges = merges;
+  a.num_tiles = 0;
+  a.split_tiles = 0;
+  a.num_tokens = 0;
+  a.part_o = static_cast<_Float16*>(workspace);
+  a.part_ml = reinterpret_cast<float*>(a.part_o + (size_t)part_rows * kHeadsQ * kHeadDim);
+  a.split_base = 0;
+  a.head_quota = nullptr;
+  a.side_count = nullptr;
+  const unsigned grid = paged_grid(n_items, 1);
+  if (grid == 0) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(paged_prefill_kernel<false>, dim3(grid), dim3(512), 0, stream, a);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || n_merges == 0) return (int)err;
+  hipLaunchKernelGGL(paged_merge_kernel, dim3((unsigned)n_merges * kBM, kHeadsQ / 8), dim3(256), 0, stream, a, 0);
   return (int)hipGetLastError();
 }
 
@@ -415,6 +500,7 @@ int abkv_paged_prefill_attn_packed(const void* q, long q_stride_t, long q_stride
   a.o_sh = out_stride_h;
   a.lse = lse;
   a.num_tokens = num_tokens;
+  a.items = a.merges = nullptr;
   a.part_o = static_cast<_Float16*>(workspace);
   a.part_ml = reinterpret_cast<float*>(a.part_o + (size_t)total * num_tokens * kHeadsQ * kHeadDim);
   a.head_quota = head_quota_dev;

@@ -619,6 +619,21 @@ def paged_split_plan(num_tiles: int, max_keys: int, target_blocks: int | None = 
     return -(-max_kt // split_tiles), split_tiles
 
 
+def paged_plan(q_start, kv_start, kv_limit, causal, num_cus: int | None = None):
+    """Work items of a paged multi-query launch (abkv_paged_plan): (items int32 [n, 5], merged tiles int32 [m, 4],
+    partial rows) from int64 host arrays, for workgroups that end together on ``num_cus`` compute units."""
+    cus = _num_cus() if num_cus is None else int(num_cus)
+    qs, ks, kl, cz = (np.ascontiguousarray(x, dtype=np.int64) for x in (q_start, kv_start, kv_limit, causal))
+    cap = int((-(-np.diff(qs) // 64)).sum()) + 3 * max(1, cus // HEADS_KV)
+    buf = np.empty(9 * cap + 3, np.int32)
+    at = buf.ctypes.data
+    rc = lib().abkv_paged_plan(qs.ctypes.data, ks.ctypes.data, kl.ctypes.data, cz.ctypes.data, ks.size, cus, at, cap,
+                               at + 20 * cap, cap, at + 36 * cap)
+    _require(rc == 0, f"abkv_paged_plan failed ({rc})")
+    n, m, rows = buf[9 * cap:].tolist()
+    return buf[: 5 * n].reshape(n, 5), buf[5 * cap: 5 * cap + 4 * m].reshape(m, 4), rows
+
+
 def _excluded_pairs(excluded, B):
     """Per-request excluded key ranges as int32 [B, 2] (an empty range for None entries), or None for none at all."""
     import numpy as np
@@ -647,7 +662,7 @@ def paged_prefill_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table
     physical positions kv_start[r] + i, seeing keys < kv_limit[r] (and <= their own position when causal).
     ``causal``: a bool for the whole batch or one flag per request (code steps and prompt chunks may share a batch).
     ``excluded``: None, or per request a physical (start, end) its queries must not see (None: nothing), e.g. the
-    code step's own-block retained tail. ``split``: key splits (None: chosen by :func:`paged_split_plan`; 1: no split).
+    code step's own-block retained tail. ``split``: key splits of every tile (None: chosen per tile by :func:`paged_plan`; 1: no split).
     Returns (out [T, 32, 128] bf16, lse [T, 32] fp32 or None). fp32 q and cache select the fp32 mode (out fp32).
     """
     import numpy as np
@@ -695,23 +710,37 @@ def paged_prefill_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table
                                                out.stride(1), _ptr(lse), C.c_void_p(_stream()))
         check(rc, "abkv_paged_prefill_attn_f32")
         return out, lse
-    tiles = [(r, q0) for r in range(B) for q0 in range(0, int(nq[r]), 64)]
-    if not tiles:
+    if qs[-1] == 0:
         return out, lse
-    tr = np.asarray(tiles, dtype=np.int32)
     dev = q.device
     cz = np.broadcast_to(np.asarray(causal, dtype=np.int64), (B,)).astype(np.int64)
+    scale = default_scale() if scale is None else float(scale)
+    if split is None:
+        items, merges, part_rows = paged_plan(qs, ks, kl, cz)
+        meta = torch.from_numpy(np.concatenate([qs, ks, kl, cz, items.reshape(-1), merges.reshape(-1)])
+                                .astype(np.int32)).to(dev)
+        o1, o2, o3, o4 = B + 1, 2 * B + 1, 3 * B + 1, 4 * B + 1
+        o5 = o4 + items.size
+        ws, ws_bytes = None, 0
+        if part_rows:
+            ws_bytes = lib().abkv_paged_prefill_workspace_size(part_rows, 1)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        rc = lib().abkv_paged_prefill_attn_items(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
+                                                 _ptr(block_table), _row_stride(block_table), W, _ptr(meta[:o1]),
+                                                 _ptr(meta[o1:o2]), _ptr(meta[o2:o3]), _ptr(ex_t), _ptr(meta[o3:o4]),
+                                                 _ptr(meta[o4:o5]), len(items), _ptr(meta[o5:]), len(merges),
+                                                 part_rows, scale, _ptr(out), out.stride(0), out.stride(1), _ptr(lse),
+                                                 _ptr(ws), ws_bytes, C.c_void_p(_stream()))
+        check(rc, "abkv_paged_prefill_attn_items")
+        return out, lse
+    tr = np.asarray([(r, q0) for r in range(B) for q0 in range(0, int(nq[r]), 64)], dtype=np.int32)
     meta = torch.from_numpy(np.concatenate([qs, ks, kl, cz]).astype(np.int32)).to(dev)
     tl = torch.from_numpy(np.ascontiguousarray(tr.T)).to(dev)
     q_start_d, kv_start_d = meta[: B + 1], meta[B + 1: 2 * B + 1]
     kv_limit_d, causal_d = meta[2 * B + 1: 3 * B + 1], meta[3 * B + 1:]
-    scale = default_scale() if scale is None else float(scale)
     max_keys = int(kl.max()) if kl.size else 0
-    if split is None:
-        n_splits, split_tiles = paged_split_plan(len(tiles), max_keys)
-    else:
-        n_splits = max(1, int(split))
-        split_tiles = -(-(-(-max_keys // 64)) // n_splits) if n_splits > 1 else 0
+    n_splits = max(1, int(split))
+    split_tiles = -(-(-(-max_keys // 64)) // n_splits) if n_splits > 1 else 0
     ws, ws_bytes = None, 0
     covered = int(qs[-1])                    # rows the launch writes; rows past q_start[-1] stay untouched
     if n_splits > 1:
@@ -721,7 +750,7 @@ def paged_prefill_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table
     rc = lib().abkv_paged_prefill_attn(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
                                        _ptr(block_table), _row_stride(block_table), W, _ptr(q_start_d),
                                        _ptr(kv_start_d), _ptr(kv_limit_d), _ptr(ex_t), _ptr(tl[0]), _ptr(tl[1]),
-                                       len(tiles),
+                                       len(tr),
                                        _ptr(causal_d), 1, scale, _ptr(out), out.stride(0), out.stride(1), _ptr(lse),
                                        covered, n_splits, split_tiles, _ptr(ws), ws_bytes, C.c_void_p(_stream()))
     check(rc, "abkv_paged_prefill_attn")

@@ -234,6 +234,24 @@ int abkv_paged_prefill_attn(const void* q, long q_stride_t, long q_stride_h, con
                             int num_tokens, int num_splits, int split_tiles, void* workspace, size_t workspace_bytes,
                             abkv_stream_t stream);
 
+/* The same launch from a plan: abkv_paged_plan (host arrays, int64; no GPU call) splits the query tiles whose key range
+ * is long so that the launch's workgroups end together on num_cus compute units, and writes work items [n][5] (request,
+ * first query row, first and end key tile, first partial row or -1) and merged tiles [m][4] (first token, rows, first
+ * partial row, parts); sizes = {n, m, partial rows}. Capacities in items and tiles: 64-row query tiles of the batch +
+ * 3 * max(1, num_cus / 8) always suffice for both. ABKV_ERR_CAPACITY: too small (sizes are set). q_start [num_reqs + 1].
+ * abkv_paged_prefill_attn_items runs it (items and merges copied to the device; workspace >=
+ * abkv_paged_prefill_workspace_size(partial rows, 1)). */
+int abkv_paged_plan(const int64_t* q_start, const int64_t* kv_start, const int64_t* kv_limit, const int64_t* causal,
+                    int num_reqs, int num_cus, int32_t* items, long items_cap, int32_t* merges, long merges_cap,
+                    int32_t* sizes);
+int abkv_paged_prefill_attn_items(const void* q, long q_stride_t, long q_stride_h, const void* kv_cache, int num_pages,
+                                  const int32_t* block_table, long block_table_stride, int block_table_width,
+                                  const int32_t* q_start, const int32_t* kv_start, const int32_t* kv_limit,
+                                  const int32_t* kv_excluded, const int32_t* causal, const int32_t* items, int n_items,
+                                  const int32_t* merges, int n_merges, int part_rows, float scale, void* out,
+                                  long out_stride_t, long out_stride_h, float* lse, void* workspace,
+                                  size_t workspace_bytes, abkv_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------------------------
  * Per-head packed code pages (the reference's packed KV sidecar for per-head quota schedules:
  * third_party/vllm_overlay/vllm/v1/worker/compresslm_packed_kv.py:12-155 PackedKVLayout, :214-284 PackedKVSidecar

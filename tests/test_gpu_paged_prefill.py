@@ -164,3 +164,30 @@ def test_rows_past_the_covered_queries_are_untouched_with_key_splits():
         ro, _ = _oracle(q[q_start[r]: q_start[r + 1]].float().cpu().numpy(), cf, tables[r], resident[r], kv_limit[r],
                         causal=False)
         assert np.abs(out[q_start[r]: q_start[r + 1]].float().cpu().numpy() - ro).max() <= TOL
+
+
+@pytest.mark.parametrize("num_cus", [8, 64, 256, 1024])
+def test_planned_items_match_the_oracle(num_cus, monkeypatch):
+    """Planned work items (no split on one slot, up to many parts on 128): requests of 1 .. 130 rows, causal and not, an
+    empty key range, ranges on and off the 64-key grid, a partial last query tile among split ones. bf16 tolerance as
+    above (probabilities and partial outputs of 8 and 11 bits under |v| <= 5)."""
+    from abridgekv_amd import ops
+    monkeypatch.setattr(ops, "_NUM_CUS", num_cus)
+    qlen = [64, 1, 130, 70, 17, 64]
+    past = [3000, 64, 900, 0, 2047, 10]
+    causal = [False, True, True, True, False, False]
+    limits = [3010, 65, 1030, 70, 2048, 0]
+    cache, tables = _setup([a + b for a, b in zip(qlen, past)], 600, 9)
+    q_start = np.concatenate([[0], np.cumsum(qlen)])
+    g = torch.Generator().manual_seed(10)
+    q = torch.randn((int(q_start[-1]), 32, 128), generator=g).to(torch.bfloat16)
+    out, lse = _run(cache, tables, q, q_start, past, limits, causal)
+    cf = cache.float().numpy()
+    for r in range(len(qlen)):
+        a, z = q_start[r], q_start[r + 1]
+        if limits[r] == 0:
+            assert np.all(out[a:z] == 0) and np.all(np.isneginf(lse[a:z]))
+            continue
+        ro, rl = _oracle(q[a:z].float().numpy(), cf, tables[r], past[r], limits[r], causal[r])
+        assert np.abs(out[a:z] - ro).max() <= TOL
+        assert np.abs(lse[a:z] - rl).max() <= TOL
