@@ -25,16 +25,180 @@ struct PrefillBwdArgs {
   float* lse2;                                // workspace [B, 32, S0p]
   float* dvec;                                // workspace [B, 32, S0p]
   int S0p;                                    // S0 rounded up to a multiple of 64
+  int* seen;                                  // [key tiles x B] query tiles that see the key tile (workspace, as the next two)
+  int* done;                                  // [slot_cap x 8] finished parts, at the tile's first item
+  float* slots;                               // [slot_cap x 8][kSlotFloats] sums of the parts
+  int slot_cap;                               // partial slots per KV head
+  int workers;                                // workgroups of the dK/dV kernel the GPU runs at once, per KV head
+  int count_blocks;                           // workgroups of the prep kernel that count
   float scale;                                // softmax scale
   __bf16* dq; long dq_sb, dq_ss, dq_sh;       // [B, S0, 32, 128]
   __bf16* dk; long dk_sb, dk_ss, dk_sh;       // [B, S0, 8, 128]
   __bf16* dv; long dv_sb, dv_ss, dv_sh;
 };
 
+// Smallest v over the wave's lanes, in VALU (DPP inside rows of 16 lanes, then lane swaps): a TileSpan is twelve of
+// these, and as chains of LDS permutes they cost 3.5 us a key tile.
+__device__ __forceinline__ int wave_min(int v) {
+  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));    // quad_perm 1,0,3,2
+  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));    // quad_perm 2,3,0,1
+  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));   // row_half_mirror
+  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));   // row_mirror
+  const auto r16 = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = min((int)r16[0], (int)r16[1]);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return __builtin_amdgcn_readfirstlane(min((int)r32[0], (int)r32[1]));
+}
+
+// Which query tiles a 64-key tile is seen by, from the query ranges of its keys (lane l: key k0 + l; wave-uniform and
+// the same in every wave): a query tile outside the hulls of the ranges is hidden, one inside the common part of the
+// first (or of the second) ranges of all 64 keys is visible throughout, the others take the ranges per key.
+struct TileSpan {
+  int a1, e1, a2, e2;        // hulls over the keys that are no codes
+  int ca, ce;                // hull over the codes
+  int f1, g1, f2, g2;        // [f1, g1) and [f2, g2): rows that see every key (given the quota)
+  int slot_min, slot_max;    // of the codes
+  __device__ __forceinline__ explicit TileSpan(const KeySpan& s) {
+    const bool code = s.slot >= 0;
+    const bool r1 = s.a1 < s.e1, r2 = s.a2 < s.e2;
+    a1 = wave_min(!code && r1 ? s.a1 : kNoKey);
+    e1 = -wave_min(!code && r1 ? -s.e1 : 0);
+    a2 = wave_min(!code && r2 ? s.a2 : kNoKey);
+    e2 = -wave_min(!code && r2 ? -s.e2 : 0);
+    ca = wave_min(code && r1 ? s.a1 : code && r2 ? s.a2 : kNoKey);
+    ce = -wave_min(code ? -max(s.e1, s.e2) : 0);
+    f1 = -wave_min(-s.a1);
+    g1 = wave_min(s.e1);
+    f2 = -wave_min(-s.a2);
+    g2 = wave_min(s.e2);
+    slot_min = wave_min(code ? s.slot : kNoKey);
+    slot_max = -wave_min(-s.slot);
+  }
+  __device__ __forceinline__ int first_row() const { return min(min(a1, a2), ca); }
+  __device__ __forceinline__ int last_row() const { return max(max(e1, e2), ce); }
+  // -1 hidden, 0 every pair visible, 1 per key
+  __device__ __forceinline__ int mode(int q0, int q1, int quota) const {
+    const bool seen = (q0 < e1 && q1 > a1) || (q0 < e2 && q1 > a2) || (slot_min < quota && q0 < ce && q1 > ca);
+    if (!seen) return -1;
+    return ((q0 >= f1 && q1 <= g1) || (q0 >= f2 && q1 <= g2)) && slot_max < quota ? 0 : 1;
+  }
+};
+
+// Work of the dK/dV kernel. A key tile's cost is the query tiles that see it: a block's content is seen by its own block
+// only, its codes and the raw prompt by all later rows, so a launch of one workgroup per key tile can wait for the first
+// codes' workgroup. Tiles longer than 3/2 of a worker's even share of the launch are split into parts of at most the
+// share; the parts leave fp32 sums in slots, and the last part to finish adds them up in part order. Parts and long tiles
+// go first. The prep kernel counts (the raw prompt's length is not known on the host), each dK/dV workgroup finds its
+// part from the counts. Forward + backward calls, one workgroup per tile in tile order -> this: B=1, 8 x (512 + 128 + 16)
+// rows (82 query tiles against a share of 16) 960 -> 652 us, B=1, 10 x (512 + 128) 911 -> 585, causal 4000 rows 877 ->
+// 811; B=2, 12 x (512 + 128) (120 against 82: not split) 1835 -> 1829, and parts of 3/4 of the share, which lose the
+// reuse of query tiles in L2, 1905; B=2, 4 x (512 + 256) with a rolling tail 812 -> 838. A least part of 8 instead of 12
+// query tiles: causal 1500 rows 246 -> 260.
+constexpr int kDkvMinPart = 12;                // query tiles (x 4 heads) a part is worth starting for
+constexpr int kSlotFloats = 2 * kBN * kHeadDim;   // dK and dV of a key tile
+// One part: parts == 1: the whole tile.
+struct DkvItem {
+  int tile;                  // key tile * B + sequence
+  int z, parts, seen;        // part z of parts; query tiles that see the tile
+  int first;                 // the tile's first slot
+};
+
+// Largest code quota of all heads.
+__device__ __forceinline__ int quota_max(const PrefillArgs& f) {
+  return f.head_quota ? -wave_min(-f.head_quota[threadIdx.x & (kHeadsQ - 1)]) : f.K;
+}
+
+// The query tiles qt0 .. qt0 + 63 that see the key tile for some head (bit i: tile qt0 + i).
+__device__ __forceinline__ unsigned long long seen_mask(const PrefillArgs& f, const TileSpan& span, int qt0, int quota) {
+  const int qt = qt0 + (int)(threadIdx.x & 63);
+  return __ballot(qt * kBN < f.S0 && span.mode(qt * kBN, min(qt * kBN + kBN, f.S0), quota) >= 0);
+}
+
+// Sum of v over the workgroup's 256 threads (uniform).
+__device__ __forceinline__ int block_sum(int v, int* lds) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return lds[0] + lds[1] + lds[2] + lds[3];
+}
+
+// Parts of a tile that `seen` query tiles see, with an even share of `share` query tiles a worker.
+__device__ __forceinline__ int dkv_parts(int seen, int share) {
+  if (2 * seen <= 3 * share) return 1;                      // (at most 3/2 seen / share parts otherwise)
+  return (seen + share - 1) / share;
+}
+// Order of issue: 0 the split tiles' parts, then whole tiles by length: 1 over the share, 2 over half of it, 3 the rest.
+__device__ __forceinline__ int dkv_class(int seen, int share) {
+  return dkv_parts(seen, share) > 1 ? 0 : seen > share ? 1 : 2 * seen > share ? 2 : 3;
+}
+
+// Item i of a KV head (workgroup of 256 threads; uniform), by class and tile; false past the last.
+__device__ __forceinline__ bool dkv_item(const int* seen, int tiles, int workers, int i, DkvItem& item) {
+  __shared__ int lds[4];
+  __shared__ DkvItem found;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  int v = 0;
+  for (int e = tid; e < tiles; e += 256) v += seen[e];
+  const int share = max(kDkvMinPart, (block_sum(v, lds) + workers - 1) / workers);
+  int at = 0, cls = 0, n = 0;                                // the class that item i lies in: items at .. at + n - 1
+  for (; cls < 4; ++cls) {
+    v = 0;
+    for (int e = tid; e < tiles; e += 256) v += dkv_class(seen[e], share) == cls ? dkv_parts(seen[e], share) : 0;
+    n = block_sum(v, lds);
+    if (i < at + n) break;                                   // uniform
+    at += n;
+  }
+  if (cls == 4) return false;
+  for (int e0 = 0; e0 < tiles; e0 += 256) {
+    const int e = e0 + tid;
+    const int mine = e < tiles && dkv_class(seen[e], share) == cls ? dkv_parts(seen[e], share) : 0;
+    int scan = mine;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+      const int up = __shfl_up(scan, m, 64);
+      scan += lane >= m ? up : 0;
+    }
+    __syncthreads();
+    if (lane == 63) lds[w] = scan;
+    __syncthreads();
+    int before = at + scan - mine;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      before += k < w ? lds[k] : 0;
+      at += lds[k];
+    }
+    if (i >= before && i < before + mine) found = DkvItem{e, i - before, mine, seen[e], before};
+    if (i < at) break;                                      // uniform
+  }
+  __syncthreads();
+  item = found;
+  return true;
+}
+
+// Prep's part of it: four key tiles a workgroup, one per wave.
+__device__ __forceinline__ void dkv_count(const PrefillBwdArgs& a, int block) {
+  const PrefillArgs& f = a.f;
+  const int lane = threadIdx.x & 63;
+  const int e = 4 * block + (threadIdx.x >> 6);
+  if (block == 0)
+    for (int i = threadIdx.x; i < a.slot_cap * kHeadsKV; i += 256) a.done[i] = 0;
+  if (e >= f.num_q_tiles * f.B) return;
+  const int b = e % f.B, k0 = e / f.B * kBN;
+  const TileSpan span(key_span(mask_shape(f), k0 + lane, f.prompt_len ? f.prompt_len[b] : 0));
+  const int quota = quota_max(f);
+  int n = 0;
+  for (int qt = span.first_row() / kBN; qt * kBN < span.last_row(); qt += 64)
+    n += __popcll(seen_mask(f, span, qt, quota));
+  if (lane == 0) a.seen[e] = n;
+}
+
 __global__ __launch_bounds__(256) void prefill_bwd_prep_kernel(PrefillBwdArgs a) {
   // 16 lanes per (row, query head): lane c takes dims 8c .. 8c + 7 of O and dO (one 16-byte load each, so a wave reads
   // four whole 256-byte rows), and the 16 partial dot products are summed by lane shuffles inside the group
-  const long idx = ((long)blockIdx.x * 256 + threadIdx.x) >> 4;
+  if ((int)blockIdx.x < a.count_blocks) return dkv_count(a, blockIdx.x);
+  const long idx = ((long)((int)blockIdx.x - a.count_blocks) * 256 + threadIdx.x) >> 4;
   const int c = threadIdx.x & 15;
   if (idx >= (long)a.f.B * kHeadsQ * a.S0p) return;         // uniform over the 16 lanes of a row
   const int i = (int)(idx % a.S0p);
@@ -213,47 +377,6 @@ __global__ __launch_bounds__(512, 1) void prefill_bwd_dq_kernel(PrefillBwdArgs a
   }
 }
 
-// Smallest v over the wave's lanes.
-__device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v = min(v, __shfl_xor(v, m, 64));
-  return __builtin_amdgcn_readfirstlane(v);
-}
-
-// Which query tiles a 64-key tile is seen by, from the query ranges of its keys (lane l: key k0 + l; wave-uniform and
-// the same in every wave): a query tile outside the hulls of the ranges is hidden, one inside the common part of the
-// first (or of the second) ranges of all 64 keys is visible throughout, the others take the ranges per key.
-struct TileSpan {
-  int a1, e1, a2, e2;        // hulls over the keys that are no codes
-  int ca, ce;                // hull over the codes
-  int f1, g1, f2, g2;        // [f1, g1) and [f2, g2): rows that see every key (given the quota)
-  int slot_min, slot_max;    // of the codes
-  __device__ __forceinline__ explicit TileSpan(const KeySpan& s) {
-    const bool code = s.slot >= 0;
-    const bool r1 = s.a1 < s.e1, r2 = s.a2 < s.e2;
-    a1 = wave_min(!code && r1 ? s.a1 : kNoKey);
-    e1 = -wave_min(!code && r1 ? -s.e1 : 0);
-    a2 = wave_min(!code && r2 ? s.a2 : kNoKey);
-    e2 = -wave_min(!code && r2 ? -s.e2 : 0);
-    ca = wave_min(code && r1 ? s.a1 : code && r2 ? s.a2 : kNoKey);
-    ce = -wave_min(code ? -max(s.e1, s.e2) : 0);
-    f1 = -wave_min(-s.a1);
-    g1 = wave_min(s.e1);
-    f2 = -wave_min(-s.a2);
-    g2 = wave_min(s.e2);
-    slot_min = wave_min(code ? s.slot : kNoKey);
-    slot_max = -wave_min(-s.slot);
-  }
-  __device__ __forceinline__ int first_row() const { return min(min(a1, a2), ca); }
-  __device__ __forceinline__ int last_row() const { return max(max(e1, e2), ce); }
-  // -1 hidden, 0 every pair visible, 1 per key
-  __device__ __forceinline__ int mode(int q0, int q1, int quota) const {
-    const bool seen = (q0 < e1 && q1 > a1) || (q0 < e2 && q1 > a2) || (slot_min < quota && q0 < ce && q1 > ca);
-    if (!seen) return -1;
-    return ((q0 >= f1 && q1 <= g1) || (q0 >= f2 && q1 <= g2)) && slot_max < quota ? 0 : 1;
-  }
-};
-
 // S = Q K^T and dP = dO V^T of a wave's 16 keys over one staged tile (32 ds_read_b128, 32 MFMAs). The two products
 // are interleaved and the reads run eight ahead of the MFMAs: at 2 waves per SIMD the other wave alone cannot cover
 // an LDS round trip per MFMA.
@@ -318,10 +441,11 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
   float* const Lb[2] = {L0, L1};
   float* const Eb[2] = {E0, E1};
   const PrefillArgs& f = a.f;
-  const GridPos gp = grid_pos(f.B);
-  const int kt = gp.rank;                                   // earlier key tiles are seen by more query tiles
-  const int kvh = gp.kvh;
-  const int b = gp.b;
+  const int kvh = blockIdx.x % kHeadsKV;                    // a KV head's workgroups on one XCD, as grid_pos
+  DkvItem item;
+  if (!dkv_item(a.seen, f.num_q_tiles * f.B, a.workers, blockIdx.x / kHeadsKV, item)) return;
+  const int kt = item.tile / f.B;
+  const int b = item.tile - kt * f.B;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int m16 = lane & 15, j = lane >> 4;
@@ -358,8 +482,24 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
   if (w == 0) key_spans[lane] = lane_key;                   // read by masked tiles (held in registers it spills);
                                                             // published by the first step's barrier
   const TileSpan span(lane_key);
-  const int qt_end = (span.last_row() + kBN - 1) / kBN;
+  int qt_end = (span.last_row() + kBN - 1) / kBN;
   int qt = span.first_row() / kBN, h = -1, mode = 0;
+  if (item.parts > 1) {                                     // this part's share of the query tiles
+    const int quota = quota_max(f);
+    auto nth = [&](int n) {                                 // the n-th query tile that sees the key tile
+      for (int t = span.first_row() / kBN; t < qt_end; t += 64) {
+        unsigned long long m = seen_mask(f, span, t, quota);
+        if (n < __popcll(m)) {
+          for (; n > 0; --n) m &= m - 1;
+          return t + __ffsll(m) - 1;
+        }
+        n -= __popcll(m);
+      }
+      return qt_end;
+    };
+    qt = nth((int)((long)item.seen * item.z / item.parts));
+    qt_end = nth((int)((long)item.seen * (item.z + 1) / item.parts));
+  }
   auto next_pair = [&]() -> bool {
     for (;;) {
       if (++h == kGroup) {
@@ -442,6 +582,42 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
     }
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  if (item.parts > 1) {
+    // sums of this part to its slot (lane order: whole 1 KiB runs); the part that finishes last adds the parts up in
+    // order. Every slot's stores are released before the count and read after it is acquired (agent scope: the parts
+    // may run on different XCDs). No part waits for another.
+    __shared__ int finished;
+    floatx4* slot = reinterpret_cast<floatx4*>(a.slots) +
+                    ((long)(item.first * kHeadsKV + kvh) * kWaves + w) * (16 * 64) + lane;
+    constexpr long kSlotStep = (long)kHeadsKV * kSlotFloats / 4;    // between the parts of a tile
+    floatx4* mine = slot + item.z * kSlotStep;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      mine[64 * i] = dk[i][0];
+      mine[64 * (8 + i)] = dv[i][0];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __syncthreads();
+    if (threadIdx.x == 0)
+      finished = __hip_atomic_fetch_add(a.done + item.first * kHeadsKV + kvh, 1, __ATOMIC_ACQ_REL,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (finished != item.parts - 1) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      dk[i][0] = slot[64 * i];
+      dv[i][0] = slot[64 * (8 + i)];
+    }
+    for (int z = 1; z < item.parts; ++z) {
+      slot += kSlotStep;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        dk[i][0] += slot[64 * i];
+        dv[i][0] += slot[64 * (8 + i)];
+      }
+    }
+  }
   if (key >= f.S0) return;
   __bf16* kp = a.dk + (long)b * a.dk_sb + (long)key * a.dk_ss + (long)kvh * a.dk_sh + 32 * j;
   __bf16* vp = a.dv + (long)b * a.dv_sb + (long)key * a.dv_ss + (long)kvh * a.dv_sh + 32 * j;
@@ -452,15 +628,38 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
   }
 }
 
+// Workspace offsets.
+struct BwdLayout {
+  size_t dvec, seen, done, slots, bytes;
+  int workers, cap;                           // cap: partial slots per KV head (parts of split tiles)
+};
+static BwdLayout bwd_layout(int batch, int seq_len) {
+  const size_t q_tiles = ((size_t)(seq_len > 0 ? seq_len : 0) + kBN - 1) / kBN;
+  const size_t tiles = q_tiles * (size_t)(batch > 0 ? batch : 0);
+  const size_t row_bytes = tiles * kBN * kHeadsQ * sizeof(float);
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  BwdLayout l;
+  l.workers = 2 * 256 / kHeadsKV;             // two workgroups a CU on 256 CUs
+  // parts (dkv_parts): at most 3/2 * workers in all (48 MiB of slots), and a tile's are under q_tiles / kDkvMinPart + 1
+  const size_t few = tiles * (q_tiles / kDkvMinPart + 1);
+  l.cap = (int)(few < (size_t)(3 * l.workers / 2) ? few : (size_t)(3 * l.workers / 2));
+  if (2 * q_tiles <= 3 * kDkvMinPart) l.cap = 0;            // nothing is split
+  l.dvec = row_bytes;
+  l.seen = up(2 * row_bytes);
+  l.done = l.seen + up(tiles * sizeof(int));
+  l.slots = l.done + up((size_t)l.cap * kHeadsKV * sizeof(int));
+  l.bytes = l.slots + (size_t)l.cap * kHeadsKV * kSlotFloats * sizeof(float) + 16;   // + the base's alignment
+  return l;
+}
+
 }  // namespace abkv
 
 extern "C" {
 
 // Workspace bytes of abkv_prefill_masked_attn_bwd: lse * log2(e) and rowsum(dO * O) per (batch, query head, row),
-// rows padded to whole 64-row tiles.
+// rows padded to whole 64-row tiles; the dK/dV counts and partial slots.
 size_t abkv_prefill_masked_bwd_workspace_size(int batch, int seq_len) {
-  const size_t s0p = ((size_t)(seq_len > 0 ? seq_len : 0) + 63) / 64 * 64;
-  return 2 * (size_t)(batch > 0 ? batch : 0) * abkv::kHeadsQ * s0p * sizeof(float);
+  return abkv::bwd_layout(batch, seq_len).bytes;
 }
 
 int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s, long q_stride_h, const void* k,
@@ -519,8 +718,16 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
   a.g_sb = dout_stride_b; a.g_ss = dout_stride_s; a.g_sh = dout_stride_h;
   a.lse = lse;
   a.S0p = f.num_q_tiles * kBM;
-  a.lse2 = static_cast<float*>(workspace);
-  a.dvec = a.lse2 + (size_t)batch * kHeadsQ * a.S0p;
+  const BwdLayout lay = bwd_layout(batch, seq_len);
+  char* ws = static_cast<char*>(workspace) + (-reinterpret_cast<uintptr_t>(workspace) & 15);
+  a.lse2 = reinterpret_cast<float*>(ws);
+  a.dvec = reinterpret_cast<float*>(ws + lay.dvec);
+  a.seen = reinterpret_cast<int*>(ws + lay.seen);
+  a.done = reinterpret_cast<int*>(ws + lay.done);
+  a.slots = reinterpret_cast<float*>(ws + lay.slots);
+  a.slot_cap = lay.cap;
+  a.workers = lay.workers;
+  a.count_blocks = (f.num_q_tiles * batch + 3) / 4;
   a.scale = scale;
   a.dq = static_cast<__bf16*>(dq);
   a.dq_sb = dq_stride_b; a.dq_ss = dq_stride_s; a.dq_sh = dq_stride_h;
@@ -530,8 +737,11 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
   a.dv_sb = dv_stride_b; a.dv_ss = dv_stride_s; a.dv_sh = dv_stride_h;
   if (prefill_grid(f.num_q_tiles, batch, 512) == 0) return (int)hipErrorInvalidValue;
   const long rows = (long)batch * kHeadsQ * a.S0p;
-  if (rows * 16 > 0xFFFFFFFFL) return (int)hipErrorInvalidValue;  // prep: 16 work-items per row and head
-  hipLaunchKernelGGL(prefill_bwd_prep_kernel, dim3((unsigned)((rows * 16 + 255) / 256)), dim3(256), 0, stream, a);
+  const long gk = ((long)lay.cap + (long)f.num_q_tiles * batch) * kHeadsKV;   // at least the items of dkv_item
+  // prep: 16 work-items per row and head, and the counting workgroups
+  if (rows * 16 + 256L * (a.count_blocks + 1) > 0xFFFFFFFFL || gk * 256 > 0xFFFFFFFFL) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(prefill_bwd_prep_kernel, dim3((unsigned)((rows * 16 + 255) / 256 + a.count_blocks)), dim3(256), 0, stream,
+                     a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return (int)err;
   const unsigned gq = prefill_grid(f.num_q_tiles, batch, 512);
@@ -544,8 +754,7 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
   else hipLaunchKernelGGL((prefill_bwd_dq_kernel<false, false, false>), gq, dim3(512), 0, stream, a);
   err = hipGetLastError();
   if (err != hipSuccess) return (int)err;
-  const unsigned gk = prefill_grid(f.num_q_tiles, batch, 256);
-  hipLaunchKernelGGL(prefill_bwd_dkv_kernel, gk, dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(prefill_bwd_dkv_kernel, dim3((unsigned)gk), dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 

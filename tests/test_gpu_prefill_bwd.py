@@ -228,3 +228,33 @@ def test_config4_full_size_sampled(case):
             ref_k, ref_v = op.masked_attention_key_grads_fp64(qb, kb, vb, gb, mask_fn, keys, scale)
             close(f"dk b{b}", dk[b].float().cpu().numpy()[keys], ref_k)
             close(f"dv b{b}", dv[b].float().cpu().numpy()[keys], ref_v)
+
+
+@pytest.mark.parametrize("case", ["aligned", "replay", "causal"])
+def test_long_key_tiles_split_into_parts(case):
+    """Sequences whose first codes (raw prompt, causal keys) are seen by enough query tiles that their dK/dV work is
+    split into two and three parts, beside tiles that are not; tolerance as above (the parts' sums are fp32)."""
+    quota = np.repeat([32, 16, 20, 32, 1, 31, 32, 8], 4).tolist()
+    if case == "aligned":
+        _check(C=256, K=64, N=5, B=1, prompt_len=[700], seed=40)
+    elif case == "replay":
+        _check(C=192, K=32, N=6, B=1, prompt_len=[300], head_quota=quota, seed=41, replay=16)
+    else:
+        _check(C=1700, K=0, N=1, B=1, seed=42)
+
+
+def test_split_parts_add_up_in_a_fixed_order():
+    """The part that finishes last adds the parts in part order: repeated backward passes are bit-identical."""
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    C, K, N, R = 512, 128, 4, 16
+    S = N * (C + K + R)
+    g = torch.Generator(device=dev).manual_seed(3)
+    q, dout = (torch.randn((1, S, 32, 128), generator=g, device=dev).bfloat16() for _ in range(2))
+    k, v = (torch.randn((1, S, 8, 128), generator=g, device=dev).bfloat16() for _ in range(2))
+    lse = torch.empty((1, 32, S), dtype=torch.float32, device=dev)
+    out, _ = ops.prefill_masked_attention(q, k, v, C, K, N, lse=lse, replay_rows=R)
+    first = ops.prefill_masked_attention_backward(q, k, v, out, lse, dout, C, K, N, replay_rows=R)
+    for _ in range(4):
+        again = ops.prefill_masked_attention_backward(q, k, v, out, lse, dout, C, K, N, replay_rows=R)
+        assert all(torch.equal(a, b) for a, b in zip(first, again))
