@@ -109,15 +109,54 @@ __device__ __forceinline__ void store_partial(const DecodeArgs& a, long slot, in
     *reinterpret_cast<floatx4*>(a.part_ml + (slot * kHeadsQ + head) * 4) = floatx4{m_run, l_tot, scale, 0.f};
 }
 
-template <int kW>
-__global__ __launch_bounds__(64 * kW) void decode_attn_kernel(DecodeArgs a) {
-  // Grid (max_splits * 8 / kW, B): kW waves per workgroup, wave = KV head; the 8 / kW workgroups of a split are
-  // adjacent in x. Split fastest (dispatch order: the splits of sequence 0, then of sequence 1, ...), measured faster
-  // than sequence-fastest orders on the saturated workload.
+// The end of a split shared by kSub waves, one wave per query head u (lane: dims 2 * lane, 2 * lane + 1): the output, or the
+// split's partial as store_partial writes it. A wave without pages left m = -inf, l = 0, o = 0.
+template <int kSub>
+__device__ __forceinline__ void combine_subs(const DecodeArgs& a, const float (&so)[kSub][kGroup][kHeadDim],
+                                             const float (&sm)[kSub][kGroup], const float (&sl)[kSub][kGroup], int b,
+                                             int split, int head, int u, int lane, bool partial) {
+  float m = -INFINITY, l = 0.f, x = 0.f, y = 0.f;
+#pragma unroll
+  for (int s = 0; s < kSub; ++s) m = fmaxf(m, sm[s][u]);
+#pragma unroll
+  for (int s = 0; s < kSub; ++s) {
+    const float f = sm[s][u] == -INFINITY ? 0.f : fast_exp2(sm[s][u] - m);
+    const float2 v = *reinterpret_cast<const float2*>(&so[s][u][2 * lane]);
+    l += sl[s][u] * f;
+    x += v.x * f;
+    y += v.y * f;
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (!partial) {
+    *reinterpret_cast<uint32_t*>(a.out + (long)b * a.o_sb + (long)head * a.o_sh + 2 * lane) =
+        pack_bf16x2(x * inv, y * inv);
+    if (a.lse != nullptr && lane == 0)
+      a.lse[(long)b * kHeadsQ + head] = l > 0.f ? (m + __log2f(l)) * 0.69314718055994531f : -INFINITY;
+    return;
+  }
+  float an = fmaxf(fabsf(x), fabsf(y)) * inv;
+#pragma unroll
+  for (int k = 1; k < 64; k <<= 1) an = fmaxf(an, __shfl_xor(an, k, 64));
+  const float scale = an > 32768.f ? an * (1.f / 32768.f) : 1.f;
+  const float f = inv / scale;
+  const long at = ((long)b * a.part_stride + split) * kHeadsQ + head;
+  *reinterpret_cast<uint32_t*>(a.part_o + at * kHeadDim + 2 * lane) = pack_f16x2(x * f, y * f);
+  if (lane == 0) *reinterpret_cast<floatx4*>(a.part_ml + at * 4) = floatx4{m, l, scale, 0.f};
+}
+
+template <int kW, int kSub>
+__global__ __launch_bounds__(64 * kW * kSub) void decode_attn_kernel(DecodeArgs a) {
+  // Grid (max_splits * 8 / kW, B): kW KV heads per workgroup, a wave each (kSub == 1); the 8 / kW workgroups of a split
+  // are adjacent in x. Split fastest (dispatch order: the splits of sequence 0, then of sequence 1, ...), measured faster
+  // than sequence-fastest orders on the saturated workload. kSub > 1 (kW == 1): kSub waves share the split of one KV
+  // head, wave s taking page pairs s, s + kSub, ..., and their results meet in LDS (see launch_decode).
+  static_assert(kSub == 1 || (kW == 1 && kSub == kGroup), "a shared split has one KV head and a wave per query head");
   const int b = blockIdx.y;
   constexpr int kParts = kHeadsKV / kW;
   const int split = blockIdx.x / kParts;
-  const int kvh = (int)(blockIdx.x % kParts) * kW + (threadIdx.x >> 6);
+  const int wave = threadIdx.x >> 6;
+  const int kvh = (int)(blockIdx.x % kParts) * kW + (kSub == 1 ? wave : 0);
+  const int sub = kSub == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave);
   const int lane = threadIdx.x & 63;
   const int m16 = lane & 15;                  // MFMA row/col index of this lane
   const int j = lane >> 4;                    // lane group (k-chunk index)
@@ -154,7 +193,7 @@ __global__ __launch_bounds__(64 * kW) void decode_attn_kernel(DecodeArgs a) {
   int pid_l = 0;
   if (lane < pg_end - pg_begin) pid_l = min(max(bt[pg_begin + lane], 0), a.num_pages - 1);
   const __bf16* kv_h = a.kv + kvh * kHeadDim;
-  for (int pg = pg_begin; pg < pg_end; pg += 2) {
+  for (int pg = pg_begin + 2 * sub; pg < pg_end; pg += 2 * kSub) {
     const int p0 = __builtin_amdgcn_readlane(pid_l, pg - pg_begin);
     const int p1 = __builtin_amdgcn_readlane(pid_l, min(pg + 1, pg_end - 1) - pg_begin);
     const __bf16* base0 = kv_h + (long)p0 * kPageElems;
@@ -246,6 +285,25 @@ __global__ __launch_bounds__(64 * kW) void decode_attn_kernel(DecodeArgs a) {
   // o[i][r] = un-normalised out[head m16][dim 32j + 8r + i]; l_run partial over this lane's slots.
   const float l_tot = sum_xor32(sum_xor16(l_run));
   const bool partial = n_splits > 1 || a.force_partials;
+  if constexpr (kSub > 1) {
+    __shared__ __attribute__((aligned(16))) float so[kSub][kGroup][kHeadDim];
+    __shared__ float sm[kSub][kGroup], sl[kSub][kGroup];
+    if (m16 < kGroup) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          *reinterpret_cast<floatx4*>(&so[sub][m16][32 * j + 8 * r + 4 * h]) =
+              floatx4{o[4 * h][r], o[4 * h + 1][r], o[4 * h + 2][r], o[4 * h + 3][r]};
+      if (j == 0) {
+        sm[sub][m16] = m_run;
+        sl[sub][m16] = l_tot;
+      }
+    }
+    __syncthreads();
+    combine_subs<kSub>(a, so, sm, sl, b, split, kvh * kGroup + wave, wave, lane, partial);
+    return;
+  }
   const float amax = partial ? column_absmax(o) : 0.f;    // (a uniform branch: all lanes take part in the shuffles)
   if (m16 >= kGroup) return;
   const int head = kvh * kGroup + m16;
@@ -502,9 +560,23 @@ __global__ __launch_bounds__(64) void decode_side_kernel(DecodeArgs a) {
 // Two waves (two KV heads) per workgroup: the four workgroups of a split are adjacent in dispatch order. Measured in
 // one process over the same pages: two waves 952.9 us per launch against four 959.1 and eight 990.5 on the saturated
 // B=256 workload, 241.5 against 245.1 and 254.7 on the B=64 full-model decode; one wave 4 % slower than four.
+// Few splits leave the GPU idle, and the launch is as long as one wave's walk over its split: then four waves share each
+// KV head's split. us a call with a wave per split / shared: one sequence of 1068 rows 19.7 / 17.6, of 9000 24.3 / 17.7,
+// 4 of 1000 .. 3000 24.6 / 17.8, 16 of 1000 .. 5000 (160 splits) 60.9 / 50.3, 64 of 50 .. 500 (one split each) 25.3 /
+// 21.3. Past that the waves are there anyway: 128 of 100 .. 500 37.4 / 39.3, 64 of 500 .. 1023 beside packed pages (128
+// splits) 253 / 256, 64 of 5000 (704) 245.5 / 250.7. Eight waves: within 2 % of four.
+inline bool share_splits(int max_splits, int num_seqs) {
+  const long splits = (long)max_splits * num_seqs;
+  return splits <= 64 || (num_seqs <= 32 && splits <= 192);
+}
 inline void launch_decode(const DecodeArgs& a, int max_splits, int num_seqs, hipStream_t stream) {
+  if (share_splits(max_splits, num_seqs)) {
+    hipLaunchKernelGGL((decode_attn_kernel<1, kGroup>), dim3(max_splits * kHeadsKV, num_seqs), dim3(64 * kGroup), 0,
+                       stream, a);
+    return;
+  }
   constexpr int kW = 2;
-  hipLaunchKernelGGL(decode_attn_kernel<kW>, dim3(max_splits * (kHeadsKV / kW), num_seqs), dim3(64 * kW), 0, stream,
+  hipLaunchKernelGGL((decode_attn_kernel<kW, 1>), dim3(max_splits * (kHeadsKV / kW), num_seqs), dim3(64 * kW), 0, stream,
                      a);
 }
 

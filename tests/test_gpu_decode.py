@@ -219,3 +219,24 @@ def test_seeded_random_batches(seed):
     ref_out, ref_lse = _oracle(q, cache, tables, sl)
     assert np.abs(out - ref_out).max() <= TOL
     assert np.abs(lse - ref_lse).max() <= TOL
+
+
+@pytest.mark.parametrize("batch", [5, 64, 65])
+@pytest.mark.parametrize("split_pages", [2, 8, 32])
+def test_shared_splits_and_one_wave_per_split_agree_with_the_oracle(batch, split_pages):
+    """Both sides of the rule that lets four waves share a split (few sequences and splits) or gives each split one
+    wave: row counts around the page pairs that the four waves start with and their second turn, a partial last pair,
+    an empty sequence. Tolerance as above."""
+    edges = [0, 1, 16, 17, 32, 33, 127, 128, 129, 160, 257, 300]
+    rng = np.random.default_rng(batch + split_pages)
+    lens = [edges[i % len(edges)] for i in range(batch)]
+    rows_k = [_bf16_round(rng.standard_normal((n, 8, 128))) for n in lens]
+    rows_v = [_bf16_round(rng.standard_normal((n, 8, 128))) for n in lens]
+    cache, tables, sl = _paged_cache(rows_k, rows_v, sum(-(-n // 16) for n in lens) + 8, rng)
+    q = _bf16_round(2 * rng.standard_normal((batch, 32, 128)))
+    out, lse = _run(q, cache, tables, sl, split_pages=split_pages)
+    ref_o, ref_l = _oracle(q, cache, tables, sl)
+    assert np.abs(out - ref_o).max() <= TOL
+    live = sl > 0
+    assert np.abs(lse[live] - ref_l[live]).max() <= TOL
+    assert np.all(np.isneginf(lse[~live])) and np.all(out[~live] == 0)
