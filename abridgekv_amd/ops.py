@@ -25,12 +25,15 @@ DEFAULT_SPLIT_PAGES = 32                       # 512 slots per split
 AUTO_SPLIT_CHOICES = (48, 40, 32)               # pages per split the host may pick (a workspace for 32 fits all)
 
 
+# Every call below is a few microseconds of GPU work in the small cases, so the wrappers stay lean: the stream's handle
+# without a Stream object, addresses as plain integers, messages built only when a check fails.
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the caller's current stream on the current device."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -54,10 +57,18 @@ def _row_stride(block_table: torch.Tensor) -> int:
     return block_table.stride(0)
 
 
+_PAGE_SHAPE = (2, PAGE, HEADS_KV, HEAD_DIM)
+_Q_ROW = (HEADS_Q, HEAD_DIM)
+_KV_ROW = (HEADS_KV, HEAD_DIM)
+
+
 def _check_cache(kv_cache: torch.Tensor, dtype=torch.bfloat16) -> None:
+    if (kv_cache.is_cuda and kv_cache.dtype == dtype and kv_cache.dim() == 5 and kv_cache.shape[1:] == _PAGE_SHAPE
+            and kv_cache.is_contiguous()):
+        return
     _require(kv_cache.is_cuda, "kv_cache must be on the GPU")
     _require(kv_cache.dtype == dtype, f"kv_cache must be {dtype}")
-    _require(kv_cache.dim() == 5 and tuple(kv_cache.shape[1:]) == (2, PAGE, HEADS_KV, HEAD_DIM),
+    _require(kv_cache.dim() == 5 and tuple(kv_cache.shape[1:]) == _PAGE_SHAPE,
              f"kv_cache must be [P, 2, {PAGE}, {HEADS_KV}, {HEAD_DIM}], got {tuple(kv_cache.shape)}")
     _require(kv_cache.is_contiguous(), "kv_cache must be contiguous")
 
@@ -110,8 +121,8 @@ def decode_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch
     if q.dtype == torch.float32:
         return _decode_attention_f32(q, kv_cache, block_table, seq_lens, scale, max_pages, out, lse)
     _check_cache(kv_cache)
-    _require(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and tuple(q.shape[1:]) == (HEADS_Q, HEAD_DIM),
-             f"q must be cuda bf16 [B, {HEADS_Q}, {HEAD_DIM}]")
+    _require(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and q.shape[1:] == _Q_ROW,
+             "q must be cuda bf16 [B, 32, 128]")
     _require(q.stride(2) == 1, "q dims must be contiguous")
     B = q.shape[0]
     _require(block_table.is_cuda and block_table.dtype == torch.int32 and block_table.dim() == 2
@@ -124,7 +135,7 @@ def decode_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch
     _require(0 < max_pages <= W, "max_pages must be in [1, block_table width]")
     if out is None:
         out = torch.empty((B, HEADS_Q, HEAD_DIM), dtype=torch.bfloat16, device=q.device)
-    _require(out.dtype == torch.bfloat16 and tuple(out.shape) == (B, HEADS_Q, HEAD_DIM) and out.stride(2) == 1,
+    _require(out.dtype == torch.bfloat16 and out.shape == (B, HEADS_Q, HEAD_DIM) and out.stride(2) == 1,
              "out must be bf16 [B, 32, 128] with contiguous dims")
     if lse is not None:
         _require(lse.dtype == torch.float32 and lse.is_contiguous() and lse.numel() >= B * HEADS_Q,
@@ -141,7 +152,7 @@ def decode_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch
                                 _ptr(block_table),
                                 _row_stride(block_table), _ptr(seq_lens), B, max_pages, split_pages, float(scale),
                                 _ptr(out), out.stride(0), out.stride(1), _ptr(lse), _ptr(workspace), ws_bytes,
-                                C.c_void_p(_stream()))
+                                _stream())
     check(rc, "abkv_decode_attn")
     return out, lse
 
@@ -183,7 +194,7 @@ def decode_attention_noalloc(q: torch.Tensor, kv_cache: torch.Tensor, block_tabl
     rc = lib().abkv_decode_attn_noalloc(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
                                         _ptr(block_table), _row_stride(block_table), _ptr(seq_lens), B, max_pages,
                                         split_pages, float(scale), _ptr(out), out.stride(0), out.stride(1),
-                                        _ptr(lse), C.c_void_p(_stream()))
+                                        _ptr(lse), _stream())
     if rc == ABKV_ERR_SCRATCH:
         raise ValueError("abkv_decode_attn_noalloc: the batch needs more than the static scratch")
     check(rc, "abkv_decode_attn_noalloc")
@@ -211,7 +222,7 @@ def _decode_attention_f32(q, kv_cache, block_table, seq_lens, scale, max_pages, 
     rc = lib().abkv_decode_attn_f32(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
                                     _ptr(block_table), _row_stride(block_table), _ptr(seq_lens), B, max_pages,
                                     float(scale), _ptr(out), out.stride(0), out.stride(1), _ptr(lse),
-                                    C.c_void_p(_stream()))
+                                    _stream())
     check(rc, "abkv_decode_attn_f32")
     return out, lse
 
@@ -237,7 +248,7 @@ def kv_move_segments(layer_caches, ops: torch.Tensor, seg_offsets: torch.Tensor)
         return
     arr, num_pages = _layer_ptrs(layer_caches)
     rc = lib().abkv_kv_move_segments(arr, len(layer_caches), num_pages, PAGE, PAGE_BYTES, HALF_BYTES, SLOT_BYTES, _ptr(ops),
-                                     _ptr(seg_offsets), n_seg, C.c_void_p(_stream()))
+                                     _ptr(seg_offsets), n_seg, _stream())
     check(rc, "abkv_kv_move_segments")
 
 
@@ -272,7 +283,7 @@ def kv_move_groups(groups) -> None:
         n += 1
     if n == 0:
         return
-    rc = lib().abkv_kv_move_groups(C.byref(table), n, PAGE, PAGE_BYTES, HALF_BYTES, SLOT_BYTES, C.c_void_p(_stream()))
+    rc = lib().abkv_kv_move_groups(C.byref(table), n, PAGE, PAGE_BYTES, HALF_BYTES, SLOT_BYTES, _stream())
     check(rc, "abkv_kv_move_groups")
 
 
@@ -297,7 +308,7 @@ def kv_copy_staged(layer_caches, ops: torch.Tensor, stage: torch.Tensor | None =
     nbytes = stage.numel() * stage.element_size()
     _require(nbytes >= need, "stage buffer too small")
     rc = lib().abkv_kv_copy_staged(arr, len(layer_caches), num_pages, PAGE, PAGE_BYTES, HALF_BYTES, SLOT_BYTES, _ptr(ops), n,
-                                   _ptr(stage), nbytes, C.c_void_p(_stream()))
+                                   _ptr(stage), nbytes, _stream())
     check(rc, "abkv_kv_copy_staged")
 
 
@@ -306,16 +317,16 @@ def kv_append(key: torch.Tensor, value: torch.Tensor, slot_mapping: torch.Tensor
     _check_cache(kv_cache)
     T = slot_mapping.numel()
     for name, t in (("key", key), ("value", value)):
-        _require(t.is_cuda and t.dtype == torch.bfloat16 and t.shape[0] >= T
-                 and tuple(t.shape[1:]) == (HEADS_KV, HEAD_DIM) and t.stride(2) == 1 and t.stride(1) == HEAD_DIM,
-                 f"{name} must be cuda bf16 [T, {HEADS_KV}, {HEAD_DIM}] with contiguous rows")
+        if not (t.is_cuda and t.dtype == torch.bfloat16 and t.shape[0] >= T and t.shape[1:] == _KV_ROW
+                and t.stride(2) == 1 and t.stride(1) == HEAD_DIM):
+            raise ValueError(f"{name} must be cuda bf16 [T, {HEADS_KV}, {HEAD_DIM}] with contiguous rows")
     _require(slot_mapping.is_cuda and slot_mapping.dtype == torch.int64 and slot_mapping.is_contiguous(),
              "slot_mapping must be contiguous cuda int64")
     if T == 0:
         return
     rc = lib().abkv_kv_append(_ptr(key), key.stride(0) * 2, _ptr(value), value.stride(0) * 2, _ptr(slot_mapping), T,
                               _ptr(kv_cache), kv_cache.shape[0], PAGE_BYTES, HALF_BYTES, SLOT_BYTES, PAGE,
-                              C.c_void_p(_stream()))
+                              _stream())
     check(rc, "abkv_kv_append")
 
 
@@ -356,12 +367,12 @@ def rope_kv_append(q: torch.Tensor, key: torch.Tensor, value: torch.Tensor, posi
     retained tail). ``max_position``: a host bound on ``positions`` (None: read back from the device, which
     synchronises); the RoPE positions it implies must lie inside ``cos_sin`` (ValueError otherwise)."""
     T = positions.numel()
-    _require(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and tuple(q.shape[1:]) == (HEADS_Q, HEAD_DIM)
+    _require(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and q.shape[1:] == _Q_ROW
              and q.stride(2) == 1 and q.shape[0] >= T, "q must be cuda bf16 [T, 32, 128] with contiguous dims")
     for name, t in (("key", key), ("value", value)):
-        _require(t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 3 and t.shape[0] >= T
-                 and tuple(t.shape[1:]) == (HEADS_KV, HEAD_DIM) and t.stride(2) == 1 and t.stride(1) == HEAD_DIM,
-                 f"{name} must be cuda bf16 [T, 8, 128] with contiguous rows")
+        if not (t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 3 and t.shape[0] >= T
+                and t.shape[1:] == _KV_ROW and t.stride(2) == 1 and t.stride(1) == HEAD_DIM):
+            raise ValueError(f"{name} must be cuda bf16 [T, 8, 128] with contiguous rows")
     _require(positions.is_cuda and positions.dtype == torch.int64 and positions.is_contiguous(),
              "positions must be contiguous cuda int64")
     _require(cos_sin.is_cuda and cos_sin.dtype == torch.float32 and cos_sin.dim() == 2
@@ -380,13 +391,13 @@ def rope_kv_append(q: torch.Tensor, key: torch.Tensor, value: torch.Tensor, posi
         return
     if max_position is None:
         max_position = int(positions.max())
-    _require(rope_bound(max_position, block_c, codes_k) < cos_sin.shape[0],
-             f"RoPE positions up to {rope_bound(max_position, block_c, codes_k)} exceed the cos/sin table "
-             f"({cos_sin.shape[0]} rows)")
+    bound = rope_bound(max_position, block_c, codes_k)
+    if bound >= cos_sin.shape[0]:
+        raise ValueError(f"RoPE positions up to {bound} exceed the cos/sin table ({cos_sin.shape[0]} rows)")
     rc = lib().abkv_rope_kv_append(_ptr(q), q.stride(0), q.stride(1), _ptr(key), key.stride(0), _ptr(value),
                                    value.stride(0), _ptr(positions), T, int(block_c), int(codes_k),
                                    int(code_span), _ptr(cos_sin), cos_sin.shape[0], _ptr(slot_mapping),
-                                   _ptr(kv_cache), num_pages, C.c_void_p(_stream()))
+                                   _ptr(kv_cache), num_pages, _stream())
     check(rc, "abkv_rope_kv_append")
 
 
@@ -408,7 +419,7 @@ def slot_mapping(req_idx: torch.Tensor, positions: torch.Tensor, block_table: to
         out = torch.empty(n, dtype=torch.int64, device=positions.device)
     _require(req_idx.numel() == n, "req_idx and positions must have the same length")
     rc = lib().abkv_slot_mapping(_ptr(req_idx), _ptr(positions), n, _ptr(block_table), block_table.shape[0],
-                                 block_table.shape[1], PAGE, _ptr(compacted), _ptr(out), C.c_void_p(_stream()))
+                                 block_table.shape[1], PAGE, _ptr(compacted), _ptr(out), _stream())
     check(rc, "abkv_slot_mapping")
     return out
 
@@ -447,8 +458,9 @@ def prefill_masked_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     _require(S0 == num_blocks * (block_c + L * codes_k + R) + cr,
              "seq_len must be num_blocks * (block_c + L * codes_k + replay_rows) + copy_rows")
     for name, t, h in (("q", q, HEADS_Q), ("k", k, HEADS_KV), ("v", v, HEADS_KV)):
-        _require(t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 4 and tuple(t.shape) == (B, S0, h, HEAD_DIM)
-                 and t.stride(3) == 1, f"{name} must be cuda bf16 [B, S0, {h}, {HEAD_DIM}] with contiguous dims")
+        if not (t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 4 and t.shape == (B, S0, h, HEAD_DIM)
+                and t.stride(3) == 1):
+            raise ValueError(f"{name} must be cuda bf16 [B, S0, {h}, {HEAD_DIM}] with contiguous dims")
     if prompt_len is not None:
         _require(prompt_len.is_cuda and prompt_len.dtype == torch.int32 and prompt_len.numel() == B
                  and prompt_len.is_contiguous(), "prompt_len must be contiguous cuda int32 [B]")
@@ -468,7 +480,7 @@ def prefill_masked_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
                                         block_c, codes_k, num_blocks, S0, _ptr(prompt_len), _ptr(head_quota),
                                         int(retain_tail), policy, xattn, L, cr, R, rx, scale, _ptr(out),
                                         out.stride(0),
-                                        out.stride(1), out.stride(2), _ptr(lse), C.c_void_p(_stream()))
+                                        out.stride(1), out.stride(2), _ptr(lse), _stream())
     check(rc, "abkv_prefill_masked_attn")
     return out, lse
 
@@ -513,7 +525,7 @@ def prefill_masked_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch
              policy, xattn, L, cr, R, rx, scale]
     for t in (dq, dk, dv):
         args += [_ptr(t), t.stride(0), t.stride(1), t.stride(2)]
-    rc = lib().abkv_prefill_masked_attn_bwd(*args, _ptr(ws), ws.numel(), C.c_void_p(_stream()))
+    rc = lib().abkv_prefill_masked_attn_bwd(*args, _ptr(ws), ws.numel(), _stream())
     check(rc, "abkv_prefill_masked_attn_bwd")
     return dq, dk, dv
 
@@ -598,7 +610,7 @@ def _prefill_masked_f32(q, k, v, block_c, codes_k, num_blocks, prompt_len, head_
                                             retain_tail, policy, xattn, passes, copy_rows, replay_rows,
                                             replay_exclude, scale, _ptr(out),
                                             out.stride(0),
-                                            out.stride(1), out.stride(2), _ptr(lse), C.c_void_p(_stream()))
+                                            out.stride(1), out.stride(2), _ptr(lse), _stream())
     check(rc, "abkv_prefill_masked_attn_f32")
     return out, lse
 
@@ -619,19 +631,36 @@ def paged_split_plan(num_tiles: int, max_keys: int, target_blocks: int | None = 
     return -(-max_kt // split_tiles), split_tiles
 
 
+def _paged_plan_from(host: np.ndarray, B: int, num_cus: int):
+    """abkv_paged_plan over one int64 array [q_start (B + 1) | kv_start | kv_limit | causal]: (buffer, items, merges,
+    partial rows), the n items from element 0 of the buffer and the m merged tiles after ``cap`` items."""
+    cap = int(((host[1: B + 1] - host[:B] + 63) >> 6).sum()) + 3 * max(1, num_cus // HEADS_KV)
+    buf = np.empty(9 * cap + 3, np.int32)
+    at, h = buf.ctypes.data, host.ctypes.data
+    rc = lib().abkv_paged_plan(h, h + 8 * (B + 1), h + 8 * (2 * B + 1), h + 8 * (3 * B + 1), B, num_cus, at, cap,
+                               at + 20 * cap, cap, at + 36 * cap)
+    _require(rc == 0, "abkv_paged_plan failed")
+    n, m, rows = buf[9 * cap:].tolist()
+    return buf[: 5 * n], buf[5 * cap: 5 * cap + 4 * m], rows
+
+
 def paged_plan(q_start, kv_start, kv_limit, causal, num_cus: int | None = None):
     """Work items of a paged multi-query launch (abkv_paged_plan): (items int32 [n, 5], merged tiles int32 [m, 4],
-    partial rows) from int64 host arrays, for workgroups that end together on ``num_cus`` compute units."""
-    cus = _num_cus() if num_cus is None else int(num_cus)
-    qs, ks, kl, cz = (np.ascontiguousarray(x, dtype=np.int64) for x in (q_start, kv_start, kv_limit, causal))
-    cap = int((-(-np.diff(qs) // 64)).sum()) + 3 * max(1, cus // HEADS_KV)
-    buf = np.empty(9 * cap + 3, np.int32)
-    at = buf.ctypes.data
-    rc = lib().abkv_paged_plan(qs.ctypes.data, ks.ctypes.data, kl.ctypes.data, cz.ctypes.data, ks.size, cus, at, cap,
-                               at + 20 * cap, cap, at + 36 * cap)
-    _require(rc == 0, f"abkv_paged_plan failed ({rc})")
-    n, m, rows = buf[9 * cap:].tolist()
-    return buf[: 5 * n].reshape(n, 5), buf[5 * cap: 5 * cap + 4 * m].reshape(m, 4), rows
+    partial rows) from host sequences, for workgroups that end together on ``num_cus`` compute units."""
+    host = np.concatenate([np.asarray(x, dtype=np.int64) for x in (q_start, kv_start, kv_limit, causal)])
+    items, merges, rows = _paged_plan_from(host, len(kv_start), _num_cus() if num_cus is None else int(num_cus))
+    return items.reshape(-1, 5), merges.reshape(-1, 4), rows
+
+
+def _upload(parts, device) -> torch.Tensor:
+    """Host integer arrays as one int32 device tensor, by one asynchronous copy from pinned memory (torch's caching host
+    allocator keeps the block until the copy is done). A pageable copy waits for everything queued on the stream."""
+    n = sum(p.size for p in parts)
+    if torch.cuda.is_current_stream_capturing():             # a captured copy would re-read the block on every replay
+        return torch.from_numpy(np.concatenate(parts).astype(np.int32)).to(device)
+    staged = torch.empty(n, dtype=torch.int32, pin_memory=True)
+    np.concatenate(parts, out=staged.numpy(), casting="unsafe")
+    return staged.to(device, non_blocking=True)
 
 
 def _excluded_pairs(excluded, B):
@@ -662,11 +691,10 @@ def paged_prefill_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table
     physical positions kv_start[r] + i, seeing keys < kv_limit[r] (and <= their own position when causal).
     ``causal``: a bool for the whole batch or one flag per request (code steps and prompt chunks may share a batch).
     ``excluded``: None, or per request a physical (start, end) its queries must not see (None: nothing), e.g. the
-    code step's own-block retained tail. ``split``: key splits of every tile (None: chosen per tile by :func:`paged_plan`; 1: no split).
+    code step's own-block retained tail. ``split``: key splits of every tile (None: chosen per tile by
+    :func:`paged_plan`; 1: no split).
     Returns (out [T, 32, 128] bf16, lse [T, 32] fp32 or None). fp32 q and cache select the fp32 mode (out fp32).
     """
-    import numpy as np
-
     f32 = q.dtype == torch.float32
     dt = torch.float32 if f32 else torch.bfloat16
     _check_cache(kv_cache, dt)
@@ -680,79 +708,71 @@ def paged_prefill_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table
     B = ks.size
     W = block_table.shape[1]
     _require(qs.size == B + 1 and kl.size == B and B <= block_table.shape[0], "q_start [B+1], kv_start/kv_limit [B]")
-    _require(qs[0] == 0 and np.all(np.diff(qs) >= 0) and qs[-1] <= q.shape[0], "q_start must be a prefix sum <= T")
-    _require(np.all(kl >= 0) and np.all(kl <= W * PAGE), "kv_limit must lie in [0, block_table width * 16]")
-    _require(np.all(ks >= 0), "kv_start must be non-negative")
-    T = q.shape[0]
+    T, total = q.shape[0], int(qs[-1])
+    _require(qs[0] == 0 and total <= T and (B == 0 or (qs[1:] >= qs[:-1]).all()), "q_start must be a prefix sum <= T")
+    _require(B == 0 or (kl.min() >= 0 and kl.max() <= W * PAGE), "kv_limit must lie in [0, block_table width * 16]")
+    _require(B == 0 or ks.min() >= 0, "kv_start must be non-negative")
     if out is None:
         out = torch.empty((T, HEADS_Q, HEAD_DIM), dtype=dt, device=q.device)
-    _require(out.dtype == dt and tuple(out.shape) == (T, HEADS_Q, HEAD_DIM) and out.stride(2) == 1,
+    _require(out.dtype == dt and out.shape == (T, HEADS_Q, HEAD_DIM) and out.stride(2) == 1,
              "out must be [T, 32, 128] (dtype of q) with contiguous dims")
     if lse is not None:
         _require(lse.dtype == torch.float32 and lse.is_contiguous() and tuple(lse.shape) == (T, HEADS_Q),
                  "lse must be contiguous fp32 [T, 32]")
-    nq = np.diff(qs)
     exd = _excluded_pairs(excluded, B)
-    ex_t = None if exd is None else torch.from_numpy(exd.astype(np.int32).reshape(-1)).to(q.device)
-    if f32:
-        if qs[-1] == 0:
-            return out, lse
-        dev = q.device
-        cz = np.broadcast_to(np.asarray(causal, dtype=np.int64), (B,)).astype(np.int64)
-        tok_req = np.repeat(np.arange(B), nq)
-        meta = torch.from_numpy(np.concatenate([qs, ks, kl, cz, tok_req]).astype(np.int32)).to(dev)
-        o1, o2, o3, o4 = B + 1, 2 * B + 1, 3 * B + 1, 4 * B + 1
-        scale = default_scale() if scale is None else float(scale)
-        rc = lib().abkv_paged_prefill_attn_f32(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
-                                               _ptr(block_table), _row_stride(block_table), W, _ptr(meta[:o1]),
-                                               _ptr(meta[o1:o2]), _ptr(meta[o2:o3]), _ptr(ex_t), _ptr(meta[o4:]),
-                                               int(qs[-1]), _ptr(meta[o3:o4]), 1, scale, _ptr(out), out.stride(0),
-                                               out.stride(1), _ptr(lse), C.c_void_p(_stream()))
-        check(rc, "abkv_paged_prefill_attn_f32")
-        return out, lse
-    if qs[-1] == 0:
+    if total == 0:
         return out, lse
     dev = q.device
-    cz = np.broadcast_to(np.asarray(causal, dtype=np.int64), (B,)).astype(np.int64)
     scale = default_scale() if scale is None else float(scale)
+    host = np.empty(4 * B + 1, np.int64)                     # q_start | kv_start | kv_limit | causal
+    host[: B + 1], host[B + 1: 2 * B + 1], host[2 * B + 1: 3 * B + 1], host[3 * B + 1:] = qs, ks, kl, causal
+    o1, o2, o3, o4 = B + 1, 2 * B + 1, 3 * B + 1, 4 * B + 1
+    ex = [] if exd is None else [exd.reshape(-1)]
+    o5 = o4 + 2 * B * len(ex)                                # end of the excluded ranges
+    if f32:
+        meta = _upload([host, *ex, np.repeat(np.arange(B), np.diff(qs))], dev)
+        at = meta.data_ptr()
+        rc = lib().abkv_paged_prefill_attn_f32(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
+                                               _ptr(block_table), _row_stride(block_table), W, at, at + 4 * o1,
+                                               at + 4 * o2, at + 4 * o4 if ex else None, at + 4 * o5, total,
+                                               at + 4 * o3, 1, scale, _ptr(out), out.stride(0), out.stride(1),
+                                               _ptr(lse), _stream())
+        check(rc, "abkv_paged_prefill_attn_f32")
+        return out, lse
     if split is None:
-        items, merges, part_rows = paged_plan(qs, ks, kl, cz)
-        meta = torch.from_numpy(np.concatenate([qs, ks, kl, cz, items.reshape(-1), merges.reshape(-1)])
-                                .astype(np.int32)).to(dev)
-        o1, o2, o3, o4 = B + 1, 2 * B + 1, 3 * B + 1, 4 * B + 1
-        o5 = o4 + items.size
+        items, merges, part_rows = _paged_plan_from(host, B, _num_cus())
+        meta = _upload([host, *ex, items, merges], dev)
+        at = meta.data_ptr()
         ws, ws_bytes = None, 0
         if part_rows:
             ws_bytes = lib().abkv_paged_prefill_workspace_size(part_rows, 1)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         rc = lib().abkv_paged_prefill_attn_items(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
-                                                 _ptr(block_table), _row_stride(block_table), W, _ptr(meta[:o1]),
-                                                 _ptr(meta[o1:o2]), _ptr(meta[o2:o3]), _ptr(ex_t), _ptr(meta[o3:o4]),
-                                                 _ptr(meta[o4:o5]), len(items), _ptr(meta[o5:]), len(merges),
+                                                 _ptr(block_table), _row_stride(block_table), W, at, at + 4 * o1,
+                                                 at + 4 * o2, at + 4 * o4 if ex else None, at + 4 * o3, at + 4 * o5,
+                                                 items.size // 5, at + 4 * (o5 + items.size), merges.size // 4,
                                                  part_rows, scale, _ptr(out), out.stride(0), out.stride(1), _ptr(lse),
-                                                 _ptr(ws), ws_bytes, C.c_void_p(_stream()))
+                                                 _ptr(ws), ws_bytes, _stream())
         check(rc, "abkv_paged_prefill_attn_items")
         return out, lse
+    nq = np.diff(qs)
     tr = np.asarray([(r, q0) for r in range(B) for q0 in range(0, int(nq[r]), 64)], dtype=np.int32)
-    meta = torch.from_numpy(np.concatenate([qs, ks, kl, cz]).astype(np.int32)).to(dev)
-    tl = torch.from_numpy(np.ascontiguousarray(tr.T)).to(dev)
-    q_start_d, kv_start_d = meta[: B + 1], meta[B + 1: 2 * B + 1]
-    kv_limit_d, causal_d = meta[2 * B + 1: 3 * B + 1], meta[3 * B + 1:]
-    max_keys = int(kl.max()) if kl.size else 0
+    meta = _upload([host, *ex, np.ascontiguousarray(tr.T).reshape(-1)], dev)
+    at = meta.data_ptr()
+    max_keys = int(kl.max())
     n_splits = max(1, int(split))
     split_tiles = -(-(-(-max_keys // 64)) // n_splits) if n_splits > 1 else 0
     ws, ws_bytes = None, 0
-    covered = int(qs[-1])                    # rows the launch writes; rows past q_start[-1] stay untouched
+    covered = total                          # rows the launch writes; rows past q_start[-1] stay untouched
     if n_splits > 1:
         _require(n_splits * split_tiles * 64 >= max_keys, "key splits must cover every key")
         ws_bytes = lib().abkv_paged_prefill_workspace_size(covered, n_splits)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     rc = lib().abkv_paged_prefill_attn(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
-                                       _ptr(block_table), _row_stride(block_table), W, _ptr(q_start_d),
-                                       _ptr(kv_start_d), _ptr(kv_limit_d), _ptr(ex_t), _ptr(tl[0]), _ptr(tl[1]),
-                                       len(tr),
-                                       _ptr(causal_d), 1, scale, _ptr(out), out.stride(0), out.stride(1), _ptr(lse),
-                                       covered, n_splits, split_tiles, _ptr(ws), ws_bytes, C.c_void_p(_stream()))
+                                       _ptr(block_table), _row_stride(block_table), W, at, at + 4 * o1, at + 4 * o2,
+                                       at + 4 * o4 if ex else None, at + 4 * o5, at + 4 * (o5 + len(tr)), len(tr),
+                                       at + 4 * o3, 1, scale, _ptr(out), out.stride(0), out.stride(1), _ptr(lse),
+                                       covered, n_splits, split_tiles, _ptr(ws), ws_bytes, _stream())
     check(rc, "abkv_paged_prefill_attn")
     return out, lse
 
@@ -812,7 +832,7 @@ def packed_capture(layer_caches, layer_pools, layer_rows: torch.Tensor, layer_qu
     rc = lib().abkv_packed_capture(_ptr(ptrs[:L]), _ptr(ptrs[L:]), _ptr(layer_rows), _ptr(layer_quota), L,
                                    layer_caches[0].shape[0], layer_pools[0].shape[0], _ptr(block_table),
                                    _row_stride(block_table), block_table.shape[1], _ptr(code_start), _ptr(dst_page),
-                                   n, C.c_void_p(_stream()))
+                                   n, _stream())
     check(rc, "abkv_packed_capture")
 
 
@@ -865,7 +885,7 @@ def decode_attention_packed(q: torch.Tensor, kv_cache: torch.Tensor, block_table
                                        split_pages, _ptr(packed_pool), packed_pool.shape[0], rows, hq_c,
                                        _ptr(packed_table), _row_stride(packed_table), _ptr(packed_count), max_packed,
                                        sr, float(scale), _ptr(out), out.stride(0), out.stride(1), _ptr(lse),
-                                       _ptr(workspace), ws_bytes, C.c_void_p(_stream()))
+                                       _ptr(workspace), ws_bytes, _stream())
     check(rc, "abkv_decode_attn_packed")
     return out, lse
 
@@ -946,7 +966,7 @@ def paged_prefill_attention_packed(q: torch.Tensor, kv_cache: torch.Tensor, bloc
         _ptr(tl[1]), len(tiles), _ptr(meta[o3:o4]), 1, _ptr(head_quota_dev), _ptr(packed_pool), packed_pool.shape[0], rows, hq_c,
         _ptr(packed_table), _row_stride(packed_table), _ptr(packed_count), max_packed, scale, _ptr(out),
         out.stride(0), out.stride(1), _ptr(lse), covered, n_splits, split_tiles, side_splits, side_split_tiles, _ptr(ws),
-        ws_bytes, C.c_void_p(_stream()))
+        ws_bytes, _stream())
     check(rc, "abkv_paged_prefill_attn_packed")
     return out, lse
 

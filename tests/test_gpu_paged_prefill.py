@@ -191,3 +191,37 @@ def test_planned_items_match_the_oracle(num_cus, monkeypatch):
         ro, rl = _oracle(q[a:z].float().numpy(), cf, tables[r], past[r], limits[r], causal[r])
         assert np.abs(out[a:z] - ro).max() <= TOL
         assert np.abs(lse[a:z] - rl).max() <= TOL
+
+
+@pytest.mark.parametrize("split", [None, 2])
+def test_calls_queued_behind_work_keep_their_own_metadata(split):
+    """Calls issued while the GPU is busy, on two streams: each call's lengths and work items are uploaded from staging
+    memory of their own, so every result equals the call made alone."""
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    cache, tables = _setup([1500], 100, 30)
+    cache, bt = cache.to(dev), torch.from_numpy(tables).to(dev)
+    q = torch.randn((64, 32, 128), generator=torch.Generator().manual_seed(31)).to(torch.bfloat16).to(dev)
+    limits = [1400 - 61 * i for i in range(20)]
+
+    def call(limit):
+        return ops.paged_prefill_attention(q, cache, bt, [0, 64], [limit - 32], [limit], False, split=split)[0]
+
+    alone = []
+    for n in limits:
+        alone.append(call(n))
+        torch.cuda.synchronize()
+    big = torch.randn((8192, 8192), device=dev, dtype=torch.bfloat16)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for s in streams:
+        with torch.cuda.stream(s):
+            for _ in range(4):
+                big @ big
+    got = []
+    for i, n in enumerate(limits):
+        with torch.cuda.stream(streams[i % 2]):
+            got.append(call(n))
+    torch.cuda.synchronize()
+    for a, b in zip(alone, got):
+        assert torch.equal(a, b)
