@@ -4,7 +4,7 @@
 // keys, values and outputs, fp32 accumulation in a fixed order and accurate expf/logf: the mode the reference's
 // PyTorch paths run in fp32 (abridgekv/gen_compress.py:359-360, 555; compresslm_packed_kv.py:608-613;
 // compress_forward.py:695-727 under FlexAttention) for tight parity checks. Every product is a fp32 matrix instruction
-// (v_mfma_f32_16x16x4_f32: fp32 inputs, fp32 sums). Masked B=1, 3 x (512 + 128) rows, 200 raw prompt rows: 1546 -> 228 us
+// (v_mfma_f32_16x16x4_f32: fp32 inputs, fp32 sums). Masked B=1, 3 x (512 + 128) rows, 200 raw prompt rows: 1546 -> 203 us
 // a call against one wave per (token, KV head) of VALU dot products with the mask's predicate per key.
 #include <cstring>
 
@@ -63,8 +63,6 @@ __device__ __forceinline__ floatx4 mfma16x16x4(float a, float b, const floatx4& 
 }
 
 constexpr int kF32Rows = 16;             // query rows of a workgroup (MFMA columns of each of its waves)
-constexpr int kF32Keys = 32;             // keys per LDS stage
-constexpr int kF32StageElems = kF32Keys * kHeadDim;
 constexpr float kF32Headroom = 8.f;      // the running max moves only when a score exceeds it by more (p <= e^8)
 
 // Scores of 16 keys x 16 columns: s[r] = q(column m16) . k(key 4g + r). The operands' contraction order is dim
@@ -126,11 +124,12 @@ struct F32Span {
   unsigned len;
 };
 struct F32Stage {
-  int k0, end;             // keys [k0, min(k0 + 32, end)); rows at or past end are replaced by row end - 1 (weight 0)
+  int k0, end;             // keys k0 .. end - 1 (one stage); rows at or past end are replaced by row end - 1 (weight 0)
   F32Span span;
 };
 
-// Stages of the compression mask: SegWalk's 64-key tiles, each in up to two stages.
+// Stages of kKeys keys of the compression mask: SegWalk's 64-key tiles cut up.
+template <int kKeys>
 struct MaskedStages {
   const float* k;
   const float* v;
@@ -154,9 +153,9 @@ struct MaskedStages {
         span.len = (unsigned)imax(tm.limit[1] - lo, 0);
       }
     }
-    st = F32Stage{k0, min(k0 + kF32Keys, k0 + left), span};
-    k0 += kF32Keys;
-    left -= kF32Keys;
+    st = F32Stage{k0, min(k0 + kKeys, k0 + left), span};
+    k0 += kKeys;
+    left -= kKeys;
     return true;
   }
   // K and V rows of half h (rows 16h .. 16h + 15) of a stage
@@ -171,7 +170,8 @@ struct MaskedStages {
   __device__ __forceinline__ static int row_of(const F32Stage& st, int row) { return min(row, st.end - 1 - st.k0); }
 };
 
-// Stages of one request's paged keys [0, n_keys) (the largest limit of the rows), with an excluded range.
+// Stages of kKeys keys of one request's paged keys [0, n_keys) (the largest limit of the rows), with an excluded range.
+template <int kKeys>
 struct PagedStages {
   const float* kv;         // cache base + head * 128
   const int32_t* table;
@@ -179,8 +179,8 @@ struct PagedStages {
   F32Span span;
   __device__ __forceinline__ bool next(F32Stage& st) {
     if (k0 >= n_keys) return false;
-    st = F32Stage{k0, min(k0 + kF32Keys, n_keys), span};
-    k0 += kF32Keys;
+    st = F32Stage{k0, min(k0 + kKeys, n_keys), span};
+    k0 += kKeys;
     return true;
   }
   struct Half {
@@ -202,15 +202,16 @@ struct PagedStages {
 // One wave's head over the stages: 16 query rows against K and V stages that the four waves of the workgroup load
 // together. The next stage's rows are on their way (in registers) while this one is multiplied. Row r's 16-byte chunk
 // c lies at chunk c ^ (r & 15), so both read patterns hit all banks.
-template <class Stages>
+template <int kKeys, class Stages>
 __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx4 (&q)[8], float scale, float& m,
                                            float& l, floatx4 (&o)[8]) {
   const int tid = threadIdx.x, lane = tid & 63, m16 = lane & 15, g = lane >> 4;
   const int r0 = tid >> 5, chunk = tid & 31;
-  floatx4 kr[4], vr[4];
+  constexpr int kHalves = kKeys / 16, kStageElems = kKeys * kHeadDim;
+  floatx4 kr[2 * kHalves], vr[2 * kHalves];
   auto load = [&](const F32Stage& st) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kHalves; ++h) {
       const auto base = src.half(st, h);
 #pragma unroll
       for (int i = 2 * h; i < 2 * h + 2; ++i) {
@@ -221,10 +222,10 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
     }
   };
   auto store = [&](int n) {                                  // buffer n: K rows, then V rows
-    float* kb = lds + 2 * n * kF32StageElems;
-    float* vb = kb + kF32StageElems;
+    float* kb = lds + 2 * n * kStageElems;
+    float* vb = kb + kStageElems;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 2 * kHalves; ++i) {
       const int row = 8 * i + r0, at = row * kHeadDim + 4 * (chunk ^ (row & 15));
       *reinterpret_cast<floatx4*>(kb + at) = kr[i];
       *reinterpret_cast<floatx4*>(vb + at) = vr[i];
@@ -238,11 +239,11 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
   for (int n = 0;; n ^= 1) {
     const bool more = src.next(nxt);
     if (more) load(nxt);
-    const float* kb = lds + 2 * n * kF32StageElems;
-    const float* vb = kb + kF32StageElems;
-    floatx4 t[2];
+    const float* kb = lds + 2 * n * kStageElems;
+    const float* vb = kb + kStageElems;
+    floatx4 t[kHalves];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < kHalves; ++i) {
       floatx4 kx[8];
 #pragma unroll
       for (int c = 0; c < 8; ++c)
@@ -257,7 +258,7 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
     }
     f32_softmax(t, m, l, o);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < kHalves; ++i) {
       floatx4 va[4], vb4[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -298,10 +299,10 @@ __device__ __forceinline__ float f32_lse(float m, float l) {
 // Multi-query attention, masked (kMasked) or paged: a workgroup of 4 waves takes 16 query rows of one KV head, one query
 // head per wave. Bound by the fp32 matrix rate (16x16x4: 256 flop per clock and CU). Matrix instructions, LDS stages
 // shared by the four heads and the segment walk instead of VALU dot products per key with the mask's predicate per
-// element: masked, B=1, 3 x (512 + 128) rows 1546 -> 228 us; a code step of 256 rows over 4000 keys 2059 -> 455 us.
-template <bool kMasked>
+// element: masked, B=1, 3 x (512 + 128) rows 1546 -> 203 us; a code step of 256 rows over 4000 keys 2059 -> 412 us.
+template <bool kMasked, int kKeys>
 __global__ __launch_bounds__(256, 2) void attn_f32_rows_kernel(F32Args a) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * kF32StageElems];
+  __shared__ __attribute__((aligned(16))) float lds[4 * kKeys * kHeadDim];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
   const int kvh = blockIdx.x % kHeadsKV;
@@ -329,11 +330,11 @@ __global__ __launch_bounds__(256, 2) void attn_f32_rows_kernel(F32Args a) {
                           a.tail_policy, a.pause_xattn, a.replay_exclude != 0};
     f32_load_q(a.q + (long)b * a.q_sb + (long)min(qrow, a.seq_len - 1) * a.q_st + (long)head * a.q_sh, g,
                qrow < a.seq_len, q);
-    MaskedStages src{a.k + (long)b * a.k_sb + (long)kvh * a.k_sh, a.v + (long)b * a.v_sb + (long)kvh * a.v_sh,
+    MaskedStages<kKeys> src{a.k + (long)b * a.k_sb + (long)kvh * a.k_sh, a.v + (long)b * a.v_sb + (long)kvh * a.v_sh,
                      a.k_ss, a.v_ss,
                      SegWalk(g_, q0, min(q0 + kF32Rows, a.seq_len) - 1, plen, qmin, qmax, quota, quota), g_,
                      row_facts(g_, qrow), plen, quota, 0};
-    f32_attend(src, lds, q, a.scale, m, l, o);
+    f32_attend<kKeys>(src, lds, q, a.scale, m, l, o);
     if (qrow >= a.seq_len) return;
     f32_store(a.out + (long)b * a.o_sb + (long)qrow * a.o_st + (long)head * a.o_sh, g, l, o);
     if (a.lse != nullptr && g == 0) a.lse[((long)b * kHeadsQ + head) * a.seq_len + qrow] = f32_lse(m, l);
@@ -358,9 +359,9 @@ __global__ __launch_bounds__(256, 2) void attn_f32_rows_kernel(F32Args a) {
         if (lo < hi) span = F32Span{min(lane_limit, lo), hi, (unsigned)max(lane_limit - hi, 0)};
       }
       f32_load_q(a.q + (long)min(row, t1 - 1) * a.q_st + (long)head * a.q_sh, g, row < t1, q);
-      PagedStages src{a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages,
+      PagedStages<kKeys> src{a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages,
                       causal ? min(limit, pos + n) : limit, 0, span};
-      f32_attend(src, lds, q, a.scale, m, l, o);
+      f32_attend<kKeys>(src, lds, q, a.scale, m, l, o);
       if (row < t1) {
         f32_store(a.out + (long)row * a.o_st + (long)head * a.o_sh, g, l, o);
         if (a.lse != nullptr && g == 0) a.lse[(long)row * kHeadsQ + head] = f32_lse(m, l);
@@ -536,7 +537,7 @@ int abkv_paged_prefill_attn_f32(const float* q, long q_stride_t, long q_stride_h
   a.lse = lse;
   const unsigned grid = f32_grid(((long)num_tokens + kF32Rows - 1) / kF32Rows);
   if (grid == 0) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(attn_f32_rows_kernel<false>, dim3(grid), dim3(256), 0, stream, a);
+  hipLaunchKernelGGL((attn_f32_rows_kernel<false, 32>), dim3(grid), dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -594,7 +595,11 @@ int abkv_prefill_masked_attn_f32(const float* q, long q_sb, long q_ss, long q_sh
   a.lse = lse;
   const unsigned grid = f32_grid(((long)seq_len + kF32Rows - 1) / kF32Rows * batch);
   if (grid == 0) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(attn_f32_rows_kernel<true>, dim3(grid), dim3(256), 0, stream, a);
+  // Stages of 16 keys (three workgroups a CU) where blocks have codes: segments are short, their last stage partly empty;
+  // of 32 (two, half the barriers) for one long causal walk. 16 / 32: 3 x (512 + 128) rows 218 / 242 us, 6 x (200 + 2 x 40)
+  // 175 / 217; causal 1337 rows 214 / 191, and a paged code step over 4000 keys 439 / 412.
+  if (codes_k > 0) hipLaunchKernelGGL((attn_f32_rows_kernel<true, 16>), dim3(grid), dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((attn_f32_rows_kernel<true, 32>), dim3(grid), dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 
