@@ -430,7 +430,7 @@ def bench_compaction(args, torch):
 
 def same_pattern_probe(torch, prepared, by_group, num_pages, args):
     """Ceiling of the mover's access pattern: abkv_probe_row_copy (libabridgekv_probes.so) copies the same rows of the
-    same layers -- every (src page, slot) -> (dst page, slot) of each group launch, 4 KiB each -- into a second set of
+    same layers -- every (src page, slot) -> (dst page, slot) of each group, 4 KiB each -- into a second set of
     caches, all ops in parallel (no segment order to keep). Swept over 4, 8 and 16 rows per workgroup; the best is
     the ceiling. Returns its GB/s (read + write bytes / time of the same launches) and the sweep."""
     import ctypes as C
