@@ -56,6 +56,7 @@ SIGNATURES = {
     "abkv_paged_prefill_attn_items": (C.c_int, [_vp, C.c_long, C.c_long, _vp, C.c_int, _vp, C.c_long, C.c_int, _vp,
                                                 _vp, _vp, _vp, _vp, _vp, C.c_int, _vp, C.c_int, C.c_int, C.c_float,
                                                 _vp, C.c_long, C.c_long, _vp, _vp, C.c_size_t, _vp]),
+    "abkv_paged_prefill_items_workspace_size": (C.c_size_t, [C.c_int]),
     "abkv_paged_prefill_workspace_size": (C.c_size_t, [C.c_int, C.c_int]),
     "abkv_paged_prefill_attn": (C.c_int, [_vp, C.c_long, C.c_long, _vp, C.c_int, _vp, C.c_long, C.c_int, _vp, _vp,
                                           _vp, _vp, _vp, _vp, C.c_int, _vp, C.c_int, C.c_float, _vp, C.c_long,

@@ -34,9 +34,12 @@ struct PagedPrefillArgs {
   int num_tiles;                               // uniform: query tiles; the grid is 8 x num_tiles x splits
   int split_tiles;                             // uniform: > 0: key tiles per split, partials to part_*
   int num_tokens;
+  // uniform splits, rows = splits x T:
   _Float16* part_o;                            // [rows, 32, 128] split output / (l * scale), fp16
-  float* part_ml;                              // [rows, 32, 4] (max in log2 units, weight sum l, scale, unused);
-                                               // uniform: rows = splits x T
+  float* part_ml;                              // [rows, 32, 4] (max in log2 units, weight sum l, scale, unused)
+  // work items:
+  float* item_o;                               // [parts][kItemFloats] weighted sums, fp32, as the lanes hold them
+  float* item_ml;                              // [parts, 8 heads, 8 waves, 2, 16 rows, 2] (max in log2 units, weight sum)
   int split_base;                              // first partial slot of this launch's splits
   const int32_t* head_quota;                   // [8] or nullptr: a non-causal request sees keys < kv_start + q_h
   // side rows (per-head packed code pages, attended by every query of the request); see PackedRows
@@ -58,6 +61,9 @@ __device__ __forceinline__ void store_acc_f16x8(_Float16* dst, const floatx4& a,
   }
   *reinterpret_cast<f16x8*>(dst) = h;
 }
+
+// Sums of a work item's KV heads: [8 heads][8 waves][head u of the wave][accumulator tile t][lane] x 4.
+constexpr int kItemFloats = kBM * kHeadsQ * kHeadDim;
 
 constexpr int kMaxSideTable = 2048;             // packed pages per request the side launch stages in LDS
 
@@ -212,10 +218,26 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
                             w, lane);
   }
 
-  // Split partials: the split's output normalised by its weight sum l, in fp16 (half the bytes the epilogue writes
-  // and the merge reads), divided by a scale that keeps every value within +-32768 (1 unless the split's V rows
-  // exceed that), and the record (m, l, scale). The scale needs the row's largest |o| over its 128 dims, which lie in
-  // the row's four lane groups (lanes m16 + 16j): reduced before any lane leaves.
+  // Partials of work items: the sums as they are, in fp32 (the plan splits tiles on its own account, also those that one
+  // workgroup could walk with its sums in registers, so no caller loses precision to it), in lane order: whole 1 KiB
+  // runs, which the merge reads the same way. Rows past the request's last are written too, and never read. One code
+  // step of 256 rows over 5200 keys, a call: 46.2 us; fp32 in rows of 128 dims 53.0; normalised fp16 in rows 46.5.
+  if (part_row >= 0 && a.items != nullptr) {
+    const long at = (part_row / kBM * kHeadsKV + kvh) * kWaves + w;
+    float* po = a.item_o + at * (kItemFloats / kHeadsKV / kWaves) + 4 * lane;
+#pragma unroll
+    for (int u = 0; u < H; ++u) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) *reinterpret_cast<floatx4*>(po + 256 * (8 * u + t)) = o[t][u];
+      if (j == 0)
+        *reinterpret_cast<float2*>(a.item_ml + ((at * H + u) * 16 + m16) * 2) = make_float2(m_run[u], l_run[u]);
+    }
+    return;
+  }
+  // Partials of uniform splits, which the caller asks for: the split's output normalised by its weight sum l, in fp16
+  // (half the bytes the epilogue writes and the merge reads), divided by a scale that keeps every value within +-32768
+  // (1 unless the split's V rows exceed that), and the record (m, l, scale). The scale needs the row's largest |o| over
+  // its 128 dims, which lie in the row's four lane groups (lanes m16 + 16j): reduced before any lane leaves.
   float amax[H];
   if (part_row >= 0) {
 #pragma unroll
@@ -258,25 +280,56 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
   }
 }
 
-// Combine the key-split partials of a query token: workgroup (token, group of 8 heads); thread t handles head
-// 8 * blockIdx.y + t / 32 and dims 4 * (t % 32) .. +4. Uniform splits: blockIdx.x is the token; work items: row
-// blockIdx.x % 64 of merged tile blockIdx.x / 64, whose splits' partials lie 64 rows apart.
+// Combine the parts of a merged tile: workgroup (tile, KV head, wave w of the attention kernel), its waves (head u of the
+// two, accumulator tiles 4 * half .. + 3) in the attention kernel's lane order, so every load is a whole 1 KiB run.
+__global__ __launch_bounds__(256) void paged_merge_items_kernel(PagedPrefillArgs a) {
+  constexpr int H = 2, kWaves = 8, kLaneRuns = kItemFloats / kHeadsKV / kWaves;
+  const int w = blockIdx.x % kWaves, kvh = blockIdx.x / kWaves % kHeadsKV;
+  const int32_t* mt = a.merges + 4 * (blockIdx.x / (kWaves * kHeadsKV));
+  const int parts = mt[3];
+  const int lane = threadIdx.x & 63, m16 = lane & 15, j = lane >> 4;
+  const int u = (threadIdx.x >> 6) & 1, half = threadIdx.x >> 7;
+  const int row = 16 * (w >> 1) + m16;                       // within the tile
+  const long first = (mt[2] / kBM * (long)kHeadsKV + kvh) * kWaves + w;
+  constexpr long kStep = kHeadsKV * kWaves;                  // between the parts
+  const float2* ml = reinterpret_cast<const float2*>(a.item_ml) + (first * H + u) * 16 + m16;
+  const float* po = a.item_o + first * kLaneRuns + 256 * (8 * u + 4 * half) + 4 * lane;
+  float M = -INFINITY;
+#pragma unroll 8
+  for (int s = 0; s < parts; ++s) M = fmaxf(M, ml[s * kStep * H * 16].x);
+  float L = 0.f;
+  floatx4 acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < parts; ++s) {
+    const float2 rec = ml[s * kStep * H * 16];               // m, l
+    const float f = rec.x == M ? 1.f : fast_exp2(rec.x - M); // (m and M are both -inf without a finite score: sums of 0,
+    L += f * rec.y;                                          // or of NaN scores, which go through)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      acc[t] += *reinterpret_cast<const floatx4*>(po + s * kStep * kLaneRuns + 256 * t) * f;
+  }
+  if (row >= mt[1]) return;
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const long tok = (long)mt[0] + row;
+  const int head = kvh * kGroup + H * (w & 1) + u;
+  __bf16* oh = a.out + tok * a.o_st + (long)head * a.o_sh + 32 * j + 16 * half;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) store_acc_bf16x8(oh + 8 * p, acc[2 * p], acc[2 * p + 1], j, inv);
+  if (a.lse != nullptr && j == 0 && half == 0)
+    a.lse[tok * kHeadsQ + head] = L > 0.f ? (M + __log2f(L)) * 0.69314718055994531f : -INFINITY;
+}
+
+// Combine the key-split partials of a query token (uniform splits): workgroup (token, group of 8 heads); thread t handles
+// head 8 * blockIdx.y + t / 32 and dims 4 * (t % 32) .. +4.
 __global__ __launch_bounds__(256) void paged_merge_kernel(PagedPrefillArgs a, int n_splits) {
   typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-  long tok = blockIdx.x, first = tok, step = a.num_tokens;   // partial rows of the token: first, first + step, ...
-  if (a.merges != nullptr) {
-    const int32_t* mt = a.merges + 4 * (blockIdx.x / kBM);
-    const int row = blockIdx.x % kBM;
-    if (row >= mt[1]) return;
-    tok = mt[0] + row;
-    first = (long)mt[2] + row;
-    step = kBM;
-    n_splits = mt[3];
-  }
+  const long tok = blockIdx.x;
   const int head = 8 * blockIdx.y + (threadIdx.x >> 5);
   const int d0 = (threadIdx.x & 31) * 4;
-  const long stride = step * kHeadsQ;                        // partial rows x heads per split
-  const float* pml = a.part_ml + (first * kHeadsQ + head) * 4;
+  const long stride = (long)a.num_tokens * kHeadsQ;          // partial rows x heads per split
+  const float* pml = a.part_ml + (tok * kHeadsQ + head) * 4;
   float M = -INFINITY;
 #pragma unroll 8
   for (int s = 0; s < n_splits; ++s) M = fmaxf(M, pml[s * stride * 4]);
@@ -289,7 +342,7 @@ __global__ __launch_bounds__(256) void paged_merge_kernel(PagedPrefillArgs a, in
       const float w = fast_exp2(rec[0] - M) * rec[1];      // the split's weight (0 for a split that saw no key)
       const float ws = w * rec[2];
       L += w;
-      const f16x4 h = *reinterpret_cast<const f16x4*>(a.part_o + ((s * stride) + first * kHeadsQ + head) * kHeadDim + d0);
+      const f16x4 h = *reinterpret_cast<const f16x4*>(a.part_o + ((s * stride) + tok * kHeadsQ + head) * kHeadDim + d0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[r] += ws * (float)h[r];
     }
@@ -322,6 +375,9 @@ size_t abkv_paged_prefill_workspace_size(int num_tokens, int num_splits) {
          (abkv::kHeadDim * sizeof(_Float16) + 4 * sizeof(float));
 }
 
+size_t abkv_paged_prefill_items_workspace_size(int part_rows) {
+  return (size_t)(part_rows > 0 ? part_rows : 0) * abkv::kHeadsQ * (abkv::kHeadDim + 2) * sizeof(float);
+}
 
 int abkv_paged_prefill_attn(const void* q, long q_stride_t, long q_stride_h, const void* kv_cache, int num_pages,
                             const int32_t* block_table, long block_table_stride, int block_table_width,
@@ -363,6 +419,7 @@ int abkv_paged_prefill_attn(const void* q, long q_stride_t, long q_stride_h, con
   a.num_tokens = num_tokens;
   a.split_tiles = 0;
   a.items = a.merges = nullptr;
+  a.item_o = a.item_ml = nullptr;
   a.part_o = nullptr;
   a.part_ml = nullptr;
   a.split_base = 0;
@@ -398,8 +455,8 @@ int abkv_paged_prefill_attn_items(const void* q, long q_stride_t, long q_stride_
   if (q == nullptr || kv_cache == nullptr || block_table == nullptr || q_start == nullptr || kv_start == nullptr ||
       kv_limit == nullptr || causal == nullptr || items == nullptr || out == nullptr || num_pages <= 0 ||
       block_table_width <= 0 || n_merges < 0 || part_rows < 0 || (n_merges > 0 && merges == nullptr) ||
-      (part_rows > 0 && (workspace == nullptr || workspace_bytes < abkv_paged_prefill_workspace_size(part_rows, 1))) ||
-      (long)n_merges * kBM * 256 > 0xFFFFFFFFL)
+      (part_rows > 0 && (workspace == nullptr || workspace_bytes < abkv_paged_prefill_items_workspace_size(part_rows))) ||
+      part_rows % kBM != 0 || (long)n_merges * 8 * kHeadsKV * 256 > 0xFFFFFFFFL)
     return (int)hipErrorInvalidValue;
   PagedPrefillArgs a;
   a.q = static_cast<const __bf16*>(q);
@@ -427,8 +484,10 @@ int abkv_paged_prefill_attn_items(const void* q, long q_stride_t, long q_stride_
   a.num_tiles = 0;
   a.split_tiles = 0;
   a.num_tokens = 0;
-  a.part_o = static_cast<_Float16*>(workspace);
-  a.part_ml = reinterpret_cast<float*>(a.part_o + (size_t)part_rows * kHeadsQ * kHeadDim);
+  a.part_o = nullptr;
+  a.part_ml = nullptr;
+  a.item_o = static_cast<float*>(workspace);
+  a.item_ml = a.item_o + (size_t)part_rows * kHeadsQ * kHeadDim;
   a.split_base = 0;
   a.head_quota = nullptr;
   a.side_count = nullptr;
@@ -437,7 +496,7 @@ int abkv_paged_prefill_attn_items(const void* q, long q_stride_t, long q_stride_
   hipLaunchKernelGGL(paged_prefill_kernel<false>, dim3(grid), dim3(512), 0, stream, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || n_merges == 0) return (int)err;
-  hipLaunchKernelGGL(paged_merge_kernel, dim3((unsigned)n_merges * kBM, kHeadsQ / 8), dim3(256), 0, stream, a, 0);
+  hipLaunchKernelGGL(paged_merge_items_kernel, dim3((unsigned)n_merges * 8 * kHeadsKV), dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -501,6 +560,7 @@ int abkv_paged_prefill_attn_packed(const void* q, long q_stride_t, long q_stride
   a.lse = lse;
   a.num_tokens = num_tokens;
   a.items = a.merges = nullptr;
+  a.item_o = a.item_ml = nullptr;
   a.part_o = static_cast<_Float16*>(workspace);
   a.part_ml = reinterpret_cast<float*>(a.part_o + (size_t)total * num_tokens * kHeadsQ * kHeadDim);
   a.head_quota = head_quota_dev;

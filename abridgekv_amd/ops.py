@@ -745,7 +745,7 @@ def paged_prefill_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table
         at = meta.data_ptr()
         ws, ws_bytes = None, 0
         if part_rows:
-            ws_bytes = lib().abkv_paged_prefill_workspace_size(part_rows, 1)
+            ws_bytes = lib().abkv_paged_prefill_items_workspace_size(part_rows)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         rc = lib().abkv_paged_prefill_attn_items(_ptr(q), q.stride(0), q.stride(1), _ptr(kv_cache), kv_cache.shape[0],
                                                  _ptr(block_table), _row_stride(block_table), W, at, at + 4 * o1,

@@ -225,3 +225,40 @@ def test_calls_queued_behind_work_keep_their_own_metadata(split):
     torch.cuda.synchronize()
     for a, b in zip(alone, got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("shift", [-24, 40])
+def test_planned_parts_keep_small_and_large_values(shift):
+    """A batch whose long tiles the plan splits: V times 2^shift gives the output times 2^shift, bit for bit. Every step
+    from V to the bf16 output is linear in V, and a power of two is exact in bf16 and in fp32 down to 2^-126; in fp16
+    partials the outputs (about 0.02) times 2^-24 would be subnormal."""
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    rows = [5000, 700, 300]
+    cache, tables = _setup(rows, 500, 40)
+    q_start, start, limit, causal = [0, 256, 456, 457], [4700, 500, 299], [4828, 700, 300], [False, True, True]
+    assert ops.paged_plan(q_start, start, limit, causal, 256)[2] > 0
+    q = torch.randn((457, 32, 128), generator=torch.Generator().manual_seed(41)).to(torch.bfloat16)
+    small = cache.clone()
+    small[:, 1] = (cache[:, 1].float() * 2.0 ** shift).to(torch.bfloat16)
+    out, lse = _run(cache, tables, q, q_start, start, limit, causal)
+    out_s, lse_s = _run(small, tables, q, q_start, start, limit, causal)
+    assert np.array_equal(out_s, out * np.float32(2.0 ** shift))
+    assert np.array_equal(lse_s, lse)
+
+
+def test_planned_parts_pass_nan_queries_on():
+    """A NaN in one row's query: its output is NaN in the heads it touches, as from a tile that is not split, and no
+    other row changes."""
+    from abridgekv_amd import ops
+    cache, tables = _setup([5000], 400, 42)
+    args = ([0, 256], [4700], [4828], False)
+    assert ops.paged_plan(args[0], args[1], args[2], [False], 256)[2] > 0
+    q = torch.randn((256, 32, 128), generator=torch.Generator().manual_seed(43)).to(torch.bfloat16)
+    bad = q.clone()
+    bad[77, 5, 3] = float("nan")
+    out, _ = _run(cache, tables, q, *args)
+    got, _ = _run(cache, tables, bad, *args)
+    assert np.isnan(got[77, 5]).all()
+    got[77, 5] = out[77, 5]
+    assert np.array_equal(got, out)
