@@ -23,6 +23,17 @@ constexpr int kSlotElems = kHeadsKV * kHeadDim;            // 1024 elements = 2 
 constexpr int kHalfElems = kPage * kSlotElems;             // 16384 elements = 32 KiB (K half of a page)
 constexpr int kPageElems = 2 * kHalfElems;                 // 32768 elements = 64 KiB
 
+// Power of two `scale` that brings x (>= 0) into [2^14, 2^15), the top of fp16's range, and its reciprocal: fp16 partials
+// keep 11 bits of every value down to 2^-28 of the largest, wherever that lies. (x under 2^-86 keeps the scale of 2^-86.)
+struct F16Range {
+  float scale, inv;
+  __device__ __forceinline__ explicit F16Range(float x) {
+    const int e = max((int)(__builtin_bit_cast(uint32_t, x) >> 23) - 14, 27);
+    scale = __builtin_bit_cast(float, (uint32_t)e << 23);
+    inv = __builtin_bit_cast(float, (uint32_t)(254 - e) << 23);
+  }
+};
+
 __device__ __forceinline__ floatx4 mfma16x16x32(const bf16x8 a, const bf16x8 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }

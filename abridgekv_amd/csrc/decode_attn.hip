@@ -88,15 +88,13 @@ __device__ __forceinline__ float column_absmax(const floatx4 (&o)[8]) {
 }
 
 // Split partial of one query head: the split's output normalised by its weight sum l, stored in fp16 (11-bit
-// mantissa, half the bytes of fp32), divided by a scale that keeps every value within +-32768 (1 unless the split's
-// V rows exceed that), and the record (m, l, scale). o[i][r] = un-normalised out[dim 32j + 8r + i]; amax =
-// column_absmax(o).
+// mantissa, half the bytes of fp32), divided by a power of two that fits the column's largest value to fp16's range
+// (F16Range), and the record (m, l, scale). o[i][r] = un-normalised out[dim 32j + 8r + i]; amax = column_absmax(o).
 __device__ __forceinline__ void store_partial(const DecodeArgs& a, long slot, int head, int j, const floatx4 (&o)[8],
                                               float amax, float m_run, float l_tot) {
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  const float an = amax * inv;
-  const float scale = an > 32768.f ? an * (1.f / 32768.f) : 1.f;
-  const float f = inv / scale;
+  const F16Range range(amax * inv);
+  const float f = inv * range.inv;
   _Float16* po = a.part_o + (slot * kHeadsQ + head) * kHeadDim + 32 * j;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -106,7 +104,7 @@ __device__ __forceinline__ void store_partial(const DecodeArgs& a, long slot, in
     *reinterpret_cast<u32x4*>(po + 8 * r) = w;
   }
   if (j == 0)
-    *reinterpret_cast<floatx4*>(a.part_ml + (slot * kHeadsQ + head) * 4) = floatx4{m_run, l_tot, scale, 0.f};
+    *reinterpret_cast<floatx4*>(a.part_ml + (slot * kHeadsQ + head) * 4) = floatx4{m_run, l_tot, range.scale, 0.f};
 }
 
 // The end of a split shared by kSub waves, one wave per query head u (lane: dims 2 * lane, 2 * lane + 1): the output, or the
@@ -137,11 +135,11 @@ __device__ __forceinline__ void combine_subs(const DecodeArgs& a, const float (&
   float an = fmaxf(fabsf(x), fabsf(y)) * inv;
 #pragma unroll
   for (int k = 1; k < 64; k <<= 1) an = fmaxf(an, __shfl_xor(an, k, 64));
-  const float scale = an > 32768.f ? an * (1.f / 32768.f) : 1.f;
-  const float f = inv / scale;
+  const F16Range range(an);
+  const float f = inv * range.inv;
   const long at = ((long)b * a.part_stride + split) * kHeadsQ + head;
   *reinterpret_cast<uint32_t*>(a.part_o + at * kHeadDim + 2 * lane) = pack_f16x2(x * f, y * f);
-  if (lane == 0) *reinterpret_cast<floatx4*>(a.part_ml + at * 4) = floatx4{m, l, scale, 0.f};
+  if (lane == 0) *reinterpret_cast<floatx4*>(a.part_ml + at * 4) = floatx4{m, l, range.scale, 0.f};
 }
 
 template <int kW, int kSub>

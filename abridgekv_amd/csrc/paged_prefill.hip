@@ -235,9 +235,9 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
     return;
   }
   // Partials of uniform splits, which the caller asks for: the split's output normalised by its weight sum l, in fp16
-  // (half the bytes the epilogue writes and the merge reads), divided by a scale that keeps every value within +-32768
-  // (1 unless the split's V rows exceed that), and the record (m, l, scale). The scale needs the row's largest |o| over
-  // its 128 dims, which lie in the row's four lane groups (lanes m16 + 16j): reduced before any lane leaves.
+  // (half the bytes the epilogue writes and the merge reads), divided by a power of two that fits the row's largest
+  // value to fp16's range (F16Range), and the record (m, l, scale). The scale needs the row's largest |o| over its 128
+  // dims, which lie in the row's four lane groups (lanes m16 + 16j): reduced before any lane leaves.
   float amax[H];
   if (part_row >= 0) {
 #pragma unroll
@@ -256,14 +256,13 @@ __global__ __launch_bounds__(512, 1) void paged_prefill_kernel(PagedPrefillArgs 
     for (int u = 0; u < H; ++u) {
       const float l = l_run[u];
       const float inv = l > 0.f ? 1.f / l : 0.f;
-      const float an = amax[u] * inv;
-      const float scale = an > 32768.f ? an * (1.f / 32768.f) : 1.f;
+      const F16Range range(amax[u] * inv);
       const int head = kvh * kGroup + hbase + u;
       const long row = (part_row + (qi - q0)) * kHeadsQ + head;
       _Float16* po = a.part_o + row * kHeadDim + 32 * j;
 #pragma unroll
-      for (int p = 0; p < 4; ++p) store_acc_f16x8(po + 8 * p, o[2 * p][u], o[2 * p + 1][u], j, inv / scale);
-      if (j == 0) *reinterpret_cast<floatx4*>(a.part_ml + row * 4) = floatx4{m_run[u], l, scale, 0.f};
+      for (int p = 0; p < 4; ++p) store_acc_f16x8(po + 8 * p, o[2 * p][u], o[2 * p + 1][u], j, inv * range.inv);
+      if (j == 0) *reinterpret_cast<floatx4*>(a.part_ml + row * 4) = floatx4{m_run[u], l, range.scale, 0.f};
     }
     return;
   }

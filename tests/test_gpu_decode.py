@@ -240,3 +240,21 @@ def test_shared_splits_and_one_wave_per_split_agree_with_the_oracle(batch, split
     live = sl > 0
     assert np.abs(lse[live] - ref_l[live]).max() <= TOL
     assert np.all(np.isneginf(lse[~live])) and np.all(out[~live] == 0)
+
+
+@pytest.mark.parametrize("shift", [-24, 40])
+@pytest.mark.parametrize("batch", [3, 70])
+def test_split_partials_keep_small_and_large_values(batch, shift):
+    """Splits walked by four waves (few of them) and by one: V times 2^shift gives the output times 2^shift, bit for
+    bit, since every step from V to the bf16 output is linear in V and powers of two are exact. In unscaled fp16
+    partials the outputs (about 0.1) times 2^-24 would be subnormal."""
+    rng = np.random.default_rng(60)
+    lens = [90 + 7 * (i % 11) for i in range(batch)]
+    rows = [rng.standard_normal((n, 8, 128)).astype(np.float32) for n in lens]
+    cache, tables, seq_lens = _paged_cache(rows, rows, 900, rng, garbage=1.0)
+    q = rng.standard_normal((batch, 32, 128)).astype(np.float32)
+    out, lse = _run(q, cache, tables, seq_lens, split_pages=2)
+    cache[:, 1] *= 2.0 ** shift
+    out_s, lse_s = _run(q, cache, tables, seq_lens, split_pages=2)
+    assert np.array_equal(out_s, out * np.float32(2.0 ** shift))
+    assert np.array_equal(lse_s, lse)

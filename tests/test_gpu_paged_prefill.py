@@ -228,10 +228,11 @@ def test_calls_queued_behind_work_keep_their_own_metadata(split):
 
 
 @pytest.mark.parametrize("shift", [-24, 40])
-def test_planned_parts_keep_small_and_large_values(shift):
-    """A batch whose long tiles the plan splits: V times 2^shift gives the output times 2^shift, bit for bit. Every step
-    from V to the bf16 output is linear in V, and a power of two is exact in bf16 and in fp32 down to 2^-126; in fp16
-    partials the outputs (about 0.02) times 2^-24 would be subnormal."""
+@pytest.mark.parametrize("split", [None, 3])
+def test_planned_parts_keep_small_and_large_values(split, shift):
+    """A batch whose long tiles the plan splits (fp32 parts), and uniform splits (scaled fp16 parts): V times 2^shift gives the output times 2^shift, bit for bit. Every step
+    from V to the bf16 output is linear in V, and a power of two is exact in bf16 and in fp32 down to 2^-126; in
+    unscaled fp16 parts the outputs (about 0.02) times 2^-24 would be subnormal."""
     from abridgekv_amd import ops
     dev = torch.device("cuda")
     rows = [5000, 700, 300]
@@ -241,8 +242,8 @@ def test_planned_parts_keep_small_and_large_values(shift):
     q = torch.randn((457, 32, 128), generator=torch.Generator().manual_seed(41)).to(torch.bfloat16)
     small = cache.clone()
     small[:, 1] = (cache[:, 1].float() * 2.0 ** shift).to(torch.bfloat16)
-    out, lse = _run(cache, tables, q, q_start, start, limit, causal)
-    out_s, lse_s = _run(small, tables, q, q_start, start, limit, causal)
+    out, lse = _run(cache, tables, q, q_start, start, limit, causal, split)
+    out_s, lse_s = _run(small, tables, q, q_start, start, limit, causal, split)
     assert np.array_equal(out_s, out * np.float32(2.0 ** shift))
     assert np.array_equal(lse_s, lse)
 
