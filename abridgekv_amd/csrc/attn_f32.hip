@@ -118,6 +118,32 @@ __device__ __forceinline__ void f32_pv(const floatx4 (&va)[4], const floatx4 (&v
     }
 }
 
+__device__ __forceinline__ bool f32_finite(float x) { return fabsf(x) < INFINITY; }
+
+// V elements that are infinite or NaN, apart from the product: a key that a column does not see has weight 0 there, but the
+// matrix instruction multiplies every key with every column, and 0 x inf is NaN. What 16 keys' such elements give the
+// columns that see them (sees(key): this lane's column sees key 0 .. 15) is added to `extra` (this lane's dims of its row,
+// each 0, infinite or NaN; the caller has them set to 0 in the operands). load(key, chunk): V row `key` of the 16, dims
+// 4 * chunk .. + 3. Rare, and kept low in registers: it must not cost the loop around it an occupancy step.
+template <class Sees, class Load>
+__device__ __forceinline__ void f32_odd_v(const floatx4& p, Sees sees, float* extra, Load load) {
+  const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+#pragma unroll 1
+  for (int key = 0; key < 16; ++key) {
+    const int r = key & 3;
+    const float mine = r == 0 ? p[0] : r == 1 ? p[1] : r == 2 ? p[2] : p[3];
+    const float pk = __shfl(mine, 16 * (key >> 2) + m16, 64);
+    const bool vis = extra != nullptr && sees(key);
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {                            // dims 16g + 4i .., then 64 + those
+      const floatx4 x = load(key, 4 * g + (i & 3) + 16 * (i >> 2));
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (vis && !f32_finite(x[e])) extra[4 * (i & 3) + 64 * (i >> 2) + e] += pk * x[e];
+    }
+  }
+}
+
 // Keys a lane's column sees in a stage: key < lim, or lo <= key < lo + len.
 struct F32Span {
   int lim, lo;
@@ -202,9 +228,13 @@ struct PagedStages {
 // One wave's head over the stages: 16 query rows against K and V stages that the four waves of the workgroup load
 // together. The next stage's rows are on their way (in registers) while this one is multiplied. Row r's 16-byte chunk
 // c lies at chunk c ^ (r & 15), so both read patterns hit all banks.
-template <int kKeys, class Stages>
-__device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx4 (&q)[8], float scale, float& m,
-                                           float& l, floatx4 (&o)[8]) {
+// kOdd = false returns whether V held values that are not finite (uniform; one FMA per loaded value): then the result
+// holds only if every column sees every key of every stage, and f32_attend walks again with kOdd = true. That one keeps such
+// values out of the product and returns whether extra (this lane's dims 16g .. of its output row; nullptr: no row) holds
+// sums of f32_odd_v to be added. As a branch of the first walk they cost 5 % (masked, 3 x (512 + 128) rows).
+template <int kKeys, bool kOdd, class Stages>
+__device__ __forceinline__ bool f32_walk(Stages src, float* lds, const floatx4 (&q)[8], float scale, float* extra,
+                                           float& m, float& l, floatx4 (&o)[8]) {
   const int tid = threadIdx.x, lane = tid & 63, m16 = lane & 15, g = lane >> 4;
   const int r0 = tid >> 5, chunk = tid & 31;
   constexpr int kHalves = kKeys / 16, kStageElems = kKeys * kHeadDim;
@@ -221,7 +251,15 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
       }
     }
   };
+  float z = 0.f;                                             // 0 while all V values of this thread were finite, then NaN
+  bool dirty = false;                                        // (kOdd) extra holds sums
   auto store = [&](int n) {                                  // buffer n: K rows, then V rows
+    if constexpr (!kOdd) {
+#pragma unroll
+      for (int i = 0; i < 2 * kHalves; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z = fmaf(vr[i][e], 0.f, z);
+    }
     float* kb = lds + 2 * n * kStageElems;
     float* vb = kb + kStageElems;
 #pragma unroll
@@ -232,7 +270,7 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
     }
   };
   F32Stage cur, nxt;
-  if (!src.next(cur)) return;
+  if (!src.next(cur)) return false;
   load(cur);
   store(0);
   __syncthreads();
@@ -240,8 +278,11 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
     const bool more = src.next(nxt);
     if (more) load(nxt);
     const float* kb = lds + 2 * n * kStageElems;
-    const float* vb = kb + kStageElems;
+    float* vb = lds + (2 * n + 1) * kStageElems;
     floatx4 t[kHalves];
+    auto sees = [&](int key) {
+      return key < cur.end && (key < cur.span.lim || (unsigned)(key - cur.span.lo) < cur.span.len);
+    };
 #pragma unroll
     for (int i = 0; i < kHalves; ++i) {
       floatx4 kx[8];
@@ -251,12 +292,22 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
       t[i] = f32_scores(kx, q);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int key = cur.k0 + 16 * i + 4 * g + r;
-        const bool vis = key < cur.end && (key < cur.span.lim || (unsigned)(key - cur.span.lo) < cur.span.len);
-        t[i][r] = vis ? t[i][r] * scale : -INFINITY;
+        t[i][r] = sees(cur.k0 + 16 * i + 4 * g + r) ? t[i][r] * scale : -INFINITY;
       }
     }
     f32_softmax(t, m, l, o);
+    if constexpr (kOdd) {
+      for (int i = 0; i < 32 && !dirty && extra != nullptr; ++i) extra[(i & 15) + 64 * (i >> 4)] = 0.f;
+      dirty = true;
+#pragma unroll
+      for (int i = 0; i < kHalves; ++i)
+        f32_odd_v(t[i], [&](int key) { return sees(cur.k0 + 16 * i + key); }, extra, [&](int key, int c) {
+          return *reinterpret_cast<const floatx4*>(vb + (16 * i + key) * kHeadDim + 4 * (c ^ key));
+        });
+      __syncthreads();                                       // every wave has seen them
+      for (int i = tid; i < kStageElems; i += 256) vb[i] = f32_finite(vb[i]) ? vb[i] : 0.f;
+      __syncthreads();
+    }
 #pragma unroll
     for (int i = 0; i < kHalves; ++i) {
       floatx4 va[4], vb4[4];
@@ -275,6 +326,18 @@ __device__ __forceinline__ void f32_attend(Stages& src, float* lds, const floatx
     cur = nxt;
   }
   l = sum_xor32(sum_xor16(l));
+  return kOdd ? dirty : __syncthreads_or(z != z) != 0;
+}
+
+template <int kKeys, class Stages>
+__device__ __forceinline__ bool f32_attend(const Stages& src, float* lds, const floatx4 (&q)[8], float scale, float* extra,
+                                           float& m, float& l, floatx4 (&o)[8]) {
+  if (!f32_walk<kKeys, false>(src, lds, q, scale, extra, m, l, o)) return false;
+  m = -INFINITY;
+  l = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  return f32_walk<kKeys, true>(src, lds, q, scale, extra, m, l, o);
 }
 
 __device__ __forceinline__ void f32_load_q(const float* row, int g, bool ok, floatx4 (&q)[8]) {
@@ -282,13 +345,18 @@ __device__ __forceinline__ void f32_load_q(const float* row, int g, bool ok, flo
   for (int c = 0; c < 8; ++c) q[c] = ok ? ldf4(row + 16 * c + 4 * g) : floatx4{0.f, 0.f, 0.f, 0.f};
 }
 
-__device__ __forceinline__ void f32_store(float* row, int g, float l, const floatx4 (&o)[8]) {
+// add: the row holds sums of f32_odd_v.
+__device__ __forceinline__ void f32_store(float* row, int g, float l, const floatx4 (&o)[8], bool add) {
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      stf4(row + 64 * h + 16 * g + 4 * r, floatx4{o[4 * h][r], o[4 * h + 1][r], o[4 * h + 2][r], o[4 * h + 3][r]} * inv);
+    for (int r = 0; r < 4; ++r) {
+      float* at = row + 64 * h + 16 * g + 4 * r;
+      floatx4 x = floatx4{o[4 * h][r], o[4 * h + 1][r], o[4 * h + 2][r], o[4 * h + 3][r]} * inv;
+      if (add) x += ldf4(at);
+      stf4(at, x);
+    }
 }
 
 // The sum in 64 bits: m lies up to the headroom below the largest score, so log(l) alone would round more coarsely.
@@ -301,7 +369,7 @@ __device__ __forceinline__ float f32_lse(float m, float l) {
 // shared by the four heads and the segment walk instead of VALU dot products per key with the mask's predicate per
 // element: masked, B=1, 3 x (512 + 128) rows 1546 -> 203 us; a code step of 256 rows over 4000 keys 2059 -> 412 us.
 template <bool kMasked, int kKeys>
-__global__ __launch_bounds__(256, 2) void attn_f32_rows_kernel(F32Args a) {
+__global__ __launch_bounds__(256, kKeys == 16 ? 3 : 2) void attn_f32_rows_kernel(F32Args a) {
   __shared__ __attribute__((aligned(16))) float lds[4 * kKeys * kHeadDim];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
@@ -334,9 +402,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32_rows_kernel(F32Args a) {
                      a.k_ss, a.v_ss,
                      SegWalk(g_, q0, min(q0 + kF32Rows, a.seq_len) - 1, plen, qmin, qmax, quota, quota), g_,
                      row_facts(g_, qrow), plen, quota, 0};
-    f32_attend<kKeys>(src, lds, q, a.scale, m, l, o);
+    float* out = a.out + (long)b * a.o_sb + (long)qrow * a.o_st + (long)head * a.o_sh;
+    const bool add = f32_attend<kKeys>(src, lds, q, a.scale, qrow < a.seq_len ? out + 16 * g : nullptr, m, l, o);
     if (qrow >= a.seq_len) return;
-    f32_store(a.out + (long)b * a.o_sb + (long)qrow * a.o_st + (long)head * a.o_sh, g, l, o);
+    f32_store(out, g, l, o, add);
     if (a.lse != nullptr && g == 0) a.lse[((long)b * kHeadsQ + head) * a.seq_len + qrow] = f32_lse(m, l);
   } else {
     // the rows of 16 consecutive tokens, request by request (uniform over the workgroup)
@@ -361,9 +430,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32_rows_kernel(F32Args a) {
       f32_load_q(a.q + (long)min(row, t1 - 1) * a.q_st + (long)head * a.q_sh, g, row < t1, q);
       PagedStages<kKeys> src{a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages,
                       causal ? min(limit, pos + n) : limit, 0, span};
-      f32_attend<kKeys>(src, lds, q, a.scale, m, l, o);
+      float* out = a.out + (long)row * a.o_st + (long)head * a.o_sh;
+      const bool add = f32_attend<kKeys>(src, lds, q, a.scale, row < t1 ? out + 16 * g : nullptr, m, l, o);
       if (row < t1) {
-        f32_store(a.out + (long)row * a.o_st + (long)head * a.o_sh, g, l, o);
+        f32_store(out, g, l, o, add);
         if (a.lse != nullptr && g == 0) a.lse[(long)row * kHeadsQ + head] = f32_lse(m, l);
       }
       t = t1;
@@ -423,6 +493,11 @@ __global__ __launch_bounds__(64 * kDecWaves, 2) void decode_f32_kernel(F32Args a
 #pragma unroll
       for (int r = 0; r < 4; ++r) t[0][r] = p * kPage + 4 * g + r < n_keys ? t[0][r] * a.scale : -INFINITY;
       f32_softmax(t, m, l, o);
+      if (n_keys - p * kPage < kPage) {                      // 0 x inf is NaN: no copies of the last row in the product
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (p * kPage + 4 * g + r >= n_keys) va[r] = vb[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
       f32_pv(va, vb, t[0], o);
     }
   }
@@ -452,7 +527,7 @@ __global__ __launch_bounds__(64 * kDecWaves, 2) void decode_f32_kernel(F32Args a
     acc += po[i][u][d] * f;
   }
   const int head = kvh * kGroup + u;
-  a.out[(long)b * a.o_st + (long)head * a.o_sh + d] = L > 0.f ? acc * (1.f / L) : 0.f;
+  a.out[(long)b * a.o_st + (long)head * a.o_sh + d] = acc * (L > 0.f ? 1.f / L : 0.f);   // (sums of NaN stay NaN)
   if (a.lse != nullptr && d == 0) a.lse[(long)b * kHeadsQ + head] = f32_lse(M, L);
 }
 

@@ -172,3 +172,78 @@ def test_paged_f32_tiles_with_rows_of_several_requests(causal):
             ro, rl = od.decode_fp64(q[a + i].numpy(), k[:n], v[:n], 128 ** -0.5)
             assert np.abs(got_o[a + i] - ro).max() <= TOL, f"request {r} row {i}"
             assert np.abs(got_l[a + i] - rl).max() <= TOL, f"request {r} row {i}"
+
+
+def _bits(x):
+    return x.cpu().numpy().view(np.uint32)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_paged_f32_infinite_values_reach_only_the_rows_that_see_them(bad):
+    """V elements of one late token of a causal chunk, and of a range hidden by `excluded`, infinite or NaN: rows that do
+    not see the token keep every bit, rows that do get it in that head's dims alone (inf with the weight's sign, NaN)."""
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    cache, tables = _paged([200, 90], 60, 30)
+    g = torch.Generator().manual_seed(31)
+    q = torch.randn((40 + 20, 32, 128), generator=g, dtype=torch.float32).to(dev)
+    bt = torch.from_numpy(tables).to(dev)
+
+    def call(c):
+        return ops.paged_prefill_attention(q, c.to(dev), bt, [0, 40, 60], [160, 60], [200, 80], [True, False],
+                                           excluded=[None, (33, 50)])[0]
+    clean = call(cache)
+    dirty = cache.clone()
+    pos, hid = 160 + 21, 40                                  # row 21's own key; a hidden key of the second request
+    dirty[tables[0, pos // 16], 1, pos % 16, 3, [0, 77]] = bad
+    dirty[tables[0, 50 // 16], 1, 50 % 16, 6, 5] = -bad       # a key that every row of the chunk sees
+    dirty[tables[1, hid // 16], 1, hid % 16] = bad
+    got = call(dirty)
+    want = clean.clone()
+    want[21:40, 12:16, 0] = want[21:40, 12:16, 77] = bad
+    want[:40, 24:28, 5] = -bad
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert np.array_equal(_bits(got.nan_to_num(nan=7.0)), _bits(want.nan_to_num(nan=7.0)))
+
+
+@pytest.mark.parametrize("K", [16, 0])
+def test_masked_f32_infinite_values_reach_only_the_rows_that_see_them(K):
+    """The same under the compression mask: content of block 0 is hidden from later blocks, a row's later keys from it."""
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    C, N = 40, 3
+    S = N * (C + K)
+    g = torch.Generator().manual_seed(32)
+    q, k, v = (torch.randn((1, S, h, 128), generator=g, dtype=torch.float32).to(dev) for h in (32, 8, 8))
+    clean = ops.prefill_masked_attention(q, k, v, C, K, N)[0]
+    bad = v.clone()
+    bad[0, 13, 2, 9] = float("inf")
+    got = ops.prefill_masked_attention(q, k, bad, C, K, N)[0]
+    sees = torch.from_numpy(np.asarray(op.arith_mask(C, K, N, None, None))).reshape(-1, S, S)[0, :, 13].to(dev)
+    want = clean.clone()
+    want[0, sees, 8:12, 9] = float("inf")
+    assert 0 < int(sees.sum()) < S - 13
+    assert np.array_equal(_bits(got), _bits(want))
+
+
+def test_decode_f32_passes_nan_and_infinities_on():
+    """A NaN key makes its head's outputs NaN; an infinite V element of a sequence's last row, whose page is partly
+    filled, makes that dim infinite and nothing else."""
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    lens = [37, 200]
+    cache, tables = _paged(lens, 40, 33)
+    q = torch.randn((2, 32, 128), generator=torch.Generator().manual_seed(34), dtype=torch.float32).to(dev)
+
+    def call(c):
+        return ops.decode_attention(q, c.to(dev), torch.from_numpy(tables).to(dev),
+                                    torch.tensor(lens, dtype=torch.int32, device=dev), 128 ** -0.5)[0]
+    want = call(cache)
+    bad = cache.clone()
+    bad[tables[0, 36 // 16], 1, 36 % 16, 1, 100] = float("inf")
+    bad[tables[1, 150 // 16], 0, 150 % 16, 5, 3] = float("nan")
+    got = call(bad)
+    want[0, 4:8, 100] = float("inf")
+    want[1, 20:24] = float("nan")
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert np.array_equal(_bits(got.nan_to_num(nan=7.0)), _bits(want.nan_to_num(nan=7.0)))
