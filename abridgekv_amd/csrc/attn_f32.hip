@@ -48,6 +48,7 @@ struct F32Args {
   int replay_rows;             // replay rows after each block's codes
   int replay_exclude;          // the codes do not see the block's last replay_rows content rows
   int num_tokens;
+  int windows, window_parts;   // paged: 16-token windows, workgroups per window and KV head
   float scale;
   float* out;
   long o_sb, o_st, o_sh;
@@ -119,6 +120,16 @@ __device__ __forceinline__ void f32_pv(const floatx4 (&va)[4], const floatx4 (&v
 }
 
 __device__ __forceinline__ bool f32_finite(float x) { return fabsf(x) < INFINITY; }
+
+// z stays 0 while all x are finite (four sums: a short chain).
+__device__ __forceinline__ void f32_probe(const floatx4& x, floatx4& z) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) z[e] = fmaf(x[e], 0.f, z[e]);
+}
+__device__ __forceinline__ bool f32_odd(const floatx4& z) {
+  const float s = (z[0] + z[1]) + (z[2] + z[3]);
+  return s != s;
+}
 
 // V elements that are infinite or NaN, apart from the product: a key that a column does not see has weight 0 there, but the
 // matrix instruction multiplies every key with every column, and 0 x inf is NaN. What 16 keys' such elements give the
@@ -251,14 +262,12 @@ __device__ __forceinline__ bool f32_walk(Stages src, float* lds, const floatx4 (
       }
     }
   };
-  float z = 0.f;                                             // 0 while all V values of this thread were finite, then NaN
+  floatx4 z = {0.f, 0.f, 0.f, 0.f};                          // 0 while all V values of this thread were finite, else a NaN
   bool dirty = false;                                        // (kOdd) extra holds sums
   auto store = [&](int n) {                                  // buffer n: K rows, then V rows
     if constexpr (!kOdd) {
 #pragma unroll
-      for (int i = 0; i < 2 * kHalves; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) z = fmaf(vr[i][e], 0.f, z);
+      for (int i = 0; i < 2 * kHalves; ++i) f32_probe(vr[i], z);
     }
     float* kb = lds + 2 * n * kStageElems;
     float* vb = kb + kStageElems;
@@ -326,7 +335,7 @@ __device__ __forceinline__ bool f32_walk(Stages src, float* lds, const floatx4 (
     cur = nxt;
   }
   l = sum_xor32(sum_xor16(l));
-  return kOdd ? dirty : __syncthreads_or(z != z) != 0;
+  return kOdd ? dirty : __syncthreads_or(f32_odd(z)) != 0;
 }
 
 template <int kKeys, class Stages>
@@ -362,6 +371,121 @@ __device__ __forceinline__ void f32_store(float* row, int g, float l, const floa
 // The sum in 64 bits: m lies up to the headroom below the largest score, so log(l) alone would round more coarsely.
 __device__ __forceinline__ float f32_lse(float m, float l) {
   return l > 0.f ? (float)((double)m + log((double)l)) : -INFINITY;
+}
+
+__device__ const float kZeroRow[kHeadDim] = {};
+
+// A wave's share of paged keys, pages w, w + kWaves, ... straight into operand registers (the next page's K loads while this
+// page is multiplied). kSpan: the columns see keys of `span`, which may differ; otherwise all of them. Returns (kSpan)
+// whether this lane met a V value that is not finite: the sums then hold only if every column sees every key.
+template <int kWaves, bool kSpan>
+__device__ __forceinline__ bool f32_pages(const float* kv, const int32_t* block_table, int num_pages, int n_keys,
+                                           const F32Span& span, float scale, int w, const floatx4 (&q)[8], float& m,
+                                           float& l, floatx4 (&o)[8]) {
+  const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+  const int n_pages = (n_keys + kPage - 1) / kPage;
+  const __attribute__((address_space(4))) int32_t* table = (const __attribute__((address_space(4))) int32_t*)block_table;
+  floatx4 kx[8], z = {0.f, 0.f, 0.f, 0.f};
+  m = -INFINITY;
+  l = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto page_of = [&](int p) { return kv + (long)min(max(table[p], 0), num_pages - 1) * kPageElems; };
+  auto load_k = [&](const float* page, int p) {              // rows past the end: the last row (not seen)
+    const float* r = page + min(m16, n_keys - 1 - p * kPage) * kSlotElems + 4 * g;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) kx[c] = ldf4(r + 16 * c);
+  };
+  if (w < n_pages) {
+    const float* page = page_of(w);
+    load_k(page, w);
+    for (int p = w; p < n_pages; p += kWaves) {
+      floatx4 va[4], vb[4], t[1];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {                          // rows past the end: zeros (0 x inf is NaN)
+        const float* vr = 4 * g + r < n_keys - p * kPage ? page + kHalfElems + (4 * g + r) * kSlotElems : kZeroRow;
+        va[r] = ldf4(vr + 4 * m16);
+        vb[r] = ldf4(vr + 4 * m16 + 64);
+        if constexpr (kSpan) {
+          f32_probe(va[r], z);
+          f32_probe(vb[r], z);
+        }
+      }
+      t[0] = f32_scores(kx, q);
+      if (p + kWaves < n_pages) {
+        page = page_of(p + kWaves);
+        load_k(page, p + kWaves);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = p * kPage + 4 * g + r;
+        const bool vis = kSpan ? key < span.lim || (unsigned)(key - span.lo) < span.len : key < n_keys;
+        t[0][r] = vis ? t[0][r] * scale : -INFINITY;
+      }
+      f32_softmax(t, m, l, o);
+      f32_pv(va, vb, t[0], o);
+    }
+  }
+  l = sum_xor32(sum_xor16(l));
+  return f32_odd(z);
+}
+
+// A lane's sums to a row of 128 dims.
+__device__ __forceinline__ void f32_put(float* row, int g, const floatx4 (&o)[8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<floatx4*>(row + 64 * h + 16 * g + 4 * r) =
+          floatx4{o[4 * h][r], o[4 * h + 1][r], o[4 * h + 2][r], o[4 * h + 3][r]};
+}
+
+// Up to kNarrowRows rows of one request against a KV head, by the four waves of a workgroup: the 16 columns are 4 heads x 4
+// rows, and the waves share the request's pages instead of the heads. A tile of 16 rows by head would leave 12 of 16
+// columns empty (16 requests of one row over 5000 keys, one after the other in both forms: 7700 us by head, 2320 so; a wave
+// of dot products per token and KV head took 2967). Writes the rows and returns false, or returns true (uniform) and writes nothing if V held values that are
+// not finite. lds: 4 x 16 x (128 + 2) floats.
+constexpr int kNarrowRows = 4;
+__device__ __forceinline__ bool f32_narrow(const F32Args& a, float* lds, const F32Span& span, int n_keys, int b, int kvh,
+                                           int t, int t1) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+  const int row = t + (m16 & 3);
+  floatx4 q[8], o[8];
+  float m, l;
+  f32_load_q(a.q + (long)min(row, t1 - 1) * a.q_st + (long)(kvh * kGroup + (m16 >> 2)) * a.q_sh, g, row < t1, q);
+  const bool odd = f32_pages<4, true>(a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages, n_keys, span,
+                                    a.scale, w, q, m, l, o);
+  float* ml = lds + 4 * 16 * kHeadDim;
+  f32_put(lds + (w * 16 + m16) * kHeadDim, g, o);
+  if (g == 0) *reinterpret_cast<float2*>(ml + 2 * (w * 16 + m16)) = make_float2(m, l);
+  if (__syncthreads_or(odd)) return true;
+  const int col = threadIdx.x >> 4, d = 8 * (threadIdx.x & 15), out_row = t + (col & 3);
+  float M = -INFINITY, L = 0.f;
+  floatx4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+  float2 rec[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    rec[i] = *reinterpret_cast<const float2*>(ml + 2 * (i * 16 + col));
+    M = fmaxf(M, rec[i].x);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float f = rec[i].x == M ? 1.f : expf(rec[i].x - M);          // (both -inf: sums of 0 or of NaN)
+    const float* p = lds + (i * 16 + col) * kHeadDim + d;
+    L += rec[i].y * f;
+    x += *reinterpret_cast<const floatx4*>(p) * f;
+    y += *reinterpret_cast<const floatx4*>(p + 4) * f;
+  }
+  if (out_row < t1) {
+    const int head = kvh * kGroup + (col >> 2);
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    float* out = a.out + (long)out_row * a.o_st + (long)head * a.o_sh + d;
+    stf4(out, x * inv);
+    stf4(out + 4, y * inv);
+    if (a.lse != nullptr && d == 0) a.lse[(long)out_row * kHeadsQ + head] = f32_lse(M, L);
+  }
+  return false;
 }
 
 // Multi-query attention, masked (kMasked) or paged: a workgroup of 4 waves takes 16 query rows of one KV head, one query
@@ -408,48 +532,55 @@ __global__ __launch_bounds__(256, kKeys == 16 ? 3 : 2) void attn_f32_rows_kernel
     f32_store(out, g, l, o, add);
     if (a.lse != nullptr && g == 0) a.lse[((long)b * kHeadsQ + head) * a.seq_len + qrow] = f32_lse(m, l);
   } else {
-    // the rows of 16 consecutive tokens, request by request (uniform over the workgroup)
-    const int t0 = blockIdx.x / kHeadsKV * kF32Rows, t_end = min(t0 + kF32Rows, a.num_tokens);
+    // windows of 16 consecutive tokens; a window's requests go to window_parts workgroups in turn (all uniform)
+    const int window = blockIdx.x / kHeadsKV % a.windows, part = blockIdx.x / kHeadsKV / a.windows;
+    const int t0 = window * kF32Rows, t_end = min(t0 + kF32Rows, a.num_tokens);
     const int my_req = a.tok_req[min(t0 + m16, t_end - 1)];
-    for (int t = t0; t < t_end;) {
+    for (int t = t0, t1, turn = 0; t < t_end; t = t1, ++turn) {
       const int b = __builtin_amdgcn_readlane(my_req, t - t0);
       // tokens of this request from t on (lanes 0 .. 15 hold the window's requests)
       const unsigned differs = (unsigned)__ballot(my_req != b) & 0xffffu & (~0u << (t - t0));
-      const int t1 = min(differs ? t0 + __ffs(differs) - 1 : t_end, t_end);
+      t1 = min(differs ? t0 + __ffs(differs) - 1 : t_end, t_end);
+      if (turn % a.window_parts != part) continue;
       const int n = t1 - t;
-      const int row = t + m16;                               // this lane's token (valid below t1)
       const int pos = a.kv_start[b] + t - a.q_start[b];      // position of row t
       const int limit = min(a.kv_limit[b], a.bt_width * kPage);
       const bool causal = a.causal ? a.causal[b] != 0 : a.causal_default != 0;
-      const int lane_limit = row >= t1 ? 0 : causal ? min(limit, pos + m16 + 1) : limit;
-      F32Span span{lane_limit, 0, 0u};
-      if (a.kv_excluded != nullptr) {
-        const int lo = a.kv_excluded[2 * b], hi = a.kv_excluded[2 * b + 1];
-        if (lo < hi) span = F32Span{min(lane_limit, lo), hi, (unsigned)max(lane_limit - hi, 0)};
-      }
-      f32_load_q(a.q + (long)min(row, t1 - 1) * a.q_st + (long)head * a.q_sh, g, row < t1, q);
-      PagedStages<kKeys> src{a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages,
-                      causal ? min(limit, pos + n) : limit, 0, span};
-      float* out = a.out + (long)row * a.o_st + (long)head * a.o_sh;
-      const bool add = f32_attend<kKeys>(src, lds, q, a.scale, row < t1 ? out + 16 * g : nullptr, m, l, o);
-      if (row < t1) {
-        f32_store(out, g, l, o, add);
-        if (a.lse != nullptr && g == 0) a.lse[(long)row * kHeadsQ + head] = f32_lse(m, l);
-      }
-      t = t1;
-      m = -INFINITY;
-      l = 0.f;
+      const int n_keys = causal ? min(limit, pos + n) : limit;
+      auto span_of = [&](int i) {                            // keys that row t + i sees
+        const int lim = i >= n ? 0 : causal ? min(limit, pos + i + 1) : limit;
+        F32Span span{lim, 0, 0u};
+        if (a.kv_excluded != nullptr) {
+          const int lo = a.kv_excluded[2 * b], hi = a.kv_excluded[2 * b + 1];
+          if (lo < hi) span = F32Span{min(lim, lo), hi, (unsigned)max(lim - hi, 0)};
+        }
+        return span;
+      };
+      if (n > kNarrowRows || f32_narrow(a, lds, span_of(m16 & 3), n_keys, b, kvh, t, t1)) {
+        const int row = t + m16;                             // this lane's token (valid below t1)
+        f32_load_q(a.q + (long)min(row, t1 - 1) * a.q_st + (long)head * a.q_sh, g, row < t1, q);
+        PagedStages<kKeys> src{a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages, n_keys, 0,
+                               span_of(m16)};
+        float* out = a.out + (long)row * a.o_st + (long)head * a.o_sh;
+        const bool add = f32_attend<kKeys>(src, lds, q, a.scale, row < t1 ? out + 16 * g : nullptr, m, l, o);
+        if (row < t1) {
+          f32_store(out, g, l, o, add);
+          if (a.lse != nullptr && g == 0) a.lse[(long)row * kHeadsQ + head] = f32_lse(m, l);
+        }
+        m = -INFINITY;
+        l = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
       __syncthreads();                                       // the next request's first stage overwrites this one's
     }
   }
 }
 
-// Decode: a workgroup of 8 waves per (sequence, KV head); wave w takes pages w, w + 8, ... straight into operand
-// registers (the next page's K loads while this page is multiplied) and the eight partial results meet in LDS. The four
-// heads fill the 16 columns four times over: the path is bound by memory, not by the matrix rate. 32 sequences of
-// 900 .. 9500 rows 7014 -> 286 us (4.8 TB/s), one of 5000 rows 2102 -> 108 us, against the VALU form of one wave each.
+// Decode: a workgroup of 8 waves per (sequence, KV head); the waves share the pages (f32_pages) and their partial results
+// meet in LDS. The four heads fill the 16 columns four times over: the path is bound by memory, not by the matrix rate. 32
+// sequences of 900 .. 9500 rows 7014 -> 286 us (4.8 TB/s), one of 5000 rows 2102 -> 108 us, against the VALU form of one
+// wave each.
 constexpr int kDecWaves = 8;
 __global__ __launch_bounds__(64 * kDecWaves, 2) void decode_f32_kernel(F32Args a) {
   __shared__ __attribute__((aligned(16))) float po[kDecWaves][kGroup][kHeadDim];
@@ -458,57 +589,13 @@ __global__ __launch_bounds__(64 * kDecWaves, 2) void decode_f32_kernel(F32Args a
   const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
   const int kvh = blockIdx.x % kHeadsKV, b = blockIdx.x / kHeadsKV;
   const int n_keys = max(min(a.seq_lens[b], a.max_pages * kPage), 0);
-  const int n_pages = (n_keys + kPage - 1) / kPage;
-  const __attribute__((address_space(4))) int32_t* table =
-      (const __attribute__((address_space(4))) int32_t*)(a.block_table + (long)b * a.bt_stride);
-  floatx4 q[8], o[8], kx[8];
+  floatx4 q[8], o[8];
   f32_load_q(a.q + (long)b * a.q_st + (long)(kvh * kGroup + (m16 & 3)) * a.q_sh, g, true, q);
-  float m = -INFINITY, l = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  auto page_of = [&](int p) {
-    return a.kv + (long)min(max(table[p], 0), a.num_pages - 1) * kPageElems + kvh * kHeadDim;
-  };
-  auto load_k = [&](const float* page, int p) {              // rows past the end: the last row (weight 0)
-    const float* r = page + min(m16, n_keys - 1 - p * kPage) * kSlotElems + 4 * g;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) kx[c] = ldf4(r + 16 * c);
-  };
-  if (w < n_pages) {
-    const float* page = page_of(w);
-    load_k(page, w);
-    for (int p = w; p < n_pages; p += kDecWaves) {
-      floatx4 va[4], vb[4], t[1];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float* vr = page + kHalfElems + min(4 * g + r, n_keys - 1 - p * kPage) * kSlotElems + 4 * m16;
-        va[r] = ldf4(vr);
-        vb[r] = ldf4(vr + 64);
-      }
-      t[0] = f32_scores(kx, q);
-      if (p + kDecWaves < n_pages) {
-        page = page_of(p + kDecWaves);
-        load_k(page, p + kDecWaves);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) t[0][r] = p * kPage + 4 * g + r < n_keys ? t[0][r] * a.scale : -INFINITY;
-      f32_softmax(t, m, l, o);
-      if (n_keys - p * kPage < kPage) {                      // 0 x inf is NaN: no copies of the last row in the product
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (p * kPage + 4 * g + r >= n_keys) va[r] = vb[r] = floatx4{0.f, 0.f, 0.f, 0.f};
-      }
-      f32_pv(va, vb, t[0], o);
-    }
-  }
-  l = sum_xor32(sum_xor16(l));
+  float m, l;
+  f32_pages<kDecWaves, false>(a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages, n_keys, F32Span{},
+                              a.scale, w, q, m, l, o);
   if (m16 < kGroup) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        *reinterpret_cast<floatx4*>(&po[w][m16][64 * h + 16 * g + 4 * r]) =
-            floatx4{o[4 * h][r], o[4 * h + 1][r], o[4 * h + 2][r], o[4 * h + 3][r]};
+    f32_put(po[w][m16], g, o);
     if (g == 0) {
       pm[w][m16] = m;
       pl[w][m16] = l;
@@ -610,7 +697,14 @@ int abkv_paged_prefill_attn_f32(const float* q, long q_stride_t, long q_stride_h
   a.o_st = out_stride_t;
   a.o_sh = out_stride_h;
   a.lse = lse;
-  const unsigned grid = f32_grid(((long)num_tokens + kF32Rows - 1) / kF32Rows);
+  // A window may hold rows of up to 16 requests, which one workgroup would walk one after the other: 16 workgroups a window
+  // where windows are few, 4 where they fill the GPU anyway. A workgroup that finds no request left ends at once: a code
+  // step and a prompt of 2000 rows take the same with 1, 4 or 16. us with 16 / 4 / 1: 16 requests of one row over 5000
+  // keys 159 / - / 2320, 256 over 2000 500 / - / 991, 1024 over 500 548 / 528 / 525, 2048 over 300 688 / 656 / 645.
+  const long windows = ((long)num_tokens + kF32Rows - 1) / kF32Rows;
+  a.windows = (int)windows;
+  a.window_parts = windows <= 32 ? 16 : f32_grid(4 * windows) != 0 ? 4 : 1;
+  const unsigned grid = f32_grid(windows * a.window_parts);
   if (grid == 0) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL((attn_f32_rows_kernel<false, 32>), dim3(grid), dim3(256), 0, stream, a);
   return (int)hipGetLastError();

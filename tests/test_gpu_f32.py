@@ -247,3 +247,48 @@ def test_decode_f32_passes_nan_and_infinities_on():
     want[1, 20:24] = float("nan")
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     assert np.array_equal(_bits(got.nan_to_num(nan=7.0)), _bits(want.nan_to_num(nan=7.0)))
+
+
+@pytest.mark.parametrize("rows", [[1, 2, 3, 4, 5], [1], [4, 17]])
+@pytest.mark.parametrize("requests", [9, 210])
+def test_paged_f32_many_short_requests(rows, requests):
+    """Windows with up to sixteen requests, few of them (a workgroup per request) and many; rows at both sides of the
+    four that share a workgroup's columns; excluded ranges. Tolerance as above."""
+    from abridgekv_amd import ops
+    qlen = [rows[i % len(rows)] for i in range(requests)]
+    past = [(11 * i) % 70 for i in range(requests)]
+    sls = [a + b for a, b in zip(qlen, past)]
+    excluded = [(5, 9) if p > 20 else None for p in past]
+    cache, tables = _paged(sls, 2000, 40)
+    qsl = np.concatenate([[0], np.cumsum(qlen)])
+    q = torch.randn((int(qsl[-1]), 32, 128), generator=torch.Generator().manual_seed(41), dtype=torch.float32)
+    dev = torch.device("cuda")
+    lse = torch.empty((int(qsl[-1]), 32), dtype=torch.float32, device=dev)
+    out, _ = ops.paged_prefill_attention(q.to(dev), cache.to(dev), torch.from_numpy(tables).to(dev), qsl, past, sls, True,
+                                         lse=lse, excluded=excluded)
+    got_o, got_l = out.cpu().numpy(), lse.cpu().numpy()
+    for r, sl in enumerate(sls):
+        k, v = od.paged_rows(cache.numpy(), tables[r], sl)
+        for i in range(qlen[r]):
+            keep = np.arange(past[r] + i + 1)
+            if excluded[r]:
+                keep = keep[(keep < 5) | (keep >= 9)]
+            ro, rl = od.decode_fp64(q[qsl[r] + i].numpy(), k[keep], v[keep], 128 ** -0.5)
+            assert np.abs(got_o[qsl[r] + i] - ro).max() <= TOL, f"request {r} row {i}"
+            assert np.abs(got_l[qsl[r] + i] - rl).max() <= TOL, f"request {r} row {i}"
+
+
+def test_paged_f32_infinite_values_in_a_short_chunk():
+    """Three rows that share a workgroup's columns, the last one's own V row infinite in one dim: nothing else changes
+    but the order of the sums (the tile is walked again, a head per wave)."""
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    cache, tables = _paged([100], 20, 50)
+    q = torch.randn((3, 32, 128), generator=torch.Generator().manual_seed(51), dtype=torch.float32).to(dev)
+    bt = torch.from_numpy(tables).to(dev)
+    clean = ops.paged_prefill_attention(q, cache.to(dev), bt, [0, 3], [97], [100], True)[0]
+    cache[tables[0, 99 // 16], 1, 99 % 16, 2, 50] = float("inf")
+    got = ops.paged_prefill_attention(q, cache.to(dev), bt, [0, 3], [97], [100], True)[0]
+    assert torch.isinf(got[2, 8:12, 50]).all()
+    got[2, 8:12, 50] = clean[2, 8:12, 50]
+    assert (got - clean).abs().max() <= TOL
