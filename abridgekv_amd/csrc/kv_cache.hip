@@ -22,6 +22,8 @@
 //
 // KV append: replaces the stock vLLM compiled op reshape_and_cache(_flash) that writes each new token's K and V
 // rows at slot_mapping[t] (slots from block_table.py:186-197); slot < 0 is skipped (padding).
+#include <algorithm>
+
 #include "abridgekv_amd.h"
 #include "common.h"
 
@@ -533,11 +535,12 @@ int abkv_kv_move_groups(const abkv_move_group* groups, int n_groups, int block_s
     if (g.n_segments == 0 && g.n_free == 0) continue;
     if ((g.n_segments > 0 && (g.ops == nullptr || g.seg_offsets == nullptr)) ||
         (g.n_free > 0 && g.free_ops == nullptr) || slot_bytes <= 0 || slot_bytes % 16 != 0 ||
-        g.layer_caches == nullptr || !fill_layers(lp, g.layer_caches, g.n_layers) ||
-        ((long)g.n_segments * kMoveParts + (g.n_free + kFreeRows - 1L) / kFreeRows) * g.n_layers > 0xFFFFFFFFL / 256)
+        g.layer_caches == nullptr || !fill_layers(lp, g.layer_caches, g.n_layers))
       return (int)hipErrorInvalidValue;
   }
-  for (int next = 0; next < n_groups;) {
+  constexpr long kMaxWorkgroups = 0xFFFFFFFFL / 256;         // work items of a launch fit 32 bits
+  int next = 0, seg = 0, op = 0;                             // next group, and its next segment and independent op
+  while (next < n_groups) {
     MoveGroupsArgs a;
     a.page_bytes = page_bytes;
     a.half_bytes = half_bytes;
@@ -546,24 +549,35 @@ int abkv_kv_move_groups(const abkv_move_group* groups, int n_groups, int block_s
     a.block_size = block_size;
     a.n_groups = 0;
     long n_ordered[kMaxMoveGroups], n_free[kMaxMoveGroups], total = 0;
-    // groups while they fit the arguments and the grid
-    for (; next < n_groups && a.n_groups < kMaxMoveGroups; ++next) {
+    // groups while they fit the arguments and the grid; of one that does not, as many segments and ops as do (they are
+    // independent of each other), the rest in the next launch
+    while (next < n_groups && a.n_groups < kMaxMoveGroups) {
       const abkv_move_group& s = groups[next];
-      if (s.n_segments == 0 && s.n_free == 0) continue;
-      const long no = (long)s.n_segments * kMoveParts * s.n_layers;
-      const long nf = (s.n_free + kFreeRows - 1L) / kFreeRows * s.n_layers;
-      if (total + no + nf > 0xFFFFFFFFL / 256) break;
-      total += no + nf;
-      n_ordered[a.n_groups] = no;
-      n_free[a.n_groups] = nf;
+      if (s.n_segments == 0 && s.n_free == 0) {
+        ++next;
+        continue;
+      }
+      const int ns = (int)std::min<long>(s.n_segments - seg, (kMaxWorkgroups - total) / (kMoveParts * s.n_layers));
+      total += (long)ns * kMoveParts * s.n_layers;
+      const int nf = (int)std::min<long>(s.n_free - op, (kMaxWorkgroups - total) / s.n_layers * kFreeRows);
+      const long nf_wgs = (nf + kFreeRows - 1L) / kFreeRows * s.n_layers;
+      total += nf_wgs;
+      if (ns + (long)nf == 0) break;
+      n_ordered[a.n_groups] = (long)ns * kMoveParts * s.n_layers;
+      n_free[a.n_groups] = nf_wgs;
       MoveGroup& g = a.group[a.n_groups++];
       fill_layers(g.layers, s.layer_caches, s.n_layers);
       g.ops = s.ops;
-      g.seg_offsets = s.seg_offsets;
-      g.free_ops = s.free_ops;
-      g.n_seg = s.n_segments;
-      g.n_free = s.n_free;
+      g.seg_offsets = s.seg_offsets + seg;
+      g.free_ops = s.free_ops + 4L * op;
+      g.n_seg = ns;
+      g.n_free = nf;
       g.num_pages = s.num_pages;
+      seg += ns;
+      op += nf;
+      if (seg < s.n_segments || op < s.n_free) break;
+      ++next;
+      seg = op = 0;
     }
     if (a.n_groups == 0) break;
     long at = 0;

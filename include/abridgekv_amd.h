@@ -87,9 +87,9 @@ int abkv_kv_move_segments(void* const* layer_caches, int n_layers, int num_pages
 int abkv_kv_move_mixed(void* const* layer_caches, int n_layers, int num_pages, int block_size, long page_bytes,
                        long half_bytes, int slot_bytes, const int32_t* ops, const int32_t* seg_offsets, int n_segments,
                        const int32_t* free_ops, int n_free, abkv_stream_t stream);
-/* abkv_kv_move_groups: abkv_kv_move_mixed over several KV-cache groups in one launch (up to 8; more take more
- * launches): group i's ops apply to its n_layers (<= 16) layer caches of num_pages pages. Groups may share layer
- * caches when no op of one group reads or writes a slot that another group writes (a planner step's groups own
+/* abkv_kv_move_groups: abkv_kv_move_mixed over several KV-cache groups in one launch (up to 8; more, or more than 2^24
+ * workgroups, take more launches): group i's ops apply to its n_layers (<= 16) layer caches of num_pages pages. Groups
+ * may share layer caches when no op of one group reads or writes a slot that another group writes (a planner step's groups own
  * disjoint pages). Groups without ops are skipped. */
 typedef struct abkv_move_group {
   void* const* layer_caches;

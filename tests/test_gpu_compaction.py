@@ -221,3 +221,23 @@ def test_move_groups_of_one_launch_and_of_several(n_groups):
     ops.kv_move_groups(groups)
     for got, w in zip(on_gpu, want):
         assert torch.equal(got.cpu().view(torch.int16), w)
+
+
+def test_moves_past_the_work_items_of_one_launch():
+    """4.3 million independent ops and a segment on 16 layer tensors: more workgroups than one launch takes. All but the
+    first and the last ops are padding (pages of -1, skipped)."""
+    dev = torch.device("cuda")
+    caches = [torch.randint(-2 ** 15, 2 ** 15, ops.kv_cache_shape(4), dtype=torch.int16,
+                            generator=torch.Generator().manual_seed(i)).view(torch.bfloat16).to(dev) for i in range(16)]
+    n = 4_300_001
+    free = torch.full((n, 4), -1, dtype=torch.int32, device=dev)
+    free[0] = torch.tensor([0, 5, 1, 6])
+    free[n - 1] = torch.tensor([2, 7, 3, 8])
+    ordered = torch.tensor([[0, 1, 0, 0], [0, 2, 0, 1]], dtype=torch.int32, device=dev)
+    want = [c.clone() for c in caches]
+    for w, c in zip(want, caches):
+        for a, b, d, e in [(0, 5, 1, 6), (2, 7, 3, 8), (0, 1, 0, 0), (0, 2, 0, 1)]:
+            w[d, :, e] = c[a, :, b]
+    ops.kv_move_mixed(caches, ordered, torch.tensor([0, 2], dtype=torch.int32, device=dev), free)
+    for got, w in zip(caches, want):
+        assert torch.equal(got.view(torch.int16), w.view(torch.int16))
