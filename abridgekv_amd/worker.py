@@ -202,19 +202,19 @@ def device_move_lists(dev_buf: torch.Tensor, parts):
 
 def launch_moves(prepared, layer_caches_by_group, events=None) -> None:
     """Device side of :func:`execute_fused_moves`: the step's groups in one launch (per 8 groups; a group of more than
-    16 layer tensors counts once per 16). No op of a step touches a slot of another group: a page of the pool belongs
-    to one request and group. ``events``, if given, is a list that receives the (start, end) CUDA events recorded
-    around the launch."""
-    start = 0
-    while start < len(prepared):
-        gids, groups = set(), []
-        for gid, ops_d, offs_d, free_d in prepared[start:]:
-            if gid in gids:                                    # a group's second list may build on its first
-                break
-            gids.add(gid)
-            caches = layer_caches_by_group[gid]
-            groups += [(caches[lo: lo + 16], ops_d, offs_d, free_d) for lo in range(0, len(caches), 16)]
-        start += len(gids)
+    16 layer tensors counts once per 16). ``prepared``: a planner step's lists, in which no op touches a slot of another
+    group (a page of the pool belongs to one request and group); lists that are not so go one group a call. A group's
+    second list may build on its first: it starts a new launch. ``events``, if given, is a list that receives the
+    (start, end) CUDA events recorded around each launch."""
+    launches, gids = [], set()
+    for gid, ops_d, offs_d, free_d in prepared:
+        if not launches or gid in gids:
+            launches.append([])
+            gids = set()
+        gids.add(gid)
+        caches = layer_caches_by_group[gid]
+        launches[-1] += [(caches[lo: lo + 16], ops_d, offs_d, free_d) for lo in range(0, len(caches), 16)]
+    for groups in launches:
         if events is not None:
             s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             s.record()
@@ -224,15 +224,28 @@ def launch_moves(prepared, layer_caches_by_group, events=None) -> None:
             events.append((s, e))
 
 
+def _groups_overlap(fused_moves: np.ndarray, layer_caches_by_group) -> bool:
+    """Whether a page of one group's rows is also in another group's with a layer tensor in common (never in a planner
+    step's rows)."""
+    gids = np.unique(fused_moves[:, 1]).tolist()
+    tensors = {g: {c.data_ptr() for c in layer_caches_by_group[g]} for g in gids}
+    pages = {g: np.unique(fused_moves[fused_moves[:, 1] == g][:, [2, 4]]) for g in gids}
+    return any(tensors[g] & tensors[h] and np.intersect1d(pages[g], pages[h], assume_unique=True).size > 0
+               for i, g in enumerate(gids) for h in gids[:i])
+
+
 def execute_fused_moves(fused_moves: np.ndarray, layer_caches_by_group, check: bool = True) -> None:
     """Apply a planner step's fused move rows (request, group, src_block, src_off, dst_block, dst_off) in one
     launch. Rows of one (request, group) are monotone (increasing source, dst < src): a run whose ops depend on
-    each other's order is walked in order by the in-register chunked copy, every other op moves independently."""
+    each other's order is walked in order by the in-register chunked copy, every other op moves independently.
+    Groups that meet on a page of a shared layer tensor are applied one after the other, in group order."""
     if fused_moves.size == 0:
         return
     num_pages = layer_caches_by_group[0][0].shape[0]
-    launch_moves(prepare_fused_moves(fused_moves, num_pages, layer_caches_by_group[0][0].device, check),
-                 layer_caches_by_group)
+    prepared = prepare_fused_moves(fused_moves, num_pages, layer_caches_by_group[0][0].device, check)
+    one_by_one = _groups_overlap(fused_moves, layer_caches_by_group)
+    for part in [[p] for p in prepared] if one_by_one else [prepared]:
+        launch_moves(part, layer_caches_by_group)
 
 
 def truncate_block_table(block_ids_by_group, keep):

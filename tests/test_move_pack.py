@@ -241,3 +241,35 @@ def test_config2_fused_moves_equal_oracle_batches():
             assert np.array_equal(got, want), (r, g)
             kept_rows += active
     assert kept_rows > 64 * G * 128
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """Group ids of every kv_move_groups call, by the layer tensors handed over (none is made)."""
+    calls = []
+    monkeypatch.setattr(worker.ops, "kv_move_groups", lambda groups: calls.append([g[0][0].data_ptr() for g in groups]))
+    return calls
+
+
+def test_groups_that_meet_on_a_page_are_launched_one_after_the_other(launches):
+    """Group 1 reads the row that group 0 writes: over a shared tensor a launch each, in group order; over tensors of
+    their own, or on pages of their own, one launch."""
+    import torch
+    shared, a, b = (torch.zeros((16, 2, 16, 1, 8)) for _ in range(3))
+    meet = np.array([[0, 0, 3, 4, 2, 1], [0, 1, 2, 1, 1, 0]], np.int64)
+    apart = np.array([[0, 0, 3, 4, 2, 1], [0, 1, 7, 1, 6, 0]], np.int64)
+    for rows, caches, want in [(meet, [[shared], [shared]], 2), (meet, [[a], [b]], 1), (apart, [[shared], [shared]], 1)]:
+        for check in (True, False):
+            launches.clear()
+            worker.execute_fused_moves(rows, caches, check=check)
+            assert len(launches) == want
+            assert sum(launches, []) == [caches[0][0].data_ptr(), caches[1][0].data_ptr()]
+
+
+def test_a_groups_second_list_starts_a_new_launch(launches):
+    """launch_moves over any iterable of lists."""
+    import torch
+    caches = [[torch.zeros(1)] for _ in range(3)]
+    ids = [c[0].data_ptr() for c in caches]
+    worker.launch_moves(((g, None, None, None) for g in (0, 1, 0, 2, 1, 1)), caches)
+    assert launches == [[ids[0], ids[1]], [ids[0], ids[2], ids[1]], [ids[1]]]
