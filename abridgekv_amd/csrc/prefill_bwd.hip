@@ -15,6 +15,8 @@
 //                            replaced a classification per tile pair, 988 -> 965 us (B=2, 12 x (512 + 128 rows))
 #include "prefill_common.h"
 
+#include "bwd_plan.h"
+
 namespace abkv {
 
 struct PrefillBwdArgs {
@@ -25,7 +27,8 @@ struct PrefillBwdArgs {
   float* lse2;                                // workspace [B, 32, S0p]
   float* dvec;                                // workspace [B, 32, S0p]
   int S0p;                                    // S0 rounded up to a multiple of 64
-  int* seen;                                  // [key tiles x B] query tiles that see the key tile (workspace, as the next two)
+  int* seen;                                  // [key tiles x B] query tiles that see the key tile (workspace, as the next
+                                              // two); nullptr: no parts, one workgroup per key tile in tile order
   int* done;                                  // [slot_cap x 8] finished parts, at the tile's first item
   float* slots;                               // [slot_cap x 8][kSlotFloats] sums of the parts
   int slot_cap;                               // partial slots per KV head
@@ -94,8 +97,7 @@ struct TileSpan {
 // 811; B=2, 12 x (512 + 128) (120 against 82: not split) 1835 -> 1829, and parts of 3/4 of the share, which lose the
 // reuse of query tiles in L2, 1905; B=2, 4 x (512 + 256) with a rolling tail 812 -> 838. A least part of 8 instead of 12
 // query tiles: causal 1500 rows 246 -> 260.
-constexpr int kDkvMinPart = 12;                // query tiles (x 4 heads) a part is worth starting for
-constexpr int kSlotFloats = 2 * kBN * kHeadDim;   // dK and dV of a key tile
+static_assert(kSlotFloats == 2 * kBN * kHeadDim && kHeadsQ == 32 && kHeadsKV == 8, "bwd_plan.h");
 // One part: parts == 1: the whole tile.
 struct DkvItem {
   int tile;                  // key tile * B + sequence
@@ -124,11 +126,6 @@ __device__ __forceinline__ int block_sum(int v, int* lds) {
   return lds[0] + lds[1] + lds[2] + lds[3];
 }
 
-// Parts of a tile that `seen` query tiles see, with an even share of `share` query tiles a worker.
-__device__ __forceinline__ int dkv_parts(int seen, int share) {
-  if (2 * seen <= 3 * share) return 1;                      // (at most 3/2 seen / share parts otherwise)
-  return (seen + share - 1) / share;
-}
 // Order of issue: 0 the split tiles' parts, then whole tiles by length: 1 over the share, 2 over half of it, 3 the rest.
 __device__ __forceinline__ int dkv_class(int seen, int share) {
   return dkv_parts(seen, share) > 1 ? 0 : seen > share ? 1 : 2 * seen > share ? 2 : 3;
@@ -141,7 +138,7 @@ __device__ __forceinline__ bool dkv_item(const int* seen, int tiles, int workers
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   int v = 0;
   for (int e = tid; e < tiles; e += 256) v += seen[e];
-  const int share = max(kDkvMinPart, (block_sum(v, lds) + workers - 1) / workers);
+  const int share = dkv_share(block_sum(v, lds), workers);
   int at = 0, cls = 0, n = 0;                                // the class that item i lies in: items at .. at + n - 1
   for (; cls < 4; ++cls) {
     v = 0;
@@ -442,8 +439,8 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
   float* const Eb[2] = {E0, E1};
   const PrefillArgs& f = a.f;
   const int kvh = blockIdx.x % kHeadsKV;                    // a KV head's workgroups on one XCD, as grid_pos
-  DkvItem item;
-  if (!dkv_item(a.seen, f.num_q_tiles * f.B, a.workers, blockIdx.x / kHeadsKV, item)) return;
+  DkvItem item{(int)(blockIdx.x / kHeadsKV), 0, 1, 0, 0};
+  if (a.seen != nullptr && !dkv_item(a.seen, f.num_q_tiles * f.B, a.workers, item.tile, item)) return;
   const int kt = item.tile / f.B;
   const int b = item.tile - kt * f.B;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -628,38 +625,16 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
   }
 }
 
-// Workspace offsets.
-struct BwdLayout {
-  size_t dvec, seen, done, slots, bytes;
-  int workers, cap;                           // cap: partial slots per KV head (parts of split tiles)
-};
-static BwdLayout bwd_layout(int batch, int seq_len) {
-  const size_t q_tiles = ((size_t)(seq_len > 0 ? seq_len : 0) + kBN - 1) / kBN;
-  const size_t tiles = q_tiles * (size_t)(batch > 0 ? batch : 0);
-  const size_t row_bytes = tiles * kBN * kHeadsQ * sizeof(float);
-  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
-  BwdLayout l;
-  l.workers = 2 * 256 / kHeadsKV;             // two workgroups a CU on 256 CUs
-  // parts (dkv_parts): at most 3/2 * workers in all (48 MiB of slots), and a tile's are under q_tiles / kDkvMinPart + 1
-  const size_t few = tiles * (q_tiles / kDkvMinPart + 1);
-  l.cap = (int)(few < (size_t)(3 * l.workers / 2) ? few : (size_t)(3 * l.workers / 2));
-  if (2 * q_tiles <= 3 * kDkvMinPart) l.cap = 0;            // nothing is split
-  l.dvec = row_bytes;
-  l.seen = up(2 * row_bytes);
-  l.done = l.seen + up(tiles * sizeof(int));
-  l.slots = l.done + up((size_t)l.cap * kHeadsKV * sizeof(int));
-  l.bytes = l.slots + (size_t)l.cap * kHeadsKV * kSlotFloats * sizeof(float) + 16;   // + the base's alignment
-  return l;
-}
+constexpr int kCus = 256;
 
 }  // namespace abkv
 
 extern "C" {
 
 // Workspace bytes of abkv_prefill_masked_attn_bwd: lse * log2(e) and rowsum(dO * O) per (batch, query head, row),
-// rows padded to whole 64-row tiles; the dK/dV counts and partial slots.
+// rows padded to whole 64-row tiles; the dK/dV counts and partial slots (up to 48 MiB).
 size_t abkv_prefill_masked_bwd_workspace_size(int batch, int seq_len) {
-  return abkv::bwd_layout(batch, seq_len).bytes;
+  return abkv::bwd_layout(batch, seq_len, abkv::kCus).bytes;
 }
 
 int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s, long q_stride_h, const void* k,
@@ -686,8 +661,9 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
       tail_policy < kTailStatic || tail_policy > kTailRaw ||
       pause_xattn < kXattnFull || pause_xattn > kXattnNone)
     return (int)hipErrorInvalidValue;
-  if (workspace == nullptr || workspace_bytes < abkv_prefill_masked_bwd_workspace_size(batch, seq_len))
-    return (int)hipErrorInvalidValue;
+  const BwdLayout lay = bwd_layout(batch, seq_len, kCus);
+  if (workspace == nullptr || workspace_bytes < lay.rows) return (int)hipErrorInvalidValue;
+  const bool parts = workspace_bytes >= lay.bytes;          // less: a workgroup per key tile, in tile order
   PrefillBwdArgs a;
   PrefillArgs& f = a.f;
   f.q = static_cast<const __bf16*>(q);
@@ -718,16 +694,15 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
   a.g_sb = dout_stride_b; a.g_ss = dout_stride_s; a.g_sh = dout_stride_h;
   a.lse = lse;
   a.S0p = f.num_q_tiles * kBM;
-  const BwdLayout lay = bwd_layout(batch, seq_len);
+  a.lse2 = static_cast<float*>(workspace);
+  a.dvec = reinterpret_cast<float*>(static_cast<char*>(workspace) + lay.dvec);
   char* ws = static_cast<char*>(workspace) + (-reinterpret_cast<uintptr_t>(workspace) & 15);
-  a.lse2 = reinterpret_cast<float*>(ws);
-  a.dvec = reinterpret_cast<float*>(ws + lay.dvec);
-  a.seen = reinterpret_cast<int*>(ws + lay.seen);
+  a.seen = parts ? reinterpret_cast<int*>(ws + lay.seen) : nullptr;
   a.done = reinterpret_cast<int*>(ws + lay.done);
   a.slots = reinterpret_cast<float*>(ws + lay.slots);
-  a.slot_cap = lay.cap;
+  a.slot_cap = parts ? lay.cap : 0;
   a.workers = lay.workers;
-  a.count_blocks = (f.num_q_tiles * batch + 3) / 4;
+  a.count_blocks = parts ? (f.num_q_tiles * batch + 3) / 4 : 0;
   a.scale = scale;
   a.dq = static_cast<__bf16*>(dq);
   a.dq_sb = dq_stride_b; a.dq_ss = dq_stride_s; a.dq_sh = dq_stride_h;
@@ -737,7 +712,7 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
   a.dv_sb = dv_stride_b; a.dv_ss = dv_stride_s; a.dv_sh = dv_stride_h;
   if (prefill_grid(f.num_q_tiles, batch, 512) == 0) return (int)hipErrorInvalidValue;
   const long rows = (long)batch * kHeadsQ * a.S0p;
-  const long gk = ((long)lay.cap + (long)f.num_q_tiles * batch) * kHeadsKV;   // at least the items of dkv_item
+  const long gk = ((long)a.slot_cap + (long)f.num_q_tiles * batch) * kHeadsKV;   // at least the items of dkv_item
   // prep: 16 work-items per row and head, and the counting workgroups
   if (rows * 16 + 256L * (a.count_blocks + 1) > 0xFFFFFFFFL || gk * 256 > 0xFFFFFFFFL) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(prefill_bwd_prep_kernel, dim3((unsigned)((rows * 16 + 255) / 256 + a.count_blocks)), dim3(256), 0, stream,

@@ -191,7 +191,9 @@ int abkv_prefill_masked_attn(const void* q, long q_stride_b, long q_stride_s, lo
  * 128] (bf16, element strides, dims contiguous; written, not accumulated) of sum(dout * out) under the same mask,
  * from the forward's out and lse (lse required). Replaces the FlexAttention backward the reference trains through
  * (abridgekv/compress_forward.py:1134-1230 under autograd; its self-test calls backward at :1329).
- * workspace >= abkv_prefill_masked_bwd_workspace_size(batch, seq_len) bytes. */
+ * workspace >= abkv_prefill_masked_bwd_workspace_size(batch, seq_len) bytes (256 bytes a row of the batch and up to 48 MiB
+ * for the partial sums of long key tiles' dK/dV). With 256 * batch * ceil(seq_len / 64) * 64 bytes or more but less than
+ * that, long key tiles are not split, which takes longer (8 blocks of 512 + 128 + 16 rows: a third). */
 size_t abkv_prefill_masked_bwd_workspace_size(int batch, int seq_len);
 int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s, long q_stride_h, const void* k,
                                  long k_stride_b, long k_stride_s, long k_stride_h, const void* v, long v_stride_b,

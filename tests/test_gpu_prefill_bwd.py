@@ -258,3 +258,34 @@ def test_split_parts_add_up_in_a_fixed_order():
     for _ in range(4):
         again = ops.prefill_masked_attention_backward(q, k, v, out, lse, dout, C, K, N, replay_rows=R)
         assert all(torch.equal(a, b) for a, b in zip(first, again))
+
+
+@pytest.mark.parametrize("extra", [0, 4096])
+def test_a_workspace_without_room_for_parts(monkeypatch, extra):
+    """Rows alone (lse and rowsum(dO O) per head), or too little beside them: no key tile is split, and the gradients are
+    those of the split launch up to the order of their sums (bf16 outputs: one rounding, 2^-8 of the value)."""
+    from abridgekv_amd import ops
+    C, K, N = 64, 64, 14                                     # 28 key tiles, codes of the first block seen by 27 query tiles
+    S = N * (C + K)
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(70)
+    q, k, v, dout = (torch.randn((1, S, h, 128), generator=g).to(torch.bfloat16).to(dev) for h in (32, 8, 8, 32))
+    lse = torch.empty((1, 32, S), dtype=torch.float32, device=dev)
+    out, _ = ops.prefill_masked_attention(q, k, v, C, K, N, lse=lse)
+    want = ops.prefill_masked_attention_backward(q, k, v, out, lse, dout, C, K, N)
+
+    class Small:
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def abkv_prefill_masked_bwd_workspace_size(self, batch, seq_len):
+            rows = 256 * batch * (-(-seq_len // 64) * 64)
+            assert rows + extra < real.abkv_prefill_masked_bwd_workspace_size(batch, seq_len)
+            return rows + extra
+    real = ops.lib()
+    monkeypatch.setattr(ops, "lib", Small)
+    got = ops.prefill_masked_attention_backward(q, k, v, out, lse, dout, C, K, N)
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):
+        err = (a.float() - b.float()).abs()
+        assert bool((err <= 2.0 ** -7 * b.float().abs() + 1e-4 * b.float().abs().max()).all())
