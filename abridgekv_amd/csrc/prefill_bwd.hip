@@ -625,16 +625,23 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(PrefillBwdArgs 
   }
 }
 
-constexpr int kCus = 256;
+// Compute units of the current device (256 without one).
+static int compute_units() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 256;
+  return n;
+}
 
 }  // namespace abkv
 
 extern "C" {
 
 // Workspace bytes of abkv_prefill_masked_attn_bwd: lse * log2(e) and rowsum(dO * O) per (batch, query head, row),
-// rows padded to whole 64-row tiles; the dK/dV counts and partial slots (up to 48 MiB).
+// rows padded to whole 64-row tiles; the dK/dV counts and partial slots (up to 48 MiB, by the device's compute units).
 size_t abkv_prefill_masked_bwd_workspace_size(int batch, int seq_len) {
-  return abkv::bwd_layout(batch, seq_len, abkv::kCus).bytes;
+  return abkv::bwd_layout(batch, seq_len, abkv::compute_units()).bytes;
 }
 
 int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s, long q_stride_h, const void* k,
@@ -661,7 +668,7 @@ int abkv_prefill_masked_attn_bwd(const void* q, long q_stride_b, long q_stride_s
       tail_policy < kTailStatic || tail_policy > kTailRaw ||
       pause_xattn < kXattnFull || pause_xattn > kXattnNone)
     return (int)hipErrorInvalidValue;
-  const BwdLayout lay = bwd_layout(batch, seq_len, kCus);
+  const BwdLayout lay = bwd_layout(batch, seq_len, compute_units());
   if (workspace == nullptr || workspace_bytes < lay.rows) return (int)hipErrorInvalidValue;
   const bool parts = workspace_bytes >= lay.bytes;          // less: a workgroup per key tile, in tile order
   PrefillBwdArgs a;

@@ -35,3 +35,14 @@ def test_parts_fit_the_slots(plan, cus):
         seen = np.ascontiguousarray(seen, np.int32)
         n = plan.slots(seen.ctypes.data_as(C.POINTER(C.c_int32)), seen.size, cus)
         assert n <= plan.layout_cap(batch, 64 * q_tiles, cus)
+
+
+def test_slots_follow_the_device(plan):
+    """Long key tiles are split for the workgroups that a device runs at once: an eighth of the CUs, an eighth of the slots."""
+    seen = np.full(2000, 100, np.int32)
+    seen[:40] = 2000
+    at = seen.ctypes.data_as(C.POINTER(C.c_int32))
+    assert plan.slots(at, seen.size, 256) == 0 and plan.slots(at, seen.size, 2048) > 0
+    assert plan.layout_cap(1, 128000, 32) == plan.layout_cap(1, 128000, 256) // 8
+    row_bytes = 256 * 128000
+    assert row_bytes < plan.layout_bytes(1, 128000, 256) < row_bytes + (49 << 20)
