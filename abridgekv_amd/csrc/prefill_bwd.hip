@@ -40,18 +40,21 @@ struct PrefillBwdArgs {
   __bf16* dv; long dv_sb, dv_ss, dv_sh;
 };
 
-// Smallest v over the wave's lanes, in VALU (DPP inside rows of 16 lanes, then lane swaps): a TileSpan is twelve of
-// these, and as chains of LDS permutes they cost 3.5 us a key tile.
-__device__ __forceinline__ int wave_min(int v) {
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));    // quad_perm 1,0,3,2
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));    // quad_perm 2,3,0,1
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));   // row_half_mirror
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));   // row_mirror
+// f over the wave's lanes (uniform), in VALU (DPP inside rows of 16 lanes, then lane swaps): a TileSpan is twelve of these,
+// and as chains of LDS permutes they cost 3.5 us a key tile.
+template <class F>
+__device__ __forceinline__ int wave_all(int v, F f) {
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));      // quad_perm 1,0,3,2
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));      // quad_perm 2,3,0,1
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));     // row_half_mirror
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));     // row_mirror
   const auto r16 = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  v = min((int)r16[0], (int)r16[1]);
+  v = f((int)r16[0], (int)r16[1]);
   const auto r32 = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return __builtin_amdgcn_readfirstlane(min((int)r32[0], (int)r32[1]));
+  return __builtin_amdgcn_readfirstlane(f((int)r32[0], (int)r32[1]));
 }
+__device__ __forceinline__ int wave_min(int v) { return wave_all(v, [](int a, int b) { return min(a, b); }); }
+__device__ __forceinline__ int wave_sum(int v) { return wave_all(v, [](int a, int b) { return a + b; }); }
 
 // Which query tiles a 64-key tile is seen by, from the query ranges of its keys (lane l: key k0 + l; wave-uniform and
 // the same in every wave): a query tile outside the hulls of the ranges is hidden, one inside the common part of the
@@ -92,11 +95,11 @@ struct TileSpan {
 // codes' workgroup. Tiles longer than 3/2 of a worker's even share of the launch are split into parts of at most the
 // share; the parts leave fp32 sums in slots, and the last part to finish adds them up in part order. Parts and long tiles
 // go first. The prep kernel counts (the raw prompt's length is not known on the host), each dK/dV workgroup finds its
-// part from the counts. Forward + backward calls, one workgroup per tile in tile order -> this: B=1, 8 x (512 + 128 + 16)
-// rows (82 query tiles against a share of 16) 960 -> 652 us, B=1, 10 x (512 + 128) 911 -> 585, causal 4000 rows 877 ->
-// 811; B=2, 12 x (512 + 128) (120 against 82: not split) 1835 -> 1829, and parts of 3/4 of the share, which lose the
-// reuse of query tiles in L2, 1905; B=2, 4 x (512 + 256) with a rolling tail 812 -> 838. A least part of 8 instead of 12
-// query tiles: causal 1500 rows 246 -> 260.
+// part from the counts. Backward calls in us, one workgroup per tile in tile order -> this: B=1, 8 x (512 + 128 + 16) rows
+// (82 query tiles against a share of 16) 829 -> 508, 4 x (512 + 128) 277 -> 152, causal 1500 rows 267 -> 230; B=2,
+// 4 x (512 + 256) with a rolling tail 466 -> 399; B=2, 12 x (512 + 128) (120 against 82: not split, only ordered)
+// 1242 -> 1119, and parts of 3/4 of the share there, which lose the reuse of query tiles in L2, 4 % slower. A least part of
+// 8 instead of 12 query tiles: causal 1500 rows 6 % slower.
 static_assert(kSlotFloats == 2 * kBN * kHeadDim && kHeadsQ == 32 && kHeadsKV == 8, "bwd_plan.h");
 // One part: parts == 1: the whole tile.
 struct DkvItem {
@@ -118,8 +121,7 @@ __device__ __forceinline__ unsigned long long seen_mask(const PrefillArgs& f, co
 
 // Sum of v over the workgroup's 256 threads (uniform).
 __device__ __forceinline__ int block_sum(int v, int* lds) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -131,14 +133,28 @@ __device__ __forceinline__ int dkv_class(int seen, int share) {
   return dkv_parts(seen, share) > 1 ? 0 : seen > share ? 1 : 2 * seen > share ? 2 : 3;
 }
 
-// Item i of a KV head (workgroup of 256 threads; uniform), by class and tile; false past the last.
+// Item i of a KV head (workgroup of 256 threads; uniform), by class and tile; false past the last. With no tile over the
+// share there is no tail to shorten, and the items are the tiles in their order, which reuses query tiles in L2: B=4,
+// 16 x (512 + 128) rows 3345 us a backward against 3430 by class.
 __device__ __forceinline__ bool dkv_item(const int* seen, int tiles, int workers, int i, DkvItem& item) {
   __shared__ int lds[4];
+  __shared__ int2 whole[4];
   __shared__ DkvItem found;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  int v = 0;
-  for (int e = tid; e < tiles; e += 256) v += seen[e];
-  const int share = dkv_share(block_sum(v, lds), workers);
+  int v = 0, longest = 0;
+  for (int e = tid; e < tiles; e += 256) {
+    v += seen[e];
+    longest = max(longest, seen[e]);
+  }
+  v = wave_sum(v);
+  longest = -wave_min(-longest);
+  if (lane == 0) whole[w] = make_int2(v, longest);
+  __syncthreads();
+  const int share = dkv_share(whole[0].x + whole[1].x + whole[2].x + whole[3].x, workers);
+  if (max(max(whole[0].y, whole[1].y), max(whole[2].y, whole[3].y)) <= share) {
+    item = DkvItem{i, 0, 1, 0, 0};
+    return i < tiles;
+  }
   int at = 0, cls = 0, n = 0;                                // the class that item i lies in: items at .. at + n - 1
   for (; cls < 4; ++cls) {
     v = 0;
