@@ -30,8 +30,9 @@ static bool visible(const MaskShape& g, const TileMask& tm, const RowFacts& r, i
 
 extern "C" {
 
-// counts [4][S0][S0]; returns the number of tiles walked, or -1 for a tile whose first key is out of range.
-long walk_counts(const int32_t* params, int plen, const int32_t* quota, uint8_t* counts) {
+// counts [4][S0][S0] over query tiles of `rows` rows; returns the number of key tiles walked, or -1 for a tile whose first
+// key is out of range.
+long walk_counts(const int32_t* params, int plen, const int32_t* quota, int rows, uint8_t* counts) {
   const MaskShape g = shape(params);
   const long S = g.S0;
   int qmin = quota[0], qmax = quota[0];
@@ -41,14 +42,14 @@ long walk_counts(const int32_t* params, int plen, const int32_t* quota, uint8_t*
   }
   long tiles = 0;
   for (int hb = 0; hb < 4; hb += 2)
-    for (int q0 = 0; q0 < g.S0; q0 += kBM) {
-      SegWalk walk(g, q0, imin(q0 + kBM, g.S0) - 1, plen, qmin, qmax, quota[hb], quota[hb + 1]);
+    for (int q0 = 0; q0 < g.S0; q0 += rows) {
+      SegWalk walk(g, q0, imin(q0 + rows, g.S0) - 1, plen, qmin, qmax, quota[hb], quota[hb + 1]);
       int k0 = 0;
       TileMask tm;
       for (bool first = true; walk.next(k0, tm, first); first = false) {
         if (k0 < 0 || k0 >= g.S0) return -1;
         ++tiles;
-        for (int q = q0; q < imin(q0 + kBM, g.S0); ++q) {
+        for (int q = q0; q < imin(q0 + rows, g.S0); ++q) {
           const RowFacts r = row_facts(g, q);
           for (int u = 0; u < 2; ++u)
             for (int key = k0; key < k0 + kBN; ++key) {
