@@ -708,6 +708,7 @@ def paged_prefill_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table
     B = ks.size
     W = block_table.shape[1]
     _require(qs.size == B + 1 and kl.size == B and B <= block_table.shape[0], "q_start [B+1], kv_start/kv_limit [B]")
+    _require(qs.ndim == ks.ndim == kl.ndim == 1 and np.ndim(causal) <= 1, "lengths and flags must be flat sequences")
     T, total = q.shape[0], int(qs[-1])
     _require(qs[0] == 0 and total <= T and (B == 0 or (qs[1:] >= qs[:-1]).all()), "q_start must be a prefix sum <= T")
     _require(B == 0 or (kl.min() >= 0 and kl.max() <= W * PAGE), "kv_limit must lie in [0, block_table width * 16]")

@@ -124,6 +124,17 @@ def test_rejects_limits_past_the_table():
                                     torch.zeros((1, 2), dtype=torch.int32, device=dev), [0, 2], [0], [33], True)
 
 
+@pytest.mark.parametrize("starts,limits,causal", [([[0]], [30], True), ([0], [[30]], True), (0, [30], True),
+                                                  ([0], [30], [[True]]), ([0], [30], [True, False])])
+def test_rejects_lengths_and_flags_that_are_not_flat(starts, limits, causal):
+    from abridgekv_amd import ops
+    dev = torch.device("cuda")
+    cache = torch.zeros((4, 2, 16, 8, 128), dtype=torch.bfloat16, device=dev)
+    with pytest.raises(ValueError):
+        ops.paged_prefill_attention(torch.zeros((2, 32, 128), dtype=torch.bfloat16, device=dev), cache,
+                                    torch.zeros((1, 2), dtype=torch.int32, device=dev), [0, 2], starts, limits, causal)
+
+
 def test_mixed_code_and_prompt_chunk_batch():
     """One launch mixing a non-causal code step (limit = code start + quota) with causal prompt chunks."""
     nq = [256, 130, 1]
