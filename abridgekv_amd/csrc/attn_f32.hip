@@ -242,7 +242,8 @@ struct PagedStages {
 // kOdd = false returns whether V held values that are not finite (uniform; one FMA per loaded value): then the result
 // holds only if every column sees every key of every stage, and f32_attend walks again with kOdd = true. That one keeps such
 // values out of the product and returns whether extra (this lane's dims 16g .. of its output row; nullptr: no row) holds
-// sums of f32_odd_v to be added. As a branch of the first walk they cost 5 % (masked, 3 x (512 + 128) rows).
+// sums of f32_odd_v to be added. As a branch of the first walk they cost 5 % (masked, 3 x (512 + 128) rows); so, the look
+// costs short walks 3 % (masked, 10 x (128 + 64) rows 141 -> 145 us) and long ones nothing.
 template <int kKeys, bool kOdd, class Stages>
 __device__ __forceinline__ bool f32_walk(Stages src, float* lds, const floatx4 (&q)[8], float scale, float* extra,
                                            float& m, float& l, floatx4 (&o)[8]) {
@@ -443,8 +444,8 @@ __device__ __forceinline__ void f32_put(float* row, int g, const floatx4 (&o)[8]
 // Up to kNarrowRows rows of one request against a KV head, by the four waves of a workgroup: the 16 columns are 4 heads x 4
 // rows, and the waves share the request's pages instead of the heads. A tile of 16 rows by head would leave 12 of 16
 // columns empty (16 requests of one row over 5000 keys, one after the other in both forms: 7700 us by head, 2320 so; a wave
-// of dot products per token and KV head took 2967). Writes the rows and returns false, or returns true (uniform) and writes nothing if V held values that are
-// not finite. lds: 4 x 16 x (128 + 2) floats.
+// of dot products per token and KV head took 2967). Writes the rows and returns false, or returns true (uniform) and writes
+// nothing if V held values that are not finite. lds: 4 x 16 x (128 + 2) floats.
 constexpr int kNarrowRows = 4;
 __device__ __forceinline__ bool f32_narrow(const F32Args& a, float* lds, const F32Span& span, int n_keys, int b, int kvh,
                                            int t, int t1) {
@@ -454,8 +455,8 @@ __device__ __forceinline__ bool f32_narrow(const F32Args& a, float* lds, const F
   floatx4 q[8], o[8];
   float m, l;
   f32_load_q(a.q + (long)min(row, t1 - 1) * a.q_st + (long)(kvh * kGroup + (m16 >> 2)) * a.q_sh, g, row < t1, q);
-  const bool odd = f32_pages<4, true>(a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages, n_keys, span,
-                                    a.scale, w, q, m, l, o);
+  const bool odd = f32_pages<4, true>(a.kv + kvh * kHeadDim, a.block_table + (long)b * a.bt_stride, a.num_pages, n_keys,
+                                      span, a.scale, w, q, m, l, o);
   float* ml = lds + 4 * 16 * kHeadDim;
   f32_put(lds + (w * 16 + m16) * kHeadDim, g, o);
   if (g == 0) *reinterpret_cast<float2*>(ml + 2 * (w * 16 + m16)) = make_float2(m, l);
@@ -491,9 +492,10 @@ __device__ __forceinline__ bool f32_narrow(const F32Args& a, float* lds, const F
 // Multi-query attention, masked (kMasked) or paged: a workgroup of 4 waves takes 16 query rows of one KV head, one query
 // head per wave. Bound by the fp32 matrix rate (16x16x4: 256 flop per clock and CU). Matrix instructions, LDS stages
 // shared by the four heads and the segment walk instead of VALU dot products per key with the mask's predicate per
-// element: masked, B=1, 3 x (512 + 128) rows 1546 -> 203 us; a code step of 256 rows over 4000 keys 2059 -> 412 us.
+// element: masked, B=1, 3 x (512 + 128) rows 1546 -> 203 us; a code step of 256 rows over 4000 keys 1909 -> 397 us.
 template <bool kMasked, int kKeys>
 __global__ __launch_bounds__(256, kKeys == 16 ? 3 : 2) void attn_f32_rows_kernel(F32Args a) {
+  static_assert(kMasked || 4 * kKeys * kHeadDim >= 4 * 16 * (kHeadDim + 2), "f32_narrow");
   __shared__ __attribute__((aligned(16))) float lds[4 * kKeys * kHeadDim];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
@@ -765,8 +767,8 @@ int abkv_prefill_masked_attn_f32(const float* q, long q_sb, long q_ss, long q_sh
   const unsigned grid = f32_grid(((long)seq_len + kF32Rows - 1) / kF32Rows * batch);
   if (grid == 0) return (int)hipErrorInvalidValue;
   // Stages of 16 keys (three workgroups a CU) where blocks have codes: segments are short, their last stage partly empty;
-  // of 32 (two, half the barriers) for one long causal walk. 16 / 32: 3 x (512 + 128) rows 218 / 242 us, 6 x (200 + 2 x 40)
-  // 175 / 217; causal 1337 rows 214 / 191, and a paged code step over 4000 keys 439 / 412.
+  // of 32 (two, half the barriers) for one long causal walk. 16 / 32 by events: 3 x (512 + 128) rows 209 / 229 us,
+  // 6 x (200 + 2 x 40) 107 / 133; causal 1337 rows 209 / 181, and a paged code step over 4000 keys 7 % slower with 16.
   if (codes_k > 0) hipLaunchKernelGGL((attn_f32_rows_kernel<true, 16>), dim3(grid), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((attn_f32_rows_kernel<true, 32>), dim3(grid), dim3(256), 0, stream, a);
   return (int)hipGetLastError();

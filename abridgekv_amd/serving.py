@@ -8,7 +8,7 @@ third_party/vllm_overlay/vllm/v1/core/compresslm/processor.py) decides every req
 ``KVPlanner.mask_token_span`` as its ``mask_span`` callback: the compaction of a block whose code run ended is exactly
 the processor's ``_finish_block`` (processor.py:419-557), and the planner turns it into fused row moves.
 
-Device side, per step: the previous step's compaction moves (``abkv_kv_move_mixed``); the slot of every new row per
+Device side, per step: the previous step's compaction moves (``abkv_kv_move_groups``); the slot of every new row per
 KV-cache group (``abkv_slot_mapping``: logical position minus the group's compacted count through the group's page
 table, gpu_model_runner.py:1579-1661 + block_table.py:186-197); then for every layer the fused RoPE + KV append
 (``abkv_rope_kv_append``, bitrev RoPE positions of the abridged layout computed on the device,

@@ -243,7 +243,7 @@ int abkv_paged_prefill_attn(const void* q, long q_stride_t, long q_stride_h, con
  * 3 * max(1, num_cus / 8) always suffice for both. ABKV_ERR_CAPACITY: too small (sizes are set). q_start [num_reqs + 1].
  * abkv_paged_prefill_attn_items runs it (items and merges copied to the device; workspace >=
  * abkv_paged_prefill_items_workspace_size(partial rows) bytes, 16-byte aligned: the parts' sums in fp32, 1064960 bytes
- * per part of 64 rows; a plan has at most the capacity above of them). */
+ * per part of 64 rows; a plan has at most 6 * max(1, num_cus / 8) of them: 204 MB on 256 compute units). */
 size_t abkv_paged_prefill_items_workspace_size(int part_rows);
 int abkv_paged_plan(const int64_t* q_start, const int64_t* kv_start, const int64_t* kv_limit, const int64_t* causal,
                     int num_reqs, int num_cus, int32_t* items, long items_cap, int32_t* merges, long merges_cap,

@@ -314,7 +314,7 @@ def test_training_gradients_match_dense_float64(tail, policy):
 
 def test_training_option_gradients_match_dense_float64():
     """Gradients through two pause passes, a query residual, code-row key/value projections and gated segment-mean
-    seeds (the kernels' per-element walk and the host-side option modules) against the dense float64 model's
+    seeds (the kernels' walk over segments and the host-side option modules) against the dense float64 model's
     autograd, as test_training_gradients_match_dense_float64 bounds them."""
     from abridgekv_amd.compress_forward import CompressLM
 

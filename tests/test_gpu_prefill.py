@@ -64,7 +64,7 @@ def test_aligned_tiles_head_quotas():
 
 
 def test_unaligned_small_blocks():
-    """C=8, K=4: every tile takes the per-element mask path; S0=60 leaves a partial query and key tile."""
+    """C=8, K=4: several blocks a query tile (the walk over segments); S0=60 leaves a partial query and key tile."""
     quota = [4, 4, 4, 4, 1, 1, 1, 1, 2, 2, 2, 2, 3, 3, 3, 3] * 2
     _check(C=8, K=4, N=5, B=2, prompt_len=[5, 13], head_quota=quota, seed=3)
 
@@ -76,7 +76,7 @@ def test_config4_shape_sampled_rows():
 
 
 def test_static_tail_aligned_blocks():
-    """Static retained tail T=32 on 64-aligned blocks (the tail forces the per-element mask path): earlier blocks'
+    """Static retained tail T=32 on 64-aligned blocks (the aligned walk's tail instance): earlier blocks'
     last 32 content rows visible to every later row, hidden from their own block's codes; raw prompt and quotas."""
     quota = np.repeat([64, 16, 40, 64, 1, 33, 64, 8], 4).tolist()
     _check(C=128, K=64, N=4, B=2, prompt_len=[100, 0], head_quota=quota, seed=6, tail=32)
@@ -107,7 +107,7 @@ def test_window_tail_aligned_blocks(policy, tail):
 
 @pytest.mark.parametrize("policy", ["rolling", "sticky"])
 def test_window_tail_unaligned_blocks(policy):
-    """C=8, K=4, T=3 (the per-element predicate) with a partial last tile."""
+    """C=8, K=4, T=3 (the walk over segments) with a partial last tile."""
     quota = [4, 4, 4, 4, 1, 1, 1, 1, 2, 2, 2, 2, 3, 3, 3, 3] * 2
     _check(C=8, K=4, N=5, B=2, prompt_len=[8, 13], head_quota=quota, seed=17, tail=3, policy=policy)
 
@@ -122,7 +122,7 @@ def test_window_tail_served_block_geometry(policy):
 @pytest.mark.parametrize("xattn", ["causal", "none"])
 @pytest.mark.parametrize("shape", ["aligned", "unaligned"])
 def test_pause_xattn(xattn, shape):
-    """Code rows attending their own block's codes causally or not at all (the per-element walk), with a raw prompt,
+    """Code rows attending their own block's codes causally or not at all (the walk over segments), with a raw prompt,
     per-head quotas and a rolling tail."""
     if shape == "aligned":
         quota = np.repeat([64, 16, 40, 64, 1, 33, 64, 8], 4).tolist()
@@ -135,7 +135,7 @@ def test_pause_xattn(xattn, shape):
 
 @pytest.mark.parametrize("passes,shape", [(2, "aligned"), (3, "unaligned"), (2, "unaligned")])
 def test_pause_passes(passes, shape):
-    """L pause passes per block (pass l reads pass l - 1, later blocks the final pass; the per-element walk), with a
+    """L pause passes per block (pass l reads pass l - 1, later blocks the final pass; the walk over segments), with a
     raw prompt, per-head quotas (a slot within its pass), a tail and non-full xattn."""
     if shape == "aligned":
         quota = np.repeat([64, 16, 40, 64, 1, 33, 64, 8], 4).tolist()

@@ -68,13 +68,13 @@ def test_aligned_head_quotas():
 
 
 def test_unaligned_small_blocks_partial_tiles():
-    """C=40, K=12: the per-element mask path; S0=208 leaves a partial query and key tile."""
+    """C=40, K=12: the walk over segments; S0=208 leaves a partial query and key tile."""
     quota = np.repeat([12, 3, 7, 12, 1, 5, 9, 12], 4).tolist()
     _check(C=40, K=12, N=4, B=2, prompt_len=[50, 0], head_quota=quota, seed=3)
 
 
 def test_static_tail_aligned_blocks():
-    """Static retained tail T=32 on 64-aligned blocks: the dK/dV pair walk must reach every later query tile of an
+    """Static retained tail T=32 on 64-aligned blocks: dK/dV must reach every later query tile of an
     earlier block's tail keys, and a block's codes must give its own tail keys no gradient."""
     quota = np.repeat([64, 16, 40, 64, 1, 33, 64, 8], 4).tolist()
     _check(C=128, K=64, N=3, B=2, prompt_len=[100, 0], head_quota=quota, seed=5, tail=32)

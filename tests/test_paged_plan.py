@@ -38,6 +38,7 @@ def test_items_cover_every_tile_once(num_cus, seed):
             used += [p[2] for p in parts]
     assert not merged
     assert sorted(used) == list(range(0, rows, 64))
+    assert len(used) <= 6 * max(1, num_cus // 8)               # the workspace bound
     lengths = items[:, 3] - items[:, 2]
     assert np.all(np.diff(lengths) <= 0)                       # longest first
 
