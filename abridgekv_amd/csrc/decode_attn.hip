@@ -559,13 +559,17 @@ __global__ __launch_bounds__(64) void decode_side_kernel(DecodeArgs a) {
 // one process over the same pages: two waves 952.9 us per launch against four 959.1 and eight 990.5 on the saturated
 // B=256 workload, 241.5 against 245.1 and 254.7 on the B=64 full-model decode; one wave 4 % slower than four.
 // Few splits leave the GPU idle, and the launch is as long as one wave's walk over its split: then four waves share each
-// KV head's split. us a call with a wave per split / shared: one sequence of 1068 rows 19.7 / 17.6, of 9000 24.3 / 17.7,
-// 4 of 1000 .. 3000 24.6 / 17.8, 16 of 1000 .. 5000 (160 splits) 60.9 / 50.3, 64 of 50 .. 500 (one split each) 25.3 /
-// 21.3. Past that the waves are there anyway: 128 of 100 .. 500 37.4 / 39.3, 64 of 500 .. 1023 beside packed pages (128
-// splits) 253 / 256, 64 of 5000 (704) 245.5 / 250.7. Eight waves: within 2 % of four.
+// KV head's split. The time of a batch of equal lengths goes in steps, by workgroups a CU: every 64 splits with two waves
+// (two heads) a workgroup, every 32 with four sharing, so the second wins in every other step. us with a wave per split /
+// shared: one sequence of 1068 rows 19.7 / 17.6, of 9000 24.3 / 17.7; 32 splits (16 of 900 rows) 26.2 / 18.2, 64 29.2 /
+// 29.4, 96 (16 of 3000) 43.0 / 40.9, 128 (16 of 4000) 48.3 / 52.3, 160 (16 of 5000) 65.8 / 64.0, 192 (32 of 3000) 69.3 /
+// 74.5. (Lengths that differ within a batch leave CUs free: 128 splits over 400 .. 4000 rows 40.4 / 37.2, but a launch
+// knows the widest only.) More sequences: 64 of 50 .. 500 (one split each) 25.3 / 21.3, 128 of 100 .. 500 37.4 / 39.3, 64
+// of 500 .. 1023 beside packed pages (128 splits) 253 / 256, 64 of 5000 (704) 245.5 / 250.7. Eight waves: within 2 % of
+// four.
 inline bool share_splits(int max_splits, int num_seqs) {
   const long splits = (long)max_splits * num_seqs;
-  return splits <= 64 || (num_seqs <= 32 && splits <= 192);
+  return splits <= 64 || (num_seqs <= 32 && (splits <= 96 || (splits > 128 && splits <= 160)));
 }
 inline void launch_decode(const DecodeArgs& a, int max_splits, int num_seqs, hipStream_t stream) {
   if (share_splits(max_splits, num_seqs)) {

@@ -258,3 +258,19 @@ def test_split_partials_keep_small_and_large_values(batch, shift):
     out_s, lse_s = _run(q, cache, tables, seq_lens, split_pages=2)
     assert np.array_equal(out_s, out * np.float32(2.0 ** shift))
     assert np.array_equal(lse_s, lse)
+
+
+@pytest.mark.parametrize("splits", [12, 13, 16, 17, 20, 21])
+def test_both_walks_at_the_borders_of_sharing(splits):
+    """Eight sequences of up to 12 .. 21 splits: 96 / 104, 128 / 136 and 160 / 168 splits lie at either side of a border
+    between a wave per split and four."""
+    rng = np.random.default_rng(splits)
+    lens = [32 * splits - 5 * i for i in range(8)]
+    rows = [rng.standard_normal((n, 8, 128)).astype(np.float32) for n in lens]
+    vals = [rng.standard_normal((n, 8, 128)).astype(np.float32) for n in lens]
+    cache, tables, seq_lens = _paged_cache(rows, vals, 500, rng)
+    q = rng.standard_normal((8, 32, 128)).astype(np.float32)
+    out, lse = _run(q, cache, tables, seq_lens, split_pages=2)
+    ref_out, ref_lse = _oracle(q, cache, tables, seq_lens)
+    assert np.abs(out - ref_out).max() <= TOL
+    assert np.abs(lse - ref_lse).max() <= TOL
