@@ -226,10 +226,20 @@ def launch_moves(prepared, layer_caches_by_group, events=None) -> None:
 
 def _groups_overlap(fused_moves: np.ndarray, layer_caches_by_group) -> bool:
     """Whether a page of one group's rows is also in another group's with a layer tensor in common (never in a planner
-    step's rows)."""
-    gids = np.unique(fused_moves[:, 1]).tolist()
+    step's rows). Rows with a page out of range are skipped, as on the device."""
+    num_pages = layer_caches_by_group[0][0].shape[0]
+    group, src, dst = (fused_moves[:, i] for i in (1, 2, 4))
+    if min(src.min(), dst.min()) < 0 or max(src.max(), dst.max()) >= num_pages:
+        ok = (np.minimum(src, dst) >= 0) & (np.maximum(src, dst) < num_pages)
+        group, src, dst = group[ok], src[ok], dst[ok]
+    owner = np.empty(num_pages, np.int64)                  # one of the groups that have the page
+    owner[src] = group
+    owner[dst] = group
+    if (owner[src] == group).all() and (owner[dst] == group).all():
+        return False
+    gids = np.unique(group).tolist()
     tensors = {g: {c.data_ptr() for c in layer_caches_by_group[g]} for g in gids}
-    pages = {g: np.unique(fused_moves[fused_moves[:, 1] == g][:, [2, 4]]) for g in gids}
+    pages = {g: np.unique(np.concatenate([src[group == g], dst[group == g]])) for g in gids}
     return any(tensors[g] & tensors[h] and np.intersect1d(pages[g], pages[h], assume_unique=True).size > 0
                for i, g in enumerate(gids) for h in gids[:i])
 

@@ -264,6 +264,8 @@ def test_groups_that_meet_on_a_page_are_launched_one_after_the_other(launches):
             worker.execute_fused_moves(rows, caches, check=check)
             assert len(launches) == want
             assert sum(launches, []) == [caches[0][0].data_ptr(), caches[1][0].data_ptr()]
+    skipped = np.array([[0, 0, -1, 4, 2, 1], [0, 1, 2, 1, 99, 0]], np.int64)     # pages out of range: no op at all
+    assert not worker._groups_overlap(skipped, [[shared], [shared]])
 
 
 def test_a_groups_second_list_starts_a_new_launch(launches):
